@@ -148,12 +148,17 @@ int ofdft_plan_create(const int nr[3], const double lattice[9], int precision, i
             const size_t work_bytes = std::max((size_t)(4 * P->N * rs), (size_t)(P->N * 8));
             OFDFT_HIP(hipMalloc(&P->work, work_bytes));
             P->red_blocks = 4096;
-            OFDFT_HIP(hipMalloc(&P->red, sizeof(double) * 4096 * 16));
+            // partial sums: 16 columns of 4096 workgroups, one of every R2C tile
+            // (2 rows or more), 7 of every point-wise workgroup (1024 points or
+            // more on fields that have more than 4096 of them)
+            const size_t nred = std::max<size_t>(
+                {4096 * 16, (size_t)nr[0] * nr[1] / 2 + 1, 7 * ((size_t)P->N / 1024 + 1)});
+            OFDFT_HIP(hipMalloc(&P->red, sizeof(double) * nred));
             OFDFT_HIP(hipMalloc(&P->scal, sizeof(double) * kScalSlots));
             OFDFT_HIP(hipMemset(P->scal, 0, sizeof(double) * kScalSlots));
             OFDFT_HIP(hipHostMalloc((void **)&P->pinned, 128 * sizeof(double), hipHostMallocMapped));
             OFDFT_HIP(hipHostGetDevicePointer((void **)&P->pinned_dev, P->pinned, 0));
-            P->ws_bytes = spec_bytes + work_bytes + sizeof(double) * (4096 * 16 + kScalSlots);
+            P->ws_bytes = spec_bytes + work_bytes + sizeof(double) * (nred + kScalSlots);
             plan_aux_setup(*P);
             P->ws_bytes += P->aux_bytes;
             OFDFT_HIP(hipDeviceSynchronize());

@@ -1,5 +1,5 @@
-// Complex helpers and in-register small DFTs (radix 2, 3, 4, 5, 7, 8, 11, 13)
-// shared by the FFT kernels.  Forward = exp(-2 pi i jk/R); INV conjugates.
+// Complex helpers and in-register small DFTs (radix 2, 3, 4, 5, 7, 8, 11, 13
+// and the composite radices up to 20) shared by the FFT kernels.  Forward = exp(-2 pi i jk/R); INV conjugates.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -151,6 +151,92 @@ template <int R, bool INV, typename C> struct DFTOdd {
         for (int k = 0; k < R; ++k) v[k] = out[k];
     }
 };
+// cos and sin of 2 pi m / R at compile time: the angle folded to the first
+// octant (in units of pi / (4 R)), then the Taylor series
+struct CosSin {
+    double c, s;
+};
+constexpr CosSin unit_root(int m, int R) {
+    int a = 8 * (m % R);
+    bool neg_s = false, neg_c = false, swap = false;
+    if (a > 4 * R) {
+        a = 8 * R - a;
+        neg_s = true;
+    }
+    if (a > 2 * R) {
+        a = 4 * R - a;
+        neg_c = true;
+    }
+    if (a > R) {
+        a = 2 * R - a;
+        swap = true;
+    }
+    const double x = 3.14159265358979323846 * a / (4.0 * R), x2 = x * x;
+    double c = 0.0, s = 0.0;
+    for (int k = 13; k >= 1; --k) {
+        c = (1.0 + c) * (-x2 / ((2 * k - 1) * (2 * k)));
+        s = (1.0 + s) * (-x2 / ((2 * k) * (2 * k + 1)));
+    }
+    c = 1.0 + c;
+    s = x * (1.0 + s);
+    const double cc = swap ? s : c, ss = swap ? c : s;
+    return {neg_c ? -cc : cc, neg_s ? -ss : ss};
+}
+template <int R> struct RootTab {
+    double c[R], s[R];
+    constexpr RootTab() : c(), s() {
+        for (int m = 0; m < R; ++m) {
+            const CosSin w = unit_root(m, R);
+            c[m] = w.c;
+            s[m] = w.s;
+        }
+    }
+};
+
+// Composite radix P Q as P-point DFTs over n1 of x[Q n1 + n2], the twiddles
+// w^(n2 k1) and Q-point DFTs over n2, result k at k1 + P k2
+template <int P, int Q, bool INV, typename C> struct DFTPQ {
+    __device__ __forceinline__ static void run(C *v) {
+        using T = decltype(v[0].x);
+        constexpr int R = P * Q;
+        constexpr RootTab<R> w{};
+        C y[P][Q];
+#pragma unroll
+        for (int n2 = 0; n2 < Q; ++n2) {
+            C t[P];
+#pragma unroll
+            for (int n1 = 0; n1 < P; ++n1) t[n1] = v[Q * n1 + n2];
+            DFT<P, INV, C>::run(t);
+#pragma unroll
+            for (int k1 = 0; k1 < P; ++k1) {
+                const int m = n2 * k1;  // < R
+                if (m == 0) {
+                    y[k1][n2] = t[k1];
+                } else if (4 * m == R) {
+                    y[k1][n2] = mul_mi<INV>(t[k1]);
+                } else {
+                    const T c = (T)w.c[m], s = (T)(INV ? w.s[m] : -w.s[m]);
+                    y[k1][n2] = C{t[k1].x * c - t[k1].y * s, t[k1].x * s + t[k1].y * c};
+                }
+            }
+        }
+#pragma unroll
+        for (int k1 = 0; k1 < P; ++k1) {
+            DFT<Q, INV, C>::run(y[k1]);
+#pragma unroll
+            for (int k2 = 0; k2 < Q; ++k2) v[k1 + P * k2] = y[k1][k2];
+        }
+    }
+};
+template <bool INV, typename C> struct DFT<6, INV, C> : DFTPQ<2, 3, INV, C> {};
+template <bool INV, typename C> struct DFT<9, INV, C> : DFTPQ<3, 3, INV, C> {};
+template <bool INV, typename C> struct DFT<10, INV, C> : DFTPQ<2, 5, INV, C> {};
+template <bool INV, typename C> struct DFT<12, INV, C> : DFTPQ<4, 3, INV, C> {};
+template <bool INV, typename C> struct DFT<14, INV, C> : DFTPQ<2, 7, INV, C> {};
+template <bool INV, typename C> struct DFT<15, INV, C> : DFTPQ<3, 5, INV, C> {};
+template <bool INV, typename C> struct DFT<16, INV, C> : DFTPQ<4, 4, INV, C> {};
+template <bool INV, typename C> struct DFT<18, INV, C> : DFTPQ<2, 9, INV, C> {};
+template <bool INV, typename C> struct DFT<20, INV, C> : DFTPQ<4, 5, INV, C> {};
 template <bool INV, typename C> struct DFT<7, INV, C> : DFTOdd<7, INV, C> {};
 template <bool INV, typename C> struct DFT<11, INV, C> : DFTOdd<11, INV, C> {};
 template <bool INV, typename C> struct DFT<13, INV, C> : DFTOdd<13, INV, C> {};

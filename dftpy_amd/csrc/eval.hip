@@ -16,9 +16,11 @@
 //      semilocal_xc.py:252-290, hartree.py:38, pseudo/__init__.py:228).
 #include <cmath>
 
+#include "fft_fixed.h"
 #include "gspace.h"
 #include "internal.h"
 #include "pointwise.h"
+#include "post.h"
 #include "stream.h"
 #include "reduce.h"
 
@@ -28,10 +30,8 @@ template <typename T>
 __global__ void k_gspace(cpx<T> *__restrict__ spec, long long nc, GParams p, const double *gate) {
     if (gate_off(gate)) return;
     // nc counts the pitched layout; columns iz >= nzc are padding
-    const double rho0 = p.rho0_dev ? *p.rho0_dev : p.rho0;
-    const double tkf = 2.0 * cbrt(3.0 * rho0 * M_PI * M_PI);
-    const double ctf = 0.3 * pow(3.0 * M_PI * M_PI, 2.0 / 3.0);
-    const double wtfac = 5.0 / (9.0 * p.alpha * p.beta * pow(rho0, p.alpha + p.beta - 5.0 / 3.0)) * ctf;
+    double tkf, wtfac;
+    wt_consts(p, tkf, wtfac);
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < nc;
          i += (long long)gridDim.x * blockDim.x) {
         const int iz = (int)(i % p.pitch);
@@ -108,10 +108,6 @@ static int grid_blocks(long long n, int per = 256 * 4) {
     return (int)b;
 }
 
-template <typename T>
-bool xfused_fixed(int n, int var, cpx<T> *data, int batch, long long bs, long long ncols, long long pitch,
-                  long long vp, const void *tw, const GParams &gp, hipStream_t s, const double *gate);
-
 // the WT exponents take the single-spectrum form of wt.py:18-22
 static bool wt_alpha_is_beta(const Plan &P) { return std::fabs(P.alpha - P.beta) < 1e-9; }
 
@@ -131,9 +127,8 @@ static void gspace_apply(Plan &P, cpx<T> *spec, int ns, long long ncp, long long
     if (gp.s_wt2 >= 0) gp.kind[gp.s_wt2] = 1;
     if (fused) {
         const long long ncols = (long long)P.nr[1] * pitch;
-        OFDFT_REQUIRE(xfused_fixed<T>(P.nr[0], P.var_cols[0], spec, ns, ncp, ncols, pitch, P.nzc, P.tw[0], gp, s,
-                                      P.gate),
-                      "fused x pass unavailable");
+        find_ops<T>(P.nr[0])->xfused(P.var_cols[0], spec, ns, ncp, ncols, pitch, P.nzc,
+                                     reinterpret_cast<const cpx<T> *>(P.tw[0]), gp, ~0u, s, P.gate);
     } else {
         hipLaunchKernelGGL((k_gspace<T>), dim3(grid_blocks(ncp)), dim3(256), 0, s, spec, ncp, gp, P.gate);
     }
@@ -182,8 +177,8 @@ __global__ void __launch_bounds__(256) k_gspace_energy(const cpx<T> *__restrict_
             const int kind = p.kind[sl];
             const cpx<T> v = spec[sl * p.bs + e];
             const double a2 = (double)v.x * (double)v.x + (double)v.y * (double)v.y;
-            double f = kernel_val<T>(p, kind, gg, g0, tkf, wtfac);
-            if (nyq) f = 0.5 * (f + kernel_val<T>(p, kind, gg2, g0, tkf, wtfac));
+            double f = kernel_val(p, kind, gg, g0, tkf, wtfac);
+            if (nyq) f = 0.5 * (f + kernel_val(p, kind, gg2, g0, tkf, wtfac));
             const double t = w * (f * p.scale) * a2;
             if (kind == 0)
                 acc_vw += t;
@@ -201,39 +196,13 @@ __global__ void __launch_bounds__(256) k_gspace_energy(const cpx<T> *__restrict_
     }
 }
 
-struct PostParams {
-    int s_vw, s_wt, s_h;
-    int s_wt2 = -1;  // alpha != beta: IFFT(K FFT(rho^alpha))
-    const void *core = nullptr;  // NLCC: the XC term sees rho + core
-    int b56;  // beta == 5/6
-    unsigned terms;
-    double x, y, alpha, beta;
-    long long n;
-    long long bs;  // work batch stride (reals)
-    int want_v, want_e;
-};
-
-// PZ LDA constants (semilocal_xc.py:257-263)
-constexpr double PZ_A = 0.0311, PZ_B = -0.048, PZ_C = 0.0020, PZ_D = -0.0116;
-constexpr double PZ_G = -0.1423, PZ_B1 = 1.0529, PZ_B2 = 0.3334;
-
-// Reciprocal and reciprocal square root: exact division for FP64; the
-// hardware approximations (about 1 ulp) for the FP32-bulk pipeline, whose
-// point-wise work is otherwise dominated by IEEE division sequences.
-template <typename CT> __device__ __forceinline__ CT rcp_p(CT x) { return fm::rcp(x); }
-template <typename CT> __device__ __forceinline__ CT rsq_p(CT x) { return fm::rsq(x); }
-
-template <typename T, typename CT, int VEC>
-__global__ void k_post(const T *__restrict__ rho, const T *__restrict__ work, const T *__restrict__ vloc,
+template <typename T, typename CT, int VEC, int G>
+__global__ void __launch_bounds__(256) k_post(const T *__restrict__ rho, const T *__restrict__ work, const T *__restrict__ vloc,
                        T *__restrict__ pot, double *partials, PostParams p, const double *gate) {
     if (gate_off(gate)) return;
-    const CT ctf = (CT)(0.3 * pow(3.0 * M_PI * M_PI, 2.0 / 3.0));
-    const CT cbrt34pi = (CT)cbrt(3.0 / (4.0 * M_PI));
-    const CT cx_e = (CT)(-3.0 / 4.0 * cbrt(3.0 / M_PI));
-    const CT cx_v = (CT)cbrt(-3.0 / M_PI);
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
     const bool xc_core = (p.terms & OFDFT_TERM_XC) && p.core;
-    pw_groups<VEC>(p.n, [&](long long i0) {
+    pw_each<VEC, G>(p.n, [&](long long i0) {
         // this group's inputs, one vector access per field present
         const PwVec<VEC, T> rv = pw_ld<VEC>(rho, i0);
         PwVec<VEC, T> av{}, cv{}, c2v{}, hv{}, lv{}, corev{}, out{};
@@ -245,92 +214,66 @@ __global__ void k_post(const T *__restrict__ rho, const T *__restrict__ work, co
         if (xc_core) corev = pw_ld<VEC>(reinterpret_cast<const T *>(p.core), i0);
 #pragma unroll
         for (int k = 0; k < VEC; ++k) {
-            const CT r = (CT)rv.v[k];
-            CT v = (CT)0;
-            // one cube root and one square root serve every term (for beta = 5/6)
-            const CT cr = fm::cbrt(r);
-            const CT rc = r < (CT)1e-30 ? (CT)1e-30 : r;
-            const CT c_rc = r < (CT)1e-30 ? (CT)1e-10 : cr;  // cbrt(max(rho, 1e-30))
-            if (p.terms & OFDFT_TERM_TF) {
-                const CT c2 = cr * cr;  // rho^(2/3)
-                if (p.want_e) acc[0] += (double)(ctf * c2 * r);
-                v += (CT)p.x * ((CT)(5.0 / 3.0) * ctf * c2);
-        }
-        if (p.s_vw >= 0) {
-            const CT a = (CT)av.v[k];
-            // 1 / sqrt(rho > 0 ? rho : 1e-30)
-            const CT isq = rsq_p<CT>((r > (CT)0 && r < (CT)1e-30) ? r : rc);
-            const CT vw = (CT)p.y * (a * isq);
-            if (p.want_e && r > (CT)0) acc[1] += (double)(r * vw);
-            v += vw;
-        }
-        if (p.s_wt >= 0 && p.s_wt2 < 0) {
-            const CT c = (CT)cv.v[k];
-            const CT rb_rc = p.b56 ? c_rc * rsq_p<CT>(rc) : fm::pow(rc, (CT)p.beta) * rcp_p<CT>(rc);  // rho^beta / rho
-            const CT vnl = (CT)(2.0 * p.alpha) * rb_rc * c;
-            if (p.want_e) acc[2] += (double)(vnl * r) / (2.0 * p.alpha);
-            v += vnl;
-        } else if (p.s_wt >= 0) {
-            // alpha != beta (wt.py:23-25,44-56): cb = K * rho^beta, ca = K * rho^alpha
-            const CT cb = (CT)cv.v[k];
-            const CT ca = (CT)c2v.v[k];
-            const CT ra = fm::pow(rc, (CT)p.alpha), rb = fm::pow(rc, (CT)p.beta);
-            const CT irc = rcp_p<CT>(rc);
-            if (p.want_e) acc[2] += (double)(ra * cb);
-            v += (CT)p.alpha * ra * irc * cb + (CT)p.beta * rb * irc * ca;
-        }
-        if (p.terms & OFDFT_TERM_XC) {
-            // xc/__init__.py:59-74: with a core density the XC term is
-            // evaluated at rho + core (energy sum_r eps(rho+core)(rho+core) dV)
-            CT rx = r, rc3 = cr;
-            if (p.core) {
-                rx = r + (CT)corev.v[k];
-                rc3 = fm::cbrt(rx);
-            }
-            if (rc3 < (CT)1e-30) rc3 = (CT)1e-30;
-            const CT rs = cbrt34pi * rcp_p<CT>(rc3);
-            CT ec, vc;
-            if (rs < (CT)1) {
-                const CT lr = fm::log(rs);
-                ec = (CT)PZ_A * lr + (CT)PZ_B + (CT)PZ_C * rs * lr + (CT)PZ_D * rs;
-                vc = lr * ((CT)PZ_A + (CT)(2.0 / 3.0 * PZ_C) * rs) + (CT)PZ_B - (CT)(1.0 / 3.0 * PZ_A) +
-                     (CT)(1.0 / 3.0 * (2 * PZ_D - PZ_C)) * rs;
-            } else {
-                const CT sr = fm::sqrt(rs);
-                const CT iden = rcp_p<CT>((CT)1 + (CT)PZ_B1 * sr + (CT)PZ_B2 * rs);
-                ec = (CT)PZ_G * iden;
-                vc = ((CT)PZ_G + (CT)(7.0 / 6.0 * PZ_G * PZ_B1) * sr + (CT)(4.0 / 3.0 * PZ_G * PZ_B2) * rs) *
-                     (iden * iden);
-            }
-            if (p.want_e) acc[3] += (double)((cx_e * rc3 + ec) * rx);
-            v += cx_v * rc3 + vc;
-        }
-        if (p.s_h >= 0) {
-            const CT vh = (CT)hv.v[k];
-            if (p.want_e) acc[4] += 0.5 * (double)vh * (double)r;
-            v += vh;
-        }
-        if (vloc) {
-            const CT vl = (CT)lv.v[k];
-            if (p.want_e) acc[5] += (double)vl * (double)r;
-            v += vl;
-        }
-        acc[6] += (double)r;
-        out.v[k] = (T)v;
+            out.v[k] = (T)post_point<CT>(p, vloc != nullptr, (CT)rv.v[k], (CT)av.v[k], (CT)cv.v[k], (CT)c2v.v[k],
+                                         (CT)hv.v[k], (CT)lv.v[k], (CT)corev.v[k], acc);
         }
         if (p.want_v) pw_st<VEC>(pot, i0, out);
     });
     if (p.want_e) block_sums<7>(acc, partials);
 }
 
-// k_post with the element width the field length allows (stream.h)
+// Launch shape of the point-wise kernels: one element per thread on fields that
+// would leave the chip idle otherwise, else four per access where the length
+// allows.  FP32 then walks the field in a loop of at most 1024 workgroups (g =
+// 0); FP64, whose constants a loop keeps in 100 registers (160^3: 43 us, 36
+// without), unrolls up to four groups per thread, as many as keep the partial
+// sums near 1500 rows (2000 rows cost the one-workgroup final sum 6 us).
+struct PointShape {
+    int vec, g = 1, nb;
+    PointShape(long long n, bool can4, bool fp64) {
+        const bool big = n >= (1LL << 19);
+        vec = can4 && big ? 4 : 1;
+        if (big && !fp64) {
+            g = 0;
+            nb = std::min(reduce_blocks(n), 1024);
+            return;
+        }
+        while (g < 4 && n > 1536LL * 256 * vec * g) g *= vec == 4 ? 2 : 4;
+        const long long per = 256LL * vec * g;
+        nb = (int)((n + per - 1) / per);
+    }
+};
+#define OFDFT_POINT_LAUNCH(K, sh, s, ...)                                                            \
+    do {                                                                                             \
+        const dim3 grid_((sh).nb), blk_(256);                                                        \
+        if constexpr (std::is_same<T, double>::value) {                                              \
+            if ((sh).vec == 4 && (sh).g == 1)                                                        \
+                hipLaunchKernelGGL((K<T, T, 4, 1>), grid_, blk_, 0, s, __VA_ARGS__);                 \
+            else if ((sh).vec == 4 && (sh).g == 2)                                                   \
+                hipLaunchKernelGGL((K<T, T, 4, 2>), grid_, blk_, 0, s, __VA_ARGS__);                 \
+            else if ((sh).vec == 4)                                                                  \
+                hipLaunchKernelGGL((K<T, T, 4, 4>), grid_, blk_, 0, s, __VA_ARGS__);                 \
+            else if ((sh).g == 4)                                                                    \
+                hipLaunchKernelGGL((K<T, T, 1, 4>), grid_, blk_, 0, s, __VA_ARGS__);                 \
+            else                                                                                     \
+                hipLaunchKernelGGL((K<T, T, 1, 1>), grid_, blk_, 0, s, __VA_ARGS__);                 \
+        } else if ((sh).g == 1) {                                                                    \
+            hipLaunchKernelGGL((K<T, T, 1, 1>), grid_, blk_, 0, s, __VA_ARGS__);                     \
+        } else if ((sh).vec == 4) {                                                                  \
+            hipLaunchKernelGGL((K<T, T, 4, 0>), grid_, blk_, 0, s, __VA_ARGS__);                     \
+        } else {                                                                                     \
+            hipLaunchKernelGGL((K<T, T, 1, 0>), grid_, blk_, 0, s, __VA_ARGS__);                     \
+        }                                                                                            \
+    } while (0)
+
+// returns the rows of partial sums
 template <typename T>
-static void launch_post(int nb, hipStream_t s, const T *rho, const T *work, const T *vloc, T *pot, double *partials,
-                        const PostParams &pp, const double *gate) {
-    if (pw_vec(pp.n) == 4 && pw_vec(pp.bs) == 4 && pw_aligned({rho, work, vloc, pot, pp.core}))
-        hipLaunchKernelGGL((k_post<T, T, 4>), dim3(nb), dim3(256), 0, s, rho, work, vloc, pot, partials, pp, gate);
-    else
-        hipLaunchKernelGGL((k_post<T, T, 1>), dim3(nb), dim3(256), 0, s, rho, work, vloc, pot, partials, pp, gate);
+static int launch_post(hipStream_t s, const T *rho, const T *work, const T *vloc, T *pot, double *partials,
+                       const PostParams &pp, const double *gate) {
+    const PointShape sh(pp.n, pw_vec(pp.n) == 4 && pw_vec(pp.bs) == 4 && pw_aligned({rho, work, vloc, pot, pp.core}),
+                        sizeof(T) == 8);
+    OFDFT_POINT_LAUNCH(k_post, sh, s, rho, work, vloc, pot, partials, pp, gate);
+    return sh.nb;
 }
 
 // energies[0..5] = term sums * dV (TF also * x), [6] = their sum + E_ion,
@@ -415,8 +358,7 @@ static void eval_energy(Plan &P, const T *rho, int ns, int s_vw, int s_wt, int s
     pp.want_v = 0;
     pp.want_e = 1;
     const T *vloc = (P.terms & OFDFT_TERM_PP) ? reinterpret_cast<const T *>(P.vloc) : nullptr;
-    const int nb = std::min(reduce_blocks(P.N), 1024);
-    launch_post<T>(nb, s, rho, nullptr, vloc, nullptr, P.red, pp, P.gate);
+    const int nb = launch_post<T>(s, rho, nullptr, vloc, nullptr, P.red, pp, P.gate);
     OFDFT_HIP(hipGetLastError());
     OFDFT_REQUIRE((long long)P.nr[0] * P.nr[1] * P.nzc < (1LL << 31), "energy pass: grid too large");
     hipLaunchKernelGGL((k_gspace_energy<T>), dim3(nb), dim3(256), 0, s, spec, ns, gp, P.y, P.red, P.gate);
@@ -526,8 +468,7 @@ void eval(Plan &P, const T *rho, unsigned calc, T *pot, double *energies, hipStr
     PostParams pp = pipeline_post(P, s_vw, s_wt, s_h, (calc & OFDFT_CALC_V) && pot != nullptr,
                                   (calc & OFDFT_CALC_E) && energies != nullptr, s_wt2);
     const T *vloc = (terms & OFDFT_TERM_PP) ? reinterpret_cast<const T *>(P.vloc) : nullptr;
-    const int nb = std::min(reduce_blocks(P.N), 1024);
-    launch_post<T>(nb, s, rho, work, vloc, pot, P.red, pp, P.gate);
+    const int nb = launch_post<T>(s, rho, work, vloc, pot, P.red, pp, P.gate);
     OFDFT_HIP(hipGetLastError());
     if (pp.want_e) {
         hipLaunchKernelGGL(k_energy_final, dim3(1), dim3(kFinalThreads), 0, s, P.red, nb, energies, P.dV, P.x, P.eion,
@@ -562,7 +503,7 @@ struct FieldParams {
 template <typename T>
 __global__ void k_fields(const T *__restrict__ rho, const T *__restrict__ work, T *__restrict__ edens,
                          T *__restrict__ v2, FieldParams p) {
-    const double ctf = 0.3 * pow(3.0 * M_PI * M_PI, 2.0 / 3.0);
+    const double ctf = kCtf;
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < p.n;
          i += (long long)gridDim.x * blockDim.x) {
         const double r = (double)rho[i];
@@ -665,8 +606,7 @@ template <typename T> void bench_eval_stage(Plan &P, int stage, const T *rho, T 
     } else {
         PostParams pp = pipeline_post(P, s_vw, s_wt, s_h, true, true);
         const T *vloc = (terms & OFDFT_TERM_PP) ? reinterpret_cast<const T *>(P.vloc) : nullptr;
-        const int nb = std::min(reduce_blocks(P.N), 1024);
-        launch_post<T>(nb, s, rho, reinterpret_cast<const T *>(P.work), vloc, pot, P.red, pp, P.gate);
+        launch_post<T>(s, rho, reinterpret_cast<const T *>(P.work), vloc, pot, P.red, pp, P.gate);
     }
     OFDFT_HIP(hipGetLastError());
 }
@@ -726,18 +666,15 @@ void eval_linear(Plan &P, const T *rho, const T *phi, const T *p, hipStream_t s)
 
 // Ap = (V - mu) p + phi dV[2 phi p]  and  sum p.Ap.
 // base_a = 1/2 L(sqrt(rho)) and base_c = C(rho^beta) of the evaluation at rho.
-template <typename T, typename CT, int VEC>
-__global__ void k_hvp(const T *__restrict__ rho, const T *__restrict__ phi,
+template <typename T, typename CT, int VEC, int G>
+__global__ void __launch_bounds__(256) k_hvp(const T *__restrict__ rho, const T *__restrict__ phi,
                       const T *__restrict__ p, const T *__restrict__ pot, const T *__restrict__ work,
                       const T *__restrict__ base_a, const T *__restrict__ base_c, const double *__restrict__ mu,
                       T *__restrict__ Ap, double *partials, PostParams pp, const double *gate) {
     if (gate_off(gate)) return;
-    const CT ctf = (CT)(0.3 * pow(3.0 * M_PI * M_PI, 2.0 / 3.0));
-    const CT cbrt34pi = (CT)cbrt(3.0 / (4.0 * M_PI));
-    const CT cx3 = (CT)(-cbrt(3.0 / M_PI) / 3.0);
     const double m = *mu;
     double acc[1] = {0.0};
-    pw_groups<VEC>(pp.n, [&](long long i0) {
+    pw_each<VEC, G>(pp.n, [&](long long i0) {
         const PwVec<VEC, T> phv = pw_ld<VEC>(phi, i0), pv = pw_ld<VEC>(p, i0), rv = pw_ld<VEC>(rho, i0),
                             potv = pw_ld<VEC>(pot, i0);
         PwVec<VEC, T> bav{}, avw{}, bcv{}, cwt{}, hv{}, out{};
@@ -752,46 +689,8 @@ __global__ void k_hvp(const T *__restrict__ rho, const T *__restrict__ phi,
         if (pp.s_h >= 0) hv = pw_ld<VEC>(work + pp.s_h * pp.bs, i0);
 #pragma unroll
         for (int k = 0; k < VEC; ++k) {
-            const T phi_i = phv.v[k], p_i = pv.v[k];
-            const CT r = (CT)rv.v[k], dr = (CT)(T)(2.0 * (double)phi_i * (double)p_i);  // drho = 2 phi p
-            const CT rp = r > (CT)1e-30 ? r : (CT)1e-30;
-            const CT c_rp = fm::cbrt(rp);
-            const CT ic = rcp_p<CT>(c_rp);  // rho^(-1/3)
-            const CT irp = ic * ic * ic;    // 1 / rho
-            CT dv = (CT)0;
-            if (pp.terms & OFDFT_TERM_TF) dv += (CT)pp.x * (CT)(10.0 / 9.0) * ctf * ic * dr;  // tf.py:38-40
-            if (pp.s_vw >= 0) {
-                const CT isq = rsq_p<CT>((r > (CT)0 && r < (CT)1e-30) ? r : rp);  // 1 / sqrt(rho > 0 ? rho : 1e-30)
-                const CT ds = (CT)0.5 * dr * isq;
-                const CT vwb = (CT)pp.y * (CT)bav.v[k] * isq;
-                dv += ((CT)pp.y * (CT)avw.v[k] - vwb * ds) * isq;
-        }
-        if (pp.s_wt >= 0) {
-            const CT rb1 = pp.b56 ? c_rp * rsq_p<CT>(rp) : fm::pow(rp, (CT)pp.beta - (CT)1);  // rho^(beta-1)
-            dv += (CT)(2.0 * pp.alpha) * (((CT)pp.beta - (CT)1) * rb1 * irp * dr * (CT)bcv.v[k] +
-                                           rb1 * (CT)cwt.v[k]);
-        }
-        if (pp.terms & OFDFT_TERM_XC) {
-            // semilocal_xc.py:291-303
-            const CT rc3 = c_rp;
-            const CT rs = cbrt34pi * ic;
-            CT fc;
-            if (rs < (CT)1) {
-                fc = -(CT)(PZ_A / 3.0) -
-                     ((CT)(PZ_C / 9.0) * (fm::log(rs) * (CT)2 + (CT)1) + (CT)(PZ_D * 2.0 / 9.0)) * rs;
-            } else {
-                const CT ta = (CT)PZ_B1 * fm::sqrt(rs), tb = (CT)PZ_B2 * rs;
-                const CT ide = rcp_p<CT>((CT)1 + ta + tb);
-                fc = (CT)(PZ_G / 36.0) *
-                     ((CT)5 * ta + (CT)7 * ta * ta + (CT)8 * tb + (CT)16 * tb * tb + (CT)21 * ta * tb) *
-                     (ide * ide * ide);
-            }
-            dv += (cx3 * rc3 + fc) * irp * dr;
-        }
-        if (pp.s_h >= 0) dv += (CT)hv.v[k];
-        const double a = ((double)potv.v[k] - m) * (double)p_i + (double)phi_i * (double)dv;
-        out.v[k] = (T)a;
-        acc[0] += (double)p_i * (double)(T)a;
+            out.v[k] = hvp_point<T, CT>(pp, m, phv.v[k], pv.v[k], rv.v[k], potv.v[k], (CT)bav.v[k], (CT)avw.v[k],
+                                        (CT)bcv.v[k], (CT)cwt.v[k], (CT)hv.v[k], acc[0]);
         }
         pw_st<VEC>(Ap, i0, out);
     });
@@ -799,8 +698,8 @@ __global__ void k_hvp(const T *__restrict__ rho, const T *__restrict__ phi,
 }
 
 template <typename T>
-void hvp(Plan &P, const T *rho, const T *phi, const T *p, const T *pot, const T *base_a, const T *base_c,
-         const double *mu, T *Ap, int nb, hipStream_t s) {
+int hvp(Plan &P, const T *rho, const T *phi, const T *p, const T *pot, const T *base_a, const T *base_c,
+         const double *mu, T *Ap, hipStream_t s) {
     OFDFT_REQUIRE(!(P.terms & OFDFT_TERM_LMGP), "the analytic Hessian product does not cover LMGP; use the "
                                                  "finite-difference one");
     OFDFT_REQUIRE(!(P.terms & OFDFT_TERM_WT) || wt_alpha_is_beta(P),
@@ -824,19 +723,18 @@ void hvp(Plan &P, const T *rho, const T *phi, const T *p, const T *pot, const T 
     pp.bs = P.N;
     pp.want_v = 1;
     pp.want_e = 0;
-    if (pw_vec(pp.n) == 4 && pw_aligned({rho, phi, p, pot, P.work, base_a, base_c, Ap}))
-        hipLaunchKernelGGL((k_hvp<T, T, 4>), dim3(nb), dim3(256), 0, s, rho, phi, p, pot,
-                           reinterpret_cast<const T *>(P.work), base_a, base_c, mu, Ap, P.red, pp, P.gate);
-    else
-        hipLaunchKernelGGL((k_hvp<T, T, 1>), dim3(nb), dim3(256), 0, s, rho, phi, p, pot,
-                           reinterpret_cast<const T *>(P.work), base_a, base_c, mu, Ap, P.red, pp, P.gate);
+    const PointShape sh(pp.n, pw_vec(pp.n) == 4 && pw_aligned({rho, phi, p, pot, P.work, base_a, base_c, Ap}),
+                        sizeof(T) == 8);
+    OFDFT_POINT_LAUNCH(k_hvp, sh, s, rho, phi, p, pot, reinterpret_cast<const T *>(P.work), base_a, base_c, mu, Ap,
+                       P.red, pp, P.gate);
     OFDFT_HIP(hipGetLastError());
+    return sh.nb;
 }
 
-template void hvp<float>(Plan &, const float *, const float *, const float *, const float *, const float *,
-                         const float *, const double *, float *, int, hipStream_t);
-template void hvp<double>(Plan &, const double *, const double *, const double *, const double *, const double *,
-                          const double *, const double *, double *, int, hipStream_t);
+template int hvp<float>(Plan &, const float *, const float *, const float *, const float *, const float *,
+                         const float *, const double *, float *, hipStream_t);
+template int hvp<double>(Plan &, const double *, const double *, const double *, const double *, const double *,
+                          const double *, const double *, double *, hipStream_t);
 
 // slots of the FFT terms in P.work after an evaluation: (vW, WT, Hartree), -1 if absent
 void work_slots(const Plan &P, int *slot) {

@@ -15,6 +15,15 @@ namespace fm {
 template <typename T> __device__ __forceinline__ T sqrt(T x) { return ::sqrt(x); }
 template <> __device__ __forceinline__ float sqrt<float>(float x) { return __builtin_amdgcn_sqrtf(x); }
 
+// FP32 square root of x > 0 from the hardware reciprocal root, corrected to
+// within about half an ulp (the vW term multiplies its rounding by G^2)
+__device__ __forceinline__ float sqrt_c(float x) {
+    const float y = __builtin_amdgcn_rsqf(x), g = x * y;
+    // denormals and infinity keep the plain hardware root
+    return x > 1e-37f && x < (float)INFINITY ? __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g)
+                                             : __builtin_amdgcn_sqrtf(x);
+}
+
 template <typename T> __device__ __forceinline__ T rcp(T x) { return (T)1 / x; }
 template <> __device__ __forceinline__ float rcp<float>(float x) { return __builtin_amdgcn_rcpf(x); }
 
@@ -46,6 +55,57 @@ template <> __device__ __forceinline__ float cbrt<float>(float x) {
     const float r = __builtin_amdgcn_rcpf(y * y);
     const float z = y - (y - x * r) * (1.0f / 3.0f);
     return x > 0.0f ? z : 0.0f;
+}
+
+// a^(-1/6) for finite a > 0 in FP64: one third-order step from the FP32
+// hardware log2 and exp2 of a scaled by a power of 2^6 into [1/2, 32), so
+// every exponent (denormals too) has the same seed.  Below 1 ulp; about 20
+// instructions, where the library's cbrt, sqrt and division, whose results
+// the powers of it give, take ten times that.
+__device__ __forceinline__ double inv_sixth_root(double a) {
+    const int e = __builtin_amdgcn_frexp_exp(a);
+    const int q = (e + 1536) / 6 - 256;  // floor(e / 6)
+    const double m = __builtin_amdgcn_ldexp(__builtin_amdgcn_frexp_mant(a), e - 6 * q);
+    double s = (double)__builtin_amdgcn_exp2f(__builtin_amdgcn_logf((float)m) * (-1.0f / 6.0f));
+    const double s3 = s * s * s;
+    const double h = __builtin_fma(-m, s3 * s3, 1.0);
+    s = __builtin_fma(s * h, __builtin_fma(h, 7.0 / 72.0, 1.0 / 6.0), s);
+    return __builtin_amdgcn_ldexp(s, -q);
+}
+// square root, reciprocal square root and cube root of a > 0 from s =
+// a^(-1/6), each with one correction
+__device__ __forceinline__ double sqrt_s(double a, double s) {
+    const double s3 = s * s * s, y = a * s3;
+    return __builtin_fma(__builtin_fma(-y, y, a), 0.5 * s3, y);
+}
+__device__ __forceinline__ double rsq_s(double a, double s) {
+    const double y = s * s * s;
+    return __builtin_fma(__builtin_fma(-a * y, y, 1.0), 0.5 * y, y);
+}
+__device__ __forceinline__ double cbrt_s(double a, double s) {
+    const double s2 = s * s, s4 = s2 * s2, y = a * s4;
+    return __builtin_fma(__builtin_fma(-y * y, y, a), s4 * (1.0 / 3.0), y);
+}
+// square root of x >= 0 in FP64 for normal x or 0: a Goldschmidt step on the
+// hardware reciprocal root and a correction
+__device__ __forceinline__ double sqrt_n(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, r, g);
+    h = __builtin_fma(h, r, h);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    return x > 0.0 ? g : x;
+}
+__device__ __forceinline__ float sqrt_n(float x) { return sqrt(x); }
+// a / b in FP64 for normal b and quotient: two Newton steps on the hardware
+// reciprocal and a correction of the quotient
+__device__ __forceinline__ double div_n(double a, double b) {
+    double r = __builtin_amdgcn_rcp(b);
+    r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
+    r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
+    const double q = a * r;
+    return __builtin_fma(__builtin_fma(-b, q, a), r, q);
 }
 
 }  // namespace fm

@@ -18,6 +18,7 @@
 #include <mutex>
 
 #include "dft.h"
+#include "fft_fixed.h"
 #include "internal.h"
 #include "pointwise.h"
 
@@ -286,24 +287,17 @@ __global__ void k_rows_c2c(const cpx<T> *__restrict__ in, cpx<T> *__restrict__ o
 }
 
 // ------------------------------------------------------------------ host side
-bool fixed_size(int n);
-template <typename T>
-bool cols_fixed(int n, int var, bool inv, const cpx<T> *in, cpx<T> *out, int batch, long long bs, long long ncols,
-                long long P, long long Q, long long S, long long vp, const void *tw, double scale, hipStream_t s,
-                const double *gate);
-template <typename T>
-bool r2c_fixed(int n, int var, const T *in, cpx<T> *out, int batch, long long in_bs, long long out_bs,
-               long long nrows, long long opitch, const void *tw, double scale, const Prologue &pro, double *partials,
-               int sum_slot, hipStream_t s, const double *gate);
-template <typename T>
-bool c2r_fixed(int n, int var, const cpx<T> *in, T *out, int batch, long long in_bs, long long out_bs,
-               long long nrows, long long ipitch, const void *tw, double scale, hipStream_t s, const double *gate);
-int r2c_fixed_tiles(int n, int var, int prec, int batch, long long nrows);
-
 int r2c_num_partials(const Plan &P, int batch) {
     const long long nrows = (long long)P.nr[0] * P.nr[1];
-    if (P.use_fixed && fixed_size(P.nr[2])) return r2c_fixed_tiles(P.nr[2], P.var_r2c, P.prec, batch, nrows);
+    if (P.use_fixed && fixed_size(P.nr[2]))
+        return P.prec == OFDFT_FP64 ? find_ops<double>(P.nr[2])->r2c_tiles(P.var_r2c, batch, nrows)
+                                    : find_ops<float>(P.nr[2])->r2c_tiles(P.var_r2c, batch, nrows);
     return (int)((nrows + P.rows_r2c.tile - 1) / P.rows_r2c.tile);
+}
+
+// the size-specialised passes of an axis, or null
+template <typename T> static const SizeOps<T> *axis_ops(const Plan &P, int axis) {
+    return P.use_fixed ? find_ops<T>(P.nr[axis]) : nullptr;
 }
 
 long long pipe_pitch(const Plan &P) {
@@ -434,12 +428,12 @@ void plan_fft_free(Plan &P) {
 
 template <typename T>
 void fft_cols(Plan &P, int axis, bool full_grid, bool inverse, const cpx<T> *in, cpx<T> *out, int batch,
-              long long bs, double scale, hipStream_t s, long long pitch) {
+              long long bs, double scale, hipStream_t s, long long pitch, unsigned mask) {
     const int n = P.nr[axis];
     const long long zlen = full_grid ? P.nr[2] : P.nzc;
     if (pitch <= 0) pitch = zlen;
     if (n == 1 && in == out && scale == 1.0) return;
-    if (P.use_fixed && fixed_size(n)) {
+    if (const SizeOps<T> *ops = axis_ops<T>(P, axis)) {
         // flattened pencils: base(c) = (c / Pp) * Qq + c % Pp, stride Ss; columns
         // at or beyond zlen within a pitched row are padding and skipped
         long long ncols, Pp, Qq, Ss;
@@ -453,13 +447,13 @@ void fft_cols(Plan &P, int axis, bool full_grid, bool inverse, const cpx<T> *in,
             Pp = Qq = pitch;
             Ss = ncols;
         }
-        cols_fixed<T>(n, P.var_cols[axis], inverse, in, out, batch, bs, ncols, Pp, Qq, Ss, zlen, P.tw[axis], scale, s,
-                      P.gate);
+        ops->cols(P.var_cols[axis], inverse, in, out, batch, bs, ncols, Pp, Qq, Ss, zlen,
+                  reinterpret_cast<const cpx<T> *>(P.tw[axis]), (T)scale, mask, s, P.gate);
         OFDFT_HIP(hipGetLastError());
         return;
     }
     OFDFT_REQUIRE(pitch == zlen, "generic column pass needs an unpadded layout");
-    OFDFT_REQUIRE(P.gate == nullptr, "gated launch of a generic FFT pass");
+    OFDFT_REQUIRE(P.gate == nullptr && mask == ~0u, "gated launch of a generic FFT pass");
     long long M, outer;
     PassShape sh;
     if (axis == 1) {
@@ -504,8 +498,10 @@ void fft_r2c(Plan &P, const T *in, cpx<T> *out, int batch, long long in_bs, long
     const PassShape sh = P.rows_r2c;
     const cpx<T> *tw = reinterpret_cast<const cpx<T> *>(P.tw[2]);
     const bool last_z = (P.nr[0] == 1 && P.nr[1] == 1);
-    if (!(P.use_fixed && r2c_fixed<T>(P.nr[2], P.var_r2c, in, out, batch, in_bs, out_bs, nrows, pitch, P.tw[2],
-                                      last_z ? scale : 1.0, pr, sum_partials, sum_slot, s, P.gate))) {
+    if (const SizeOps<T> *ops = axis_ops<T>(P, 2)) {
+        ops->r2c(P.var_r2c, in, out, batch, in_bs, out_bs, nrows, pitch, tw, (T)(last_z ? scale : 1.0), pr, sum_partials,
+                 sum_slot, s, P.gate);
+    } else {
         OFDFT_REQUIRE(pitch == P.nzc, "generic R2C pass needs an unpadded layout");
         OFDFT_REQUIRE(P.gate == nullptr, "gated launch of a generic FFT pass");
         dim3 grid((unsigned)((nrows + sh.tile - 1) / sh.tile), (unsigned)batch);
@@ -534,8 +530,9 @@ void fft_c2r(Plan &P, const cpx<T> *in, cpx<T> *tmp, T *out, int batch, long lon
     const long long nrows = (long long)P.nr[0] * P.nr[1];
     const PassShape sh = P.rows_c2r;
     const cpx<T> *tw = reinterpret_cast<const cpx<T> *>(P.tw[2]);
-    if (!(P.use_fixed && c2r_fixed<T>(P.nr[2], P.var_c2r, src, out, batch, src_bs, out_bs, nrows, pitch, P.tw[2],
-                                      scale, s, P.gate))) {
+    if (const SizeOps<T> *ops = axis_ops<T>(P, 2)) {
+        ops->c2r(P.var_c2r, src, out, batch, src_bs, out_bs, nrows, pitch, tw, (T)scale, s, P.gate);
+    } else {
         OFDFT_REQUIRE(pitch == P.nzc, "generic C2R pass needs an unpadded layout");
         OFDFT_REQUIRE(P.gate == nullptr, "gated launch of a generic FFT pass");
         dim3 grid((unsigned)((nrows + sh.tile - 1) / sh.tile), (unsigned)batch);
@@ -555,7 +552,12 @@ void fft_c2c(Plan &P, const cpx<T> *in, cpx<T> *out, bool inverse, int batch, lo
     const bool last_z = (P.nr[0] == 1 && P.nr[1] == 1);
     const T sz = (T)(last_z ? scale : 1.0);
     OFDFT_REQUIRE(P.gate == nullptr, "gated launch of a generic FFT pass");
-    if (inverse)
+    if (const SizeOps<T> *ops = axis_ops<T>(P, 2)) {
+        if (inverse)
+            ops->rows_inv(0, in, out, batch, bs, nrows, tw, sz, ApplyArgs<T>{}, 0, ~0u, s, nullptr);
+        else
+            ops->rows_fwd(in, out, batch, bs, nrows, tw, sz, nullptr, ~0u, s, nullptr);
+    } else if (inverse)
         hipLaunchKernelGGL((k_rows_c2c<T, true>), grid, dim3(sh.threads), sh.lds, s, in, out, bs, nrows, P.nr[2],
                            P.ax[2], tw, sh.tile, sz);
     else
@@ -571,8 +573,9 @@ template <typename T>
 void bench_rows_r2c(Plan &P, const T *in, cpx<T> *out, int batch, const Prologue *pro, hipStream_t s) {
     const long long nrows = (long long)P.nr[0] * P.nr[1];
     const long long pitch = pipe_pitch(P);
-    if (P.use_fixed && r2c_fixed<T>(P.nr[2], P.var_r2c, in, out, batch, 0LL, (long long)P.nr[0] * P.nr[1] * pitch, nrows, pitch,
-                                    P.tw[2], 1.0, *pro, nullptr, -1, s, nullptr)) {
+    if (const SizeOps<T> *ops = axis_ops<T>(P, 2)) {
+        ops->r2c(P.var_r2c, in, out, batch, 0LL, (long long)P.nr[0] * P.nr[1] * pitch, nrows, pitch,
+                 reinterpret_cast<const cpx<T> *>(P.tw[2]), (T)1, *pro, nullptr, -1, s, nullptr);
         OFDFT_HIP(hipGetLastError());
         return;
     }
@@ -587,8 +590,9 @@ void bench_rows_r2c(Plan &P, const T *in, cpx<T> *out, int batch, const Prologue
 template <typename T> void bench_rows_c2r(Plan &P, const cpx<T> *in, T *out, int batch, hipStream_t s) {
     const long long nrows = (long long)P.nr[0] * P.nr[1];
     const long long pitch = pipe_pitch(P);
-    if (P.use_fixed && c2r_fixed<T>(P.nr[2], P.var_c2r, in, out, batch, (long long)P.nr[0] * P.nr[1] * pitch, P.N, nrows, pitch,
-                                    P.tw[2], 1.0, s, nullptr)) {
+    if (const SizeOps<T> *ops = axis_ops<T>(P, 2)) {
+        ops->c2r(P.var_c2r, in, out, batch, (long long)P.nr[0] * P.nr[1] * pitch, P.N, nrows, pitch,
+                 reinterpret_cast<const cpx<T> *>(P.tw[2]), (T)1, s, nullptr);
         OFDFT_HIP(hipGetLastError());
         return;
     }
@@ -600,7 +604,7 @@ template <typename T> void bench_rows_c2r(Plan &P, const cpx<T> *in, T *out, int
 }
 
 // ------------------------------------------------------------------ autotuner
-// Times every tile variant of the size-specialised passes on the plan's own
+// Times both tiles of each size-specialised pass on the plan's own
 // shapes (3 spectra, the evaluation pipeline's batch) and keeps the fastest.
 // Runs on the plan's workspace; the data are whatever it holds.
 template <typename F> static float time_launches(hipStream_t s, int iters, F &&f) {
@@ -625,13 +629,13 @@ template <typename T> static void autotune_t(Plan &P, hipStream_t s, float *time
     cpx<T> *spec = reinterpret_cast<cpx<T> *>(P.spec);
     T *work = reinterpret_cast<T *>(P.work);
     const int iters = 4;
-    // times: kColVariants per slot; the row passes have kTileVariants
-    auto pick = [&](int *var, int slot, int nvar, auto &&run) {
+    // times: kColVariants per slot
+    auto pick = [&](int *var, int slot, auto &&run) {
         float best = 1e30f;
         int bv = 0;
         for (int v = 0; v < kColVariants; ++v)
             if (times) times[slot * kColVariants + v] = -1.0f;
-        for (int v = 0; v < nvar; ++v) {
+        for (int v = 0; v < kTiles; ++v) {
             *var = v;
             const float t = time_launches(s, iters, run);
             if (times) times[slot * kColVariants + v] = t;
@@ -648,14 +652,14 @@ template <typename T> static void autotune_t(Plan &P, hipStream_t s, float *time
         pro.code[1] = OP_POW_BETA;
         pro.beta = P.beta;
         pro.b56 = 1;
-        pick(&P.var_r2c, 0, kTileVariants, [&] { bench_rows_r2c<T>(P, work, spec, 3, &pro, s); });
-        pick(&P.var_c2r, 1, kTileVariants, [&] { bench_rows_c2r<T>(P, spec, work, 3, s); });
+        pick(&P.var_r2c, 0, [&] { bench_rows_r2c<T>(P, work, spec, 3, &pro, s); });
+        pick(&P.var_c2r, 1, [&] { bench_rows_c2r<T>(P, spec, work, 3, s); });
     }
     // the x variant is timed on the pass the evaluation runs: the fused
     // forward x, G-space multiply and inverse x where the axis has one
     for (int axis = 0; axis < 2; ++axis)
         if (fixed_size(P.nr[axis]))
-            pick(&P.var_cols[axis], 2 + axis, kColVariants, [&] {
+            pick(&P.var_cols[axis], 2 + axis, [&] {
                 if (axis != 0 || !bench_xfused<T>(P, s))
                     fft_cols<T>(P, axis, false, false, spec, spec, 3, ncp, 1.0, s, pitch);
             });
@@ -663,8 +667,7 @@ template <typename T> static void autotune_t(Plan &P, hipStream_t s, float *time
 
 // The variants chosen for a grid shape and precision are kept for the rest of
 // the process: every later plan of that shape takes them without timing, so
-// all plans of a shape transform identically (the radix order changes the
-// rounding) whichever thread or stream created them.
+// all plans of a shape run the same kernels whichever thread or stream created them.
 void plan_autotune(Plan &P, hipStream_t s, float *times) {
     if (!P.use_fixed) return;
     using Key = std::array<int, 5>;
@@ -697,7 +700,7 @@ template void bench_rows_c2r<double>(Plan &, const double2 *, double *, int, hip
 
 #define INST(T)                                                                                               \
     template void fft_cols<T>(Plan &, int, bool, bool, const cpx<T> *, cpx<T> *, int, long long, double,       \
-                              hipStream_t, long long);                                                        \
+                              hipStream_t, long long, unsigned);                                              \
     template void fft_r2c<T>(Plan &, const T *, cpx<T> *, int, long long, long long, double, const Prologue *, \
                              double *, hipStream_t, long long, bool);                                               \
     template void fft_c2r<T>(Plan &, const cpx<T> *, cpx<T> *, T *, int, long long, long long, long long,      \

@@ -1,16 +1,24 @@
-// Size-specialised FFT passes for the common 2/3/5-smooth lengths (kernels and
-// launch templates; instantiated per precision in fft_fixed_f32.hip and
-// fft_fixed_f64.hip).
+// Size-specialised FFT passes: every even length from 16 to 256 with primes up
+// to 13, which is what a grid chosen for an FFT has (kernels and launchers;
+// instantiated per precision and range of lengths in fft_fixed_f32_*.hip and
+// fft_fixed_f64_*.hip).
 //
-// The length N, the tile and the radix sequence are compile-time, so all
-// index arithmetic folds to shifts and constant multiplies.  The first radix
-// stage reads its inputs straight from HBM into registers and the last stage
-// (column passes, C2R rows) writes straight back, both coalesced across the
-// `TILE` adjacent pencils of a workgroup; intermediate stages exchange
-// through LDS.  Column passes address a flattened set of pencils
-// c in [0, ncols): base(c) = (c / P) * Q + c % P, element stride S, which
-// covers the y pass (P = nzc, Q = ny*nzc, S = nzc) and the x pass
-// (P = Q = S = ny*nzc) without partial tiles at plane boundaries.
+// The length, the tile and the radices are compile-time, so all index
+// arithmetic folds to shifts and constant multiplies.  The first DFT takes its
+// inputs from HBM into registers and the last one writes straight back (column
+// and complex row passes); between DFTs the elements cross LDS once.  Few
+// large radices (two, where they fit) mean few crossings and barriers, which
+// bound FP32; their registers cost occupancy, which bounds FP64: radices stop
+// at 20 and 13.  160^3, three spectra: FP32 x pass with the multiply 38 us with
+// 8 4 5, 26 with 10 16; FP64 column passes take 126 registers with 10 16 and 50
+// with 4 5 8 (33 us either way), the z C2R 37 and 33 us.  A length without
+// passes of its own takes the generic kernels (fft.hip): 52 x 78 x 104, FP64,
+// three spectra: y pass 29 us there, 4.5 here.
+//
+// Column passes address a flattened set of pencils c in [0, ncols): base(c) =
+// (c / P) * Q + c % P, element stride S, which covers the y pass (P = nzc, Q =
+// ny*nzc, S = nzc) and the x pass (P = Q = S = ny*nzc) without partial tiles
+// at plane boundaries.
 #pragma once
 #include <algorithm>
 #include <type_traits>
@@ -19,505 +27,477 @@
 #include "gspace.h"
 #include "internal.h"
 #include "pointwise.h"
+#include "post.h"
+#include "stream.h"
 
 namespace ofdft {
 
-struct StageList {
-    int nst;
-    int rad[kMaxStages];
-    int rmin;
+struct Radices {
+    int n = 0;  // number of DFTs, 0: no such split
+    int r[3] = {1, 1, 1};
 };
-
-// radices 8/4/2 for the power of two (8s first, 4 4 instead of 8 2), then 5, 3
-constexpr StageList factorize(int n) {
-    StageList s{};
-    s.nst = 0;
-    s.rmin = 64;
-    int m = n, e2 = 0;
-    while (m % 2 == 0) {
-        m /= 2;
-        ++e2;
-    }
-    int r8 = 0, r4 = 0, r2 = 0;
-    if (e2 % 3 == 0) {
-        r8 = e2 / 3;
-    } else if (e2 % 3 == 1) {
-        if (e2 >= 4) {
-            r8 = e2 / 3 - 1;
-            r4 = 2;
-        } else {
-            r2 = 1;
+// two or three factors up to `most`, the largest as small and then the
+// smallest as large as possible, in ascending order (the first DFT has the
+// most threads, the last leaves the others idle)
+constexpr Radices split(int n, int most) {
+    Radices s{};
+    for (int a = 2; a * a <= n; ++a)
+        if (n % a == 0 && n / a <= most) {
+            s.n = 2;
+            s.r[0] = a;
+            s.r[1] = n / a;
         }
-    } else {
-        r8 = e2 / 3;
-        r4 = 1;
-    }
-    for (int i = 0; i < r8; ++i) s.rad[s.nst++] = 8;
-    for (int i = 0; i < r4; ++i) s.rad[s.nst++] = 4;
-    for (int i = 0; i < r2; ++i) s.rad[s.nst++] = 2;
-    while (m % 5 == 0) {
-        m /= 5;
-        s.rad[s.nst++] = 5;
-    }
-    while (m % 3 == 0) {
-        m /= 3;
-        s.rad[s.nst++] = 3;
-    }
-    for (int i = 0; i < s.nst; ++i) s.rmin = s.rad[i] < s.rmin ? s.rad[i] : s.rmin;
-    if (m != 1) s.nst = -1;
-    return s;
-}
-
-// radix order ORD: 0 as factorize lists it (8s first); 1 reversed (the odd
-// radices first), a variant of the column passes the autotuner times
-constexpr StageList factorize_ord(int n, int ord) {
-    StageList s = factorize(n);
-    if (ord == 1)
-        for (int i = 0, k = s.nst - 1; i < k; ++i, --k) {
-            const int t = s.rad[i];
-            s.rad[i] = s.rad[k];
-            s.rad[k] = t;
+    if (s.n) return s;
+    int top = most + 1;
+    for (int a = 2; a * a * a <= n; ++a)
+        for (int b = a; a * b * b <= n; ++b) {
+            const int c = n / (a * b);
+            if (n % (a * b) == 0 && c <= top) {
+                top = c;
+                s.n = 3;
+                s.r[0] = a;
+                s.r[1] = b;
+                s.r[2] = c;
+            }
         }
     return s;
 }
 
-template <int N, int ORD = 0> struct SL {
-    static constexpr StageList s = factorize_ord(N, ORD);
-    static constexpr int nst = s.nst;
-    static constexpr int rmin = s.rmin;
-    static constexpr int tpp = N / s.rmin;  // threads per pencil
-    template <int I> static constexpr int rad() { return s.rad[I]; }
+// the DFTs of length N; REV: in the opposite order
+template <typename T, int N> struct SL {
+    // FP64: 14 where 13 leaves only a split from 2 (98, 154, 182)
+    static constexpr int most = sizeof(T) == 4 ? 20 : (split(N, 13).r[0] > 2 ? 13 : 14);
+    static constexpr Radices s = split(N, most);
+    static_assert(s.n >= 2, "length without a split");
+    static constexpr int n = s.n;
+    static constexpr int TP = N / s.r[0];  // threads per pencil
+    template <bool REV, int I> static constexpr int rad() { return REV ? s.r[n - 1 - I] : s.r[I]; }
+    static constexpr int first = s.r[0], last = s.r[n - 1];
 };
 
-template <typename C> struct Real;
-template <> struct Real<float2> { using type = float; };
-template <> struct Real<double2> { using type = double; };
+// Which butterfly j of which pencil a thread takes in a DFT of NB butterflies
+// per pencil, and where the pencil's elements are in LDS.  Columns: TILE
+// adjacent pencils, the pencil fixed per thread (its column in HBM).  Rows:
+// NPEN pencils LD apart, the butterflies of all pencils packed onto the first
+// threads, so that a large radix leaves whole waves idle and not lanes of all.
+template <int TILE> struct ColMap {
+    static constexpr int STRIDE = TILE;
+    template <int NB> struct At {
+        int pen, j, base;
+        bool act;
+        __device__ __forceinline__ explicit At(int t) : pen(t % TILE), j(t / TILE), base(pen), act(j < NB) {}
+    };
+};
+template <int NPEN, int LD> struct RowMap {
+    static constexpr int STRIDE = 1;
+    template <int NB> struct At {
+        int pen, j, base;
+        bool act;
+        __device__ __forceinline__ explicit At(int t) : pen(t / NB), j(t - pen * NB), base(pen * LD), act(pen < NPEN) {}
+    };
+};
 
-// ---------------------------------------------------------------- column pass
-// One stage for TILE pencils, pencil element e of pencil p at buf[e*TILE + p].
-template <typename C, int N, int TILE, int R, int NS, bool INV, bool FIRST, bool LAST>
-__device__ __forceinline__ void cstage(C *buf, const C *tw, const C *__restrict__ src, C *__restrict__ dst,
-                                       long long S, bool valid, int pen, int j, typename Real<C>::type scale) {
-    using T = typename Real<C>::type;
-    constexpr int NB = N / R;
-    const bool act = j < NB;
-    C v[R];
-    if (act) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (FIRST)
-                v[r] = valid ? src[(long long)(j + r * NB) * S] : C{(T)0, (T)0};
-            else
-                v[r] = buf[(j + r * NB) * TILE + pen];
-        }
-        if (NS > 1) {
-            const int k = j % NS;
+// DFT I and the ones after it, from the inputs v (elements j + r N / R of the
+// thread's butterfly); done() gets the butterfly and outputs of the last one
+// (elements j + r N / R again).  Twiddles w^(r k) from the LDS table.
+template <typename T, int N, typename MAP, bool INV, bool REV, int I, int NS, typename C, int R, typename F>
+__device__ __forceinline__ void dfts(C *buf, const C *tw, C (&v)[R], F &&done) {
+    using L = SL<T, N>;
+    const typename MAP::template At<N / R> m((int)threadIdx.x);
+    if (m.act) {
+        if constexpr (NS > 1) {
+            const int k = m.j % NS;
 #pragma unroll
             for (int r = 1; r < R; ++r) {
-                C w = tw[(r * k * (N / (NS * R))) % N];
+                C w = tw[r * k * (N / (NS * R))];
                 if (INV) w.y = -w.y;
                 v[r] = cmul(v[r], w);
             }
         }
-    }
-    if (!FIRST || LAST) __syncthreads();
-    if (act) {
         DFT<R, INV, C>::run(v);
-        const int k = j % NS;
-        const int d = (j / NS) * NS * R + k;
+    }
+    if constexpr (I + 1 == L::n) {
+        done(m, v);
+    } else {
+        if constexpr (I > 0) __syncthreads();  // everyone has read the last exchange
+        if (m.act) {
+            const int d = (m.j / NS) * NS * R + m.j % NS;
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (LAST) {
-                if (valid) dst[(long long)(d + r * NS) * S] = C{v[r].x * scale, v[r].y * scale};
-            } else {
-                buf[(d + r * NS) * TILE + pen] = v[r];
-            }
+            for (int r = 0; r < R; ++r) buf[m.base + (d + r * NS) * MAP::STRIDE] = v[r];
         }
-    }
-    if (!LAST) __syncthreads();
-}
-
-template <typename C, int N, int TILE, bool INV, int I, int NS, int ORD>
-__device__ __forceinline__ void cstages(C *buf, const C *tw, const C *src, C *dst, long long S, bool valid, int pen,
-                                        int j, typename Real<C>::type scale) {
-    if constexpr (I < SL<N, ORD>::nst) {
-        constexpr int R = SL<N, ORD>::template rad<I>();
-        cstage<C, N, TILE, R, NS, INV, I == 0, I == SL<N, ORD>::nst - 1>(buf, tw, src, dst, S, valid, pen, j, scale);
-        cstages<C, N, TILE, INV, I + 1, NS * R, ORD>(buf, tw, src, dst, S, valid, pen, j, scale);
+        __syncthreads();
+        constexpr int R2 = L::template rad<REV, I + 1>();
+        const typename MAP::template At<N / R2> m2((int)threadIdx.x);
+        C u[R2];
+        if (m2.act) {
+#pragma unroll
+            for (int r = 0; r < R2; ++r) u[r] = buf[m2.base + (m2.j + r * (N / R2)) * MAP::STRIDE];
+        }
+        dfts<T, N, MAP, INV, REV, I + 1, NS * R>(buf, tw, u, done);
     }
 }
 
-template <typename T, int N, int TILE, bool INV, int ORD>
-__global__ void __launch_bounds__(TILE *SL<N>::tpp)
-    k_cols_f(const cpx<T> *__restrict__ in, cpx<T> *__restrict__ out, long long bs, long long ncols, long long P,
-             long long Q, long long S, long long vp, const cpx<T> *__restrict__ twg, T scale, const double *gate) {
-    if (gate_off(gate)) return;
+// runs of a batch that a launch leaves out (a set bit takes part)
+__device__ __forceinline__ bool run_off(unsigned mask, unsigned b) { return b < 32 && !((mask >> b) & 1u); }
+
+// ---------------------------------------------------------------- column pass
+template <typename T, int N, int TILE, bool INV>
+__global__ void __launch_bounds__((TILE *SL<T, N>::TP))
+    k_cols_f(const cpx<T> *in, cpx<T> *out, long long bs, unsigned ncols, unsigned P, long long Q, long long S,
+             unsigned vp, const cpx<T> *__restrict__ twg, T scale, unsigned mask, const double *gate) {
+    if (gate_off(gate) || run_off(mask, blockIdx.y)) return;
     using C = cpx<T>;
+    constexpr int R = SL<T, N>::first, TP = SL<T, N>::TP;
     __shared__ C tw[N];
     __shared__ C buf[N * TILE];
     const int pen = threadIdx.x % TILE;
     const int j = threadIdx.x / TILE;
-    for (int i = threadIdx.x; i < N; i += TILE * SL<N>::tpp) tw[i] = twg[i];
-    const long long c = (long long)blockIdx.x * TILE + pen;
-    const long long cp = c % P;
+    const unsigned c = blockIdx.x * TILE + pen;
+    const unsigned row = c / P, cp = c - row * P;
     const bool valid = c < ncols && cp < vp;  // pad columns of a pitched layout are skipped
-    const long long base = valid ? (c / P) * Q + cp : 0;
-    const long long off = (long long)blockIdx.y * bs + base;
-    cstages<C, N, TILE, INV, 0, 1, ORD>(buf, tw, in + off, out + off, S, valid, pen, j, scale);
+    const long long off = (long long)blockIdx.y * bs + (valid ? (long long)row * Q + cp : 0) + j * S;
+    C v[R];
+    const C *src = in + off;
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r] = valid ? src[r * TP * S] : C{(T)0, (T)0};
+    for (int i = threadIdx.x; i < N; i += TILE * TP) tw[i] = twg[i];
+    dfts<T, N, ColMap<TILE>, INV, false, 0, 1>(buf, tw, v, [&](auto &m, auto &u) {
+        constexpr int RL = SL<T, N>::last;
+        if (!valid || !m.act) return;
+        C *dst = out + off;
+#pragma unroll
+        for (int r = 0; r < RL; ++r) dst[r * (N / RL) * S] = C{u[r].x * scale, u[r].y * scale};
+    });
 }
 
-// Stages with a choice of source and destination: GIN reads the first stage
-// from HBM (else from LDS), GOUT writes the last stage to HBM (else to LDS in
-// natural order).
-template <typename C, int N, int TILE, bool INV, int I, int NS, bool GIN, bool GOUT, int ORD>
-__device__ __forceinline__ void cstages_io(C *buf, const C *tw, const C *src, C *dst, long long S, bool valid,
-                                           int pen, int j, typename Real<C>::type scale) {
-    if constexpr (I < SL<N, ORD>::nst) {
-        constexpr int R = SL<N, ORD>::template rad<I>();
-        cstage<C, N, TILE, R, NS, INV, GIN && I == 0, GOUT && I == SL<N, ORD>::nst - 1>(buf, tw, src, dst, S, valid,
-                                                                                         pen, j, scale);
-        cstages_io<C, N, TILE, INV, I + 1, NS * R, GIN, GOUT, ORD>(buf, tw, src, dst, S, valid, pen, j, scale);
+// G-space factors of the elements e = j, j + TP, ... of one (iy, iz) column,
+// into fac[e * TILE], from |G|^2 of the column's fixed part plus fx * b1 in
+// the plan precision (the kinetic operator's in FP64).  Unrolled: around a
+// loop the compiler keeps the constants of the FP64 functions in 100
+// registers more.
+template <typename T, int N, int TILE>
+__device__ __forceinline__ void xfactors(T *fac, const GParams &gp, int kind, int iy, int iz, int j, double tkf,
+                                         double wtfac) {
+    constexpr int TP = SL<T, N>::TP;
+    const int fy = ffreq(iy, gp.ny);
+    // kinetic: the complex grid (fftfreq on all axes)
+    const int fz = kind == 4 ? ffreq(iz, gp.nz) : (gp.full ? wrapf(iz, gp.nz) : iz);
+    const double cx = fy * gp.B[3] + fz * gp.B[6], cy = fy * gp.B[4] + fz * gp.B[7], cz = fy * gp.B[5] + fz * gp.B[8];
+    const bool yz0 = iy == 0 && iz == 0;
+    const bool yznyq =
+        gp.full && (((gp.ny & 1) == 0 && iy == gp.ny / 2) || ((gp.nz & 1) == 0 && iz == gp.nz / 2));
+    auto each = [&](auto one, auto &&val) {
+        using CT = decltype(one);
+        const CT bx = (CT)gp.B[0], by = (CT)gp.B[1], bz = (CT)gp.B[2], dx = (CT)cx, dy = (CT)cy, dz = (CT)cz;
+#pragma unroll
+        for (int i = 0; i < N / TP; ++i) {
+            const int e = j + i * TP;
+            const CT fx = (CT)ffreq(e, N);
+            const CT gx = fx * bx + dx, gy = fx * by + dy, gz = fx * bz + dz;
+            CT f = val(gx * gx + gy * gy + gz * gz, yz0 && e == 0);
+            // a Nyquist point of a full grid: the mean with the alias partner
+            if (kind != 4 && (yznyq || (gp.full && 2 * e == N)))
+                f = (CT)0.5 * (f + val((CT)gsq(gp.B, wrapf(-ffreq(e, N), N), wrapf(-fy, gp.ny), wrapf(-fz, gp.nz)),
+                                       false));
+            fac[e * TILE] = (T)f;
+        }
+    };
+    const T sc = (T)gp.scale;
+    if (kind == 0) {
+        const T sig = (T)(gp.sigma * gp.sigma / 4.0);
+        each((T)1, [&](T gg, bool) {
+            T f = (T)0.5 * gg * sc;
+            if (gp.sigma > 0) f *= exp(-gg * sig);
+            return f;
+        });
+    } else if (kind == 1) {
+        const T itkf = (T)(1.0 / tkf), wsc = (T)(wtfac * gp.scale), lb = (T)gp.lbda;
+        each((T)1, [&](T gg, bool) { return lindhard_t<T>(fm::sqrt_n(gg) * itkf, lb, (T)1) * wsc; });
+    } else if (kind == 2) {
+        each((T)1, [&](T gg, bool g0) { return g0 ? (T)0 : gdiv<T>((T)(4.0 * M_PI) * sc, gg); });
+    } else if (kind == 3) {
+        each((T)1, [&](T gg, bool) { return (T)(radial_table(gp, sqrt((double)gg)) * gp.scale); });
+    } else {
+        // kinetic: 1/2 G^2 exp(-G^2 sigma^2 / 2)
+        const double s2 = gp.sigma * gp.sigma / 2.0;
+        each(1.0, [&](double gg, bool) { return 0.5 * gg * exp(-gg * s2) * gp.scale; });
     }
 }
 
-// x pass of the evaluation pipeline with the G-space multiply fused in: the
-// forward x transform of a column tile ends in LDS, each element is scaled by
-// its kernel value (gfactor: vW, WT or Hartree by spectrum slot), and the
-// inverse x transform starts from LDS and writes back in place.  Saves one
-// HBM round trip of every spectrum on each side of the multiply.
-template <typename T, int N, int TILE, int ORD>
-__global__ void __launch_bounds__(TILE *SL<N>::tpp)
-    k_xfused_f(cpx<T> *__restrict__ data, long long bs, long long ncols, long long pitch, long long vp,
-               const cpx<T> *__restrict__ twg, GParams gp, const double *gate) {
-    if (gate_off(gate)) return;
+// x pass of the evaluation pipeline with the G-space multiply fused in:
+// forward x transform, kernel value by spectrum slot, inverse x transform, in
+// place.  With its radices in the opposite order, the inverse starts from the
+// very elements a thread holds after the forward transform, so the multiply
+// works on registers.  All threads make the factors (fewer hold spectrum
+// elements after a large last radix) while the column loads are on their way,
+// and hand them over in LDS.
+template <typename T, int N, int TILE>
+__global__ void __launch_bounds__((TILE *SL<T, N>::TP))
+    k_xfused_f(cpx<T> *data, long long bs, unsigned ncols, unsigned pitch, unsigned vp,
+               const cpx<T> *__restrict__ twg, GParams gp, unsigned mask, const double *gate) {
+    if (gate_off(gate) || run_off(mask, blockIdx.y)) return;
     using C = cpx<T>;
+    constexpr int R = SL<T, N>::first, RL = SL<T, N>::last, TP = SL<T, N>::TP;
     __shared__ C tw[N];
     __shared__ C buf[N * TILE];
-    constexpr int NT = TILE * SL<N>::tpp;
+    __shared__ T fac[N * TILE];
     const int pen = threadIdx.x % TILE;
     const int j = threadIdx.x / TILE;
-    for (int i = threadIdx.x; i < N; i += NT) tw[i] = twg[i];
-    const long long c = (long long)blockIdx.x * TILE + pen;
-    const bool valid = c < ncols && c % pitch < vp;
-    C *col = data + (long long)blockIdx.y * bs + (valid ? c : 0);
+    const unsigned c = blockIdx.x * TILE + pen;
+    const unsigned iy = c / pitch, iz = c - iy * pitch;
+    const bool valid = c < ncols && iz < vp;
     const long long S = ncols;  // x stride of the (nx, ny, pitch) layout
+    C *col = data + (long long)blockIdx.y * bs + (valid ? c : 0) + j * S;
+    C v[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r] = valid ? col[r * TP * S] : C{(T)0, (T)0};
+    for (int i = threadIdx.x; i < N; i += TILE * TP) tw[i] = twg[i];
+    const int kind = gp.kind[gp.c2c ? 0 : blockIdx.y];
     double tkf = 1.0, wtfac = 1.0;
-    const int kind = gp.kind[blockIdx.y];
     if (kind == 1) wt_consts(gp, tkf, wtfac);
-    cstages_io<C, N, TILE, false, 0, 1, true, false, ORD>(buf, tw, col, nullptr, S, valid, pen, j, (T)1);
-    // multiply: this thread's pencil (pen) is one (iy, iz) column, its
-    // elements are e = j, j + tpp, ...; |G|^2 is built from the column's
-    // fixed part plus fx * b1 in the plan precision
-    if (valid) {
-        const int iy = (int)(c / pitch), iz = (int)(c - (long long)iy * pitch);
-        constexpr int TPP = SL<N>::tpp;
-        constexpr int PER = N / TPP;
-        if (gp.full) {
+    if (valid) xfactors<T, N, TILE>(fac + pen, gp, kind, (int)iy, (int)iz, j, tkf, wtfac);
+    C u[RL];
+    dfts<T, N, ColMap<TILE>, false, false, 0, 1>(buf, tw, v, [&](auto &, auto &w) {
 #pragma unroll
-            for (int k = 0; k < PER; ++k) {
-                const int e = j + k * TPP;
-                const double f = gfactor<T>(gp, kind, e, iy, iz, tkf, wtfac);
-                C v = buf[e * TILE + pen];
-                v.x = (T)(v.x * f);
-                v.y = (T)(v.y * f);
-                buf[e * TILE + pen] = v;
-            }
-        } else {
-            const int fy = ffreq(iy, gp.ny);
-            const T cx = (T)(fy * gp.B[3] + iz * gp.B[6]);
-            const T cy = (T)(fy * gp.B[4] + iz * gp.B[7]);
-            const T cz = (T)(fy * gp.B[5] + iz * gp.B[8]);
-            const T bx = (T)gp.B[0], by = (T)gp.B[1], bz = (T)gp.B[2];
-            const T sc = (T)gp.scale;
-            const T itkf = (T)(1.0 / tkf), wsc = (T)(wtfac * gp.scale), lb = (T)gp.lbda;
-            const T sig = (T)(gp.sigma * gp.sigma / 4.0);
-            const bool yz0 = iy == 0 && iz == 0;
+        for (int r = 0; r < RL; ++r) u[r] = w[r];
+    });
+    // the factors are in LDS since the first exchange's barrier
+    if (j < N / RL) {
 #pragma unroll
-            for (int k = 0; k < PER; ++k) {
-                const int e = j + k * TPP;
-                const T fx = (T)ffreq(e, N);
-                const T gx = fx * bx + cx, gy = fx * by + cy, gz = fx * bz + cz;
-                const T gg = gx * gx + gy * gy + gz * gz;
-                T f;
-                if (kind == 0) {
-                    f = (T)0.5 * gg * sc;
-                    if (gp.sigma > 0) f *= exp(-gg * sig);
-                } else if (kind == 1) {
-                    f = lindhard_t<T>(fm::sqrt(gg) * itkf, lb, (T)1) * wsc;
-                } else if (kind == 3) {
-                    f = (T)(radial_table(gp, sqrt((double)gg)) * gp.scale);
-                } else {
-                    f = (yz0 && e == 0) ? (T)0 : fm::div((T)(4.0 * M_PI) * sc, gg);
-                }
-                C v = buf[e * TILE + pen];
-                v.x *= f;
-                v.y *= f;
-                buf[e * TILE + pen] = v;
-            }
+        for (int r = 0; r < RL; ++r) {
+            const T f = fac[(j + r * (N / RL)) * TILE + pen];
+            u[r].x *= f;
+            u[r].y *= f;
         }
     }
     __syncthreads();
-    cstages_io<C, N, TILE, true, 0, 1, false, true, ORD>(buf, tw, nullptr, col, S, valid, pen, j, (T)1);
+    dfts<T, N, ColMap<TILE>, true, true, 0, 1>(buf, tw, u, [&](auto &, auto &w) {
+        if (!valid) return;
+#pragma unroll
+        for (int r = 0; r < R; ++r) col[r * TP * S] = w[r];
+    });
 }
 
 // ---------------------------------------------------------------- rows passes
-// LDS stage for contiguous rows: pencil p element e at buf[p*LD + e].
-template <typename C, int N, int LD, int NPEN, int R, int NS, bool INV>
-__device__ __forceinline__ void rstage(C *buf, const C *tw, int tid) {
-    constexpr int NB = N / R;
-    const int p = tid / NB;  // pencil
-    const int j = tid % NB;
-    const bool act = p < NPEN;
+// the transforms of NPEN pencils staged in LDS in natural order, back to
+// natural order (between two barriers of the caller's)
+template <typename T, int N, int NPEN, int LD, bool INV>
+__device__ __forceinline__ void row_ffts(cpx<T> *buf, const cpx<T> *tw) {
+    using C = cpx<T>;
+    using MAP = RowMap<NPEN, LD>;
+    constexpr int R = SL<T, N>::first, RL = SL<T, N>::last, TP = SL<T, N>::TP;
+    const typename MAP::template At<TP> m((int)threadIdx.x);
     C v[R];
-    if (act) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) v[r] = buf[p * LD + j + r * NB];
-        if (NS > 1) {
-            const int k = j % NS;
+    for (int r = 0; r < R; ++r) v[r] = buf[m.base + m.j + r * TP];
+    __syncthreads();
+    dfts<T, N, MAP, INV, false, 0, 1>(buf, tw, v, [&](auto &ml, auto &u) {
+        __syncthreads();
+        if (ml.act) {
 #pragma unroll
-            for (int r = 1; r < R; ++r) {
-                C w = tw[(r * k * (N / (NS * R))) % N];
-                if (INV) w.y = -w.y;
-                v[r] = cmul(v[r], w);
-            }
+            for (int r = 0; r < RL; ++r) buf[ml.base + ml.j + r * (N / RL)] = u[r];
         }
-    }
-    __syncthreads();
-    if (act) {
-        DFT<R, INV, C>::run(v);
-        const int k = j % NS;
-        const int d = (j / NS) * NS * R + k;
-#pragma unroll
-        for (int r = 0; r < R; ++r) buf[p * LD + d + r * NS] = v[r];
-    }
-    __syncthreads();
+    });
 }
 
-template <typename C, int N, int LD, int NPEN, bool INV, int I, int NS>
-__device__ __forceinline__ void rstages(C *buf, const C *tw, int tid) {
-    if constexpr (I < SL<N>::nst) {
-        constexpr int R = SL<N>::template rad<I>();
-        rstage<C, N, LD, NPEN, R, NS, INV>(buf, tw, tid);
-        rstages<C, N, LD, NPEN, INV, I + 1, NS * R>(buf, tw, tid);
-    }
-}
-
-// Prologue of one spectrum of the R2C pass.  AUX and B56 are fixed per
-// launch (block-uniform branches select the instance), so the compiler never
-// evaluates the linear-response cases or the general power speculatively for
-// the element-wise ops that do not need them.  Without AUX the
-// linear-response codes (which need rho) cannot occur: the host rejects them.
-template <typename T, bool AUX, bool B56> __device__ __forceinline__ T prologue_t(int code, T x, T beta, T r) {
-    switch (code) {
-        case OP_SQRT_RHOM: return fm::sqrt(x > (T)0 ? x : (T)1e-30);
-        case OP_POW_BETA: {
-            const T xc = x < (T)1e-30 ? (T)1e-30 : x;
-            if constexpr (B56)
-                return fm::sqrt(xc) * fm::cbrt(xc);
-            else
-                return fm::pow(xc, beta);
+// Prologues of the NF spectra at a point x (and rho r for the linear-response
+// ops).  AUX and B56 are fixed per launch (block-uniform branches select the
+// instance), so the compiler never evaluates the linear-response cases or the
+// general power speculatively for the element-wise ops that do not need them.
+// Without AUX the linear-response codes (which need rho) cannot occur: the
+// host rejects them.  In FP64 the square and cube roots of a point's spectra
+// come from one inverse sixth root.
+template <typename T, bool AUX, bool B56, int NF>
+__device__ __forceinline__ void prologue_t(const int (&code)[NF], T x, T beta, T r, T (&out)[NF]) {
+    const T base = AUX ? r : x;
+    T sq = (T)0, cb = (T)0, rc = (T)0;  // of max(base, 1e-30) (sqrt: of base > 0)
+    bool roots = false;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) roots |= code[f] != OP_IDENTITY;
+    if (roots) {
+        rc = base < (T)1e-30 ? (T)1e-30 : base;
+        if constexpr (std::is_same<T, double>::value) {
+            const bool fin = rc < (double)INFINITY;
+            const double a = base > 0.0 ? base : 1e-30, s = fm::inv_sixth_root(a);
+            sq = fin ? fm::sqrt_s(a, s) : rc;
+            if constexpr (B56) cb = base < 1e-30 ? 1e-10 : (fin ? fm::cbrt_s(a, s) : rc);
+        } else {
+            sq = fm::sqrt_c(base > (T)0 ? base : (T)1e-30);
+            if constexpr (B56) cb = fm::cbrt(rc);
         }
-        case OP_DSQRT:
-            if constexpr (AUX)
-                return fm::div(x, (T)2 * fm::sqrt(r > (T)0 ? r : (T)1e-30));
-            else
-                return x;
-        case OP_DPOW_BETA:
-            if constexpr (AUX) {
-                const T rc = r < (T)1e-30 ? (T)1e-30 : r;
+    }
+    const T sqc = base < (T)1e-30 ? (T)1e-15 : sq;  // sqrt(max(base, 1e-30))
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+        switch (code[f]) {
+            case OP_SQRT_RHOM: out[f] = sq; break;
+            case OP_POW_BETA:
                 if constexpr (B56)
-                    return beta * fm::div(fm::cbrt(rc), fm::sqrt(rc)) * x;
+                    out[f] = sqc * cb;
                 else
-                    return beta * fm::pow(rc, beta - (T)1) * x;
-            } else {
-                return x;
-            }
-        default: return x;
+                    out[f] = fm::pow(rc, beta);
+                break;
+            case OP_DSQRT: out[f] = AUX ? fm::div(x, (T)2 * sq) : x; break;
+            case OP_DPOW_BETA:
+                if constexpr (AUX && B56)
+                    out[f] = beta * fm::div(cb, sqc) * x;
+                else if constexpr (AUX)
+                    out[f] = beta * fm::pow(rc, beta - (T)1) * x;
+                else
+                    out[f] = x;
+                break;
+            default: out[f] = x;
+        }
     }
 }
 
-// Rows R2C for NF spectra at once: NPEN packed pairs of rows per spectrum,
-// so the NF*NPEN pencils run through the same LDS stages.  When all spectra
-// transform the same input (in_bs == 0, each with its own prologue) the input
-// rows are read once.  Output rows have pitch opitch >= N/2+1.
-//
-// Every load of the tile is issued at once, before the twiddles, with
-// addresses clamped into the tile instead of branches (the rows past the end
-// of a partial tile are zeroed afterwards), so a workgroup waits for one
-// memory round trip rather than one per element.  Consecutive lanes take
-// consecutive elements: the loads and the LDS writes stay unit-stride.
-// partials[blockIdx.y] receives the FP64 sum of slot sum_slot over the tile.
+// Rows R2C for NF spectra at once: NPEN packed pairs of rows per spectrum.
+// The NF spectra transform the same input, each with its own prologue (NF = 1:
+// spectrum blockIdx.y of inputs in_bs apart).  A thread's loads go out
+// together, with row addresses clamped into the tile instead of branches (rows
+// past the end are zeroed afterwards).  Output rows have pitch opitch >= N/2+1.
+// partials[blockIdx.x] receives the FP64 sum of slot sum_slot over the tile.
 template <typename T, int N, int NPEN, int NF>
-__global__ void __launch_bounds__(NF *NPEN *SL<N>::tpp)
+__global__ void __launch_bounds__((NF *NPEN *SL<T, N>::TP))
     k_rows_r2c_f(const T *__restrict__ in, cpx<T> *__restrict__ out, long long in_bs, long long out_bs, long long nrows,
-                 long long opitch, const cpx<T> *__restrict__ twg, T scale, Prologue pro, double *partials,
+                 int opitch, const cpx<T> *__restrict__ twg, T scale, Prologue pro, double *partials,
                  int sum_slot, const double *gate) {
     if (gate_off(gate)) return;
     using C = cpx<T>;
-    constexpr int NT = NF * NPEN * SL<N>::tpp;
+    constexpr int TP = SL<T, N>::TP, LD = N + 1;
+    constexpr int NT = NF * NPEN * TP;
     constexpr int ROWS = 2 * NPEN;
     constexpr int NZC = N / 2 + 1;
-    constexpr int LD = N + 1;
-    constexpr int NE = ROWS * N;
-    constexpr int PER = (NE + NT - 1) / NT;
     __shared__ C tw[N];
     __shared__ C buf[NF * NPEN * LD];
-    __shared__ double red[16];
-    const int slot0 = blockIdx.x * NF;
-    const long long row0 = (long long)blockIdx.y * ROWS;
-    const int nv = (int)min((long long)ROWS, nrows - row0);
-    const int lim = nv * N;
-    const T beta = (T)pro.beta;
-    const bool b56 = pro.b56 != 0;
+    const int slot0 = blockIdx.y * NF;
+    const T *src = in + slot0 * in_bs;
     const T *aux = reinterpret_cast<const T *>(pro.aux);
     const T *phi = reinterpret_cast<const T *>(pro.phi);
-    const bool sep = in_bs != 0;
+    const T beta = (T)pro.beta;
     const bool do_sum = partials != nullptr && sum_slot >= slot0 && sum_slot < slot0 + NF;
-    const T *src = in + slot0 * in_bs + row0 * N;
-    T x0[PER];
+    int code[NF];
+#pragma unroll
+    for (int f = 0; f < NF; ++f) code[f] = pro.code[(slot0 + f) & 3];
+    for (int i = threadIdx.x; i < N; i += NT) tw[i] = twg[i];
+    double acc[1] = {0.0};
+    const long long row0 = (long long)blockIdx.x * ROWS;
+    const int nv = (int)min((long long)ROWS, nrows - row0);
+    constexpr int NW = NPEN * N, PER = (NW + NT - 1) / NT;
+    // point (pair, pos) of both rows: all loads of a thread go out together
+    C x0[PER];
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-        const int e = threadIdx.x + i * NT;
-        x0[i] = src[e < lim ? e : lim - 1];
-    }
-    C twv = (threadIdx.x < N) ? twg[threadIdx.x] : C{};
-    T pv[PER], av[PER];
-    if (phi) {
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int e = threadIdx.x + i * NT;
-            pv[i] = phi[row0 * N + (e < lim ? e : lim - 1)];
+        const int w = min((int)threadIdx.x + i * NT, NW - 1);
+        const int p = w / N;
+        const long long ea = (row0 + (2 * p < nv ? 2 * p : 0)) * N + (w - p * N);
+        const long long eb = 2 * p + 1 < nv ? ea + N : ea;
+        x0[i] = C{src[ea], src[eb]};
+        if (phi) {
+            const C f{phi[ea], phi[eb]};
+            x0[i] = C{(T)(2.0 * (double)f.x * (double)x0[i].x), (T)(2.0 * (double)f.y * (double)x0[i].y)};
         }
     }
-    if (aux) {
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int e = threadIdx.x + i * NT;
-            av[i] = aux[row0 * N + (e < lim ? e : lim - 1)];
-        }
+    for (int i = 0; i < PER; ++i) {
+        const int w = threadIdx.x + i * NT;
+        if (NW % NT == 0 || w < NW) buf[w / N * LD + w % N] = x0[i];
     }
-    for (int i = threadIdx.x + NT; i < N; i += NT) tw[i] = twg[i];
-    if (threadIdx.x < N) tw[threadIdx.x] = twv;
-    double acc = 0.0;
-    auto write = [&](auto aux_c, auto b56_c) {
+    // the prologues, each thread on its own points (unrolled only for the
+    // fused spectra, where a thread has few)
+    auto prep = [&](auto aux_c, auto b56_c) {
         constexpr bool AUX = decltype(aux_c)::value, B56 = decltype(b56_c)::value;
-#pragma unroll
+#pragma unroll NF == 3 ? PER : 1
         for (int i = 0; i < PER; ++i) {
-            const int e = threadIdx.x + i * NT;
-            if (NE % NT == 0 || e < NE) {
-                const int r = e / N;
-                const int pos = e - r * N;
-                const bool live = e < lim;
-                T xa = live ? x0[i] : (T)0;
-                if (live && phi) xa = (T)(2.0 * (double)pv[i] * (double)xa);
-                const T a = AUX ? av[i] : (T)0;
-#pragma unroll
-                for (int f = 0; f < NF; ++f) {
-                    T x = xa;
-                    if (f > 0 && sep && live) x = in[(long long)(slot0 + f) * in_bs + row0 * N + e];
-                    if (do_sum && slot0 + f == sum_slot) acc += (double)x;
-                    if (live) x = prologue_t<T, AUX, B56>(pro.code[(slot0 + f) & 3], x, beta, a);
-                    reinterpret_cast<T *>(&buf[(f * NPEN + (r >> 1)) * LD + pos])[r & 1] = x;
-                }
+            const int w = threadIdx.x + i * NT;
+            if (NW % NT != 0 && w >= NW) break;
+            const int p = w / N, pos = w - p * N;
+            const bool la = 2 * p < nv, lb = 2 * p + 1 < nv;
+            const C x = buf[p * LD + pos];
+            C a{(T)0, (T)0};
+            if constexpr (AUX) {
+                const long long ea = (row0 + (la ? 2 * p : 0)) * N + pos;
+                a = C{aux[ea], aux[lb ? ea + N : ea]};
             }
+            T oa[NF], ob[NF];
+            prologue_t<T, AUX, B56, NF>(code, x.x, beta, a.x, oa);
+            prologue_t<T, AUX, B56, NF>(code, x.y, beta, a.y, ob);
+            if (do_sum) acc[0] += (la ? (double)x.x : 0.0) + (lb ? (double)x.y : 0.0);
+#pragma unroll
+            for (int f = 0; f < NF; ++f)
+                buf[(f * NPEN + p) * LD + pos] = C{la ? oa[f] : (T)0, lb ? ob[f] : (T)0};
         }
     };
     if (aux) {
-        if (b56)
-            write(std::true_type{}, std::true_type{});
+        if (pro.b56)
+            prep(std::true_type{}, std::true_type{});
         else
-            write(std::true_type{}, std::false_type{});
+            prep(std::true_type{}, std::false_type{});
     } else {
-        if (b56)
-            write(std::false_type{}, std::true_type{});
+        if (pro.b56)
+            prep(std::false_type{}, std::true_type{});
         else
-            write(std::false_type{}, std::false_type{});
-    }
-    if (do_sum) {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+            prep(std::false_type{}, std::false_type{});
     }
     __syncthreads();
-    if (do_sum && threadIdx.x == 0) {
-        double sm = 0.0;
-        for (int w = 0; w < (NT + 63) / 64; ++w) sm += red[w];
-        partials[blockIdx.y] = sm;
+    row_ffts<T, N, NF * NPEN, LD, false>(buf, tw);
+    __syncthreads();
+    // separate the packed rows: A_k = (Z_k + conj Z_{N-k}) / 2, B_k = (Z_k - conj Z_{N-k}) / 2i
+    for (int e = threadIdx.x; e < NF * NPEN * NZC; e += NT) {
+        const int qq = e / NZC, k = e - qq * NZC;
+        const int ff = qq / NPEN, pp = qq - ff * NPEN;
+        const C z = buf[qq * LD + k];
+        C zc = buf[qq * LD + (k == 0 ? 0 : N - k)];
+        zc.y = -zc.y;
+        C *o = out + (long long)(slot0 + ff) * out_bs + (row0 + 2 * pp) * opitch + k;
+        if (2 * pp < nv) *o = C{(z.x + zc.x) * (T)0.5 * scale, (z.y + zc.y) * (T)0.5 * scale};
+        if (2 * pp + 1 < nv) o[opitch] = C{(z.y - zc.y) * (T)0.5 * scale, -(z.x - zc.x) * (T)0.5 * scale};
     }
-    rstages<C, N, LD, NF * NPEN, false, 0, 1>(buf, tw, (int)threadIdx.x);
-    for (int e = threadIdx.x; e < NF * ROWS * NZC; e += NT) {
-        const int fr = e / NZC, k = e - fr * NZC;
-        const int f = fr / ROWS, r = fr - f * ROWS;
-        if (r < nv) {
-            const int p = f * NPEN + (r >> 1);
-            const C z = buf[p * LD + k];
-            C zc = buf[p * LD + (k == 0 ? 0 : N - k)];
-            zc.y = -zc.y;
-            C o;
-            if ((r & 1) == 0)
-                o = C{(z.x + zc.x) * (T)0.5, (z.y + zc.y) * (T)0.5};
-            else
-                o = C{(z.y - zc.y) * (T)0.5, -(z.x - zc.x) * (T)0.5};
-            out[(long long)(slot0 + f) * out_bs + (row0 + r) * opitch + k] = C{o.x * scale, o.y * scale};
-        }
-    }
+    if (do_sum) block_sums<1>(acc, partials);
 }
 
 // Rows C2R (irfft semantics: imaginary parts of k = 0 and Nyquist ignored).
 // Each thread loads column k of a row pair (A of row 2p, B of row 2p+1) and
-// writes A + iB to column k and its Hermitian image conj(A) + i conj(B) to
-// column N - k of the packed pencil, so the half spectrum goes from registers
-// to the pencil in one LDS pass.  All loads of the tile are issued at once
-// with clamped addresses.
+// stages A + iB at k and its Hermitian image conj(A) + i conj(B) at N - k of
+// the packed pencil.  All loads of a tile are issued at once with clamped
+// addresses.
 template <typename T, int N, int NPEN>
-__global__ void __launch_bounds__(NPEN *SL<N>::tpp)
+__global__ void __launch_bounds__((NPEN *SL<T, N>::TP))
     k_rows_c2r_f(const cpx<T> *__restrict__ in, T *__restrict__ out, long long in_bs, long long out_bs,
-                 long long nrows, long long ipitch, const cpx<T> *__restrict__ twg, T scale, const double *gate) {
+                 long long nrows, int ipitch, const cpx<T> *__restrict__ twg, T scale, const double *gate) {
     if (gate_off(gate)) return;
     using C = cpx<T>;
-    constexpr int NT = NPEN * SL<N>::tpp;
-    constexpr int ROWS = 2 * NPEN;
-    constexpr int NZC = N / 2 + 1;
-    constexpr int LD = N + 1;
-    constexpr int NW = NPEN * NZC;
-    constexpr int PER = (NW + NT - 1) / NT;
+    constexpr int TP = SL<T, N>::TP, LD = N + 1, NT = NPEN * TP, ROWS = 2 * NPEN;
+    constexpr int NZC = N / 2 + 1, NW = NPEN * NZC, PER = (NW + NT - 1) / NT;
     __shared__ C tw[N];
     __shared__ C buf[NPEN * LD];
-    const long long row0 = (long long)blockIdx.y * ROWS;
-    const C *src = in + (long long)blockIdx.x * in_bs + row0 * ipitch;
-    T *dst = out + (long long)blockIdx.x * out_bs + row0 * N;
+    const long long row0 = (long long)blockIdx.x * ROWS;
     const int nv = (int)min((long long)ROWS, nrows - row0);
+    in += (long long)blockIdx.y * in_bs;
+    T *dst = out + (long long)blockIdx.y * out_bs + row0 * N;
     C ra[PER], rb[PER];
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-        const int w = threadIdx.x + i * NT;
-        const int wc = w < NW ? w : NW - 1;
-        const int p = wc / NZC, k = wc - p * NZC;
-        const int r0 = 2 * p < nv ? 2 * p : nv - 1;
-        const int r1 = 2 * p + 1 < nv ? 2 * p + 1 : nv - 1;
-        ra[i] = src[r0 * ipitch + k];
-        rb[i] = src[r1 * ipitch + k];
+        const int w = min((int)threadIdx.x + i * NT, NW - 1);
+        const int p = w / NZC, k = w - p * NZC;
+        const C *a = in + (row0 + (2 * p < nv ? 2 * p : 0)) * ipitch + k;
+        ra[i] = *a;
+        rb[i] = a[2 * p + 1 < nv ? ipitch : 0];
     }
-    C twv = (threadIdx.x < N) ? twg[threadIdx.x] : C{};
-    for (int i = threadIdx.x + NT; i < N; i += NT) tw[i] = twg[i];
-    if (threadIdx.x < N) tw[threadIdx.x] = twv;
+    for (int i = threadIdx.x; i < N; i += NT) tw[i] = twg[i];
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const int w = threadIdx.x + i * NT;
-        if (NW % NT == 0 || w < NW) {
-            const int p = w / NZC, k = w - p * NZC;
-            C A = 2 * p < nv ? ra[i] : C{};
-            C B = 2 * p + 1 < nv ? rb[i] : C{};
-            if (k == 0 || 2 * k == N) {
-                A.y = (T)0;
-                B.y = (T)0;
-            }
-            buf[p * LD + k] = C{A.x - B.y, A.y + B.x};
-            if (k > 0 && 2 * k < N) buf[p * LD + N - k] = C{A.x + B.y, B.x - A.y};
-        }
+        if (NW % NT != 0 && w >= NW) continue;
+        const int p = w / NZC, k = w - p * NZC;
+        C a = ra[i], b = rb[i];
+        if (k == 0 || 2 * k == N) a.y = b.y = (T)0;
+        buf[p * LD + k] = C{a.x - b.y, a.y + b.x};
+        if (k > 0 && 2 * k < N) buf[p * LD + N - k] = C{a.x + b.y, b.x - a.y};
     }
     __syncthreads();
-    rstages<C, N, LD, NPEN, true, 0, 1>(buf, tw, (int)threadIdx.x);
+    row_ffts<T, N, NPEN, LD, true>(buf, tw);
+    __syncthreads();
     for (int e = threadIdx.x; e < nv * N; e += NT) {
         const int r = e / N;
         const C z = buf[(r >> 1) * LD + (e - r * N)];
@@ -525,208 +505,320 @@ __global__ void __launch_bounds__(NPEN *SL<N>::tpp)
     }
 }
 
+// ---------------------------------------------------------------- complex rows
+// per-run scalars of a lock-step batch of linear solves
+constexpr int kMaxRuns = 16;
+struct RunScalars {
+    double ar[kMaxRuns], ai[kMaxRuns], br[kMaxRuns], bi[kMaxRuns];
+    int active[kMaxRuns];
+};
+
+// What the forward z pass of a lock-step batch reads: the field itself, or
+// the conjugate-gradient step x += a p, p = res + b p (the new p is
+// transformed on its way to memory)
+template <typename T> struct CgStep {
+    cpx<T> *x, *p;
+    const cpx<T> *res;
+    RunScalars s;
+};
+
+// Rows C2C forward.  STEP: the CG update above, else `in` is transformed.
+template <typename T, int N, int NPEN, bool STEP>
+__global__ void __launch_bounds__((NPEN *SL<T, N>::TP))
+    k_rows_fwd_f(const cpx<T> *in, cpx<T> *out, long long bs, int nrows, const cpx<T> *__restrict__ twg, T scale,
+                 CgStep<T> cg, unsigned mask, const double *gate) {
+    if (gate_off(gate) || run_off(mask, blockIdx.y)) return;
+    using C = cpx<T>;
+    constexpr int R = SL<T, N>::first, RL = SL<T, N>::last, TP = SL<T, N>::TP, LD = N + 1;
+    __shared__ C tw[N];
+    __shared__ C buf[NPEN * LD];
+    const int j = threadIdx.x % TP, q = threadIdx.x / TP;
+    const int row = blockIdx.x * NPEN + q;
+    const bool act = row < nrows;
+    const long long o = (long long)blockIdx.y * bs + (long long)(act ? row : 0) * N + j;
+    C v[R];
+    if constexpr (STEP) {
+        C r0[R], x0[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            v[r] = cg.p[o + r * TP];
+            r0[r] = cg.res[o + r * TP];
+            x0[r] = cg.x[o + r * TP];
+        }
+        const double ar = cg.s.ar[blockIdx.y], ai = cg.s.ai[blockIdx.y], br = cg.s.br[blockIdx.y],
+                     bi = cg.s.bi[blockIdx.y];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const C pp = v[r], xx = x0[r], rr = r0[r];
+            x0[r] = C{(T)(xx.x + ar * pp.x - ai * pp.y), (T)(xx.y + ar * pp.y + ai * pp.x)};
+            v[r] = C{(T)(rr.x + br * pp.x - bi * pp.y), (T)(rr.y + br * pp.y + bi * pp.x)};
+        }
+        if (act) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                cg.x[o + r * TP] = x0[r];
+                cg.p[o + r * TP] = v[r];
+            }
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] = in[o + r * TP];
+    }
+    for (int i = threadIdx.x; i < N; i += NPEN * TP) tw[i] = twg[i];
+    dfts<T, N, RowMap<NPEN, LD>, false, false, 0, 1>(buf, tw, v, [&](auto &m, auto &u) {
+        const int rl = blockIdx.x * NPEN + m.pen;
+        if (!m.act || rl >= nrows) return;
+        C *dst = out + (long long)blockIdx.y * bs + (long long)rl * N + m.j;
+#pragma unroll
+        for (int r = 0; r < RL; ++r) dst[r * (N / RL)] = C{u[r].x * scale, u[r].y * scale};
+    });
+}
+
+// Inverse z pass.  MODE 0: the transform is stored.  MODE 1 to 3 finish the
+// Hamiltonian product A x = x + sgn i (dt/2) (kin + v x), kin the transform:
+// 1 stores A x and sums x . A x (no conjugation, two columns), 2 stores it
+// and sums |A x|^2 (one column), 3 stores it.  Partial sums per run: row
+// run * gridDim.x + blockIdx.x.
+template <typename T> struct ApplyArgs {
+    const cpx<T> *x;
+    const T *v;
+    double hdt;
+    double *partials;
+};
+
+template <typename T, int N, int NPEN, int MODE>
+__global__ void __launch_bounds__((NPEN *SL<T, N>::TP))
+    k_rows_inv_f(const cpx<T> *in, cpx<T> *out, long long bs, int nrows, int ntiles, const cpx<T> *__restrict__ twg,
+                 T scale, ApplyArgs<T> ap, unsigned mask, const double *gate) {
+    if (gate_off(gate) || run_off(mask, blockIdx.y)) return;
+    using C = cpx<T>;
+    constexpr int R = SL<T, N>::first, RL = SL<T, N>::last, TP = SL<T, N>::TP, LD = N + 1;
+    constexpr int K = MODE == 1 ? 2 : 1;
+    __shared__ C tw[N];
+    __shared__ C buf[NPEN * LD];
+    const int j = threadIdx.x % TP, q = threadIdx.x / TP;
+    for (int i = threadIdx.x; i < N; i += NPEN * TP) tw[i] = twg[i];
+    double acc[K] = {};
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const int row = tile * NPEN + q;
+        const C *src = in + (long long)blockIdx.y * bs + (long long)(row < nrows ? row : 0) * N + j;
+        C v[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] = src[r * TP];
+        dfts<T, N, RowMap<NPEN, LD>, true, false, 0, 1>(buf, tw, v, [&](auto &m, auto &u) {
+            const int rl = tile * NPEN + m.pen;
+            if (!m.act || rl >= nrows) return;
+            const long long o = (long long)blockIdx.y * bs + (long long)rl * N + m.j;
+            if constexpr (MODE == 0) {
+#pragma unroll
+                for (int r = 0; r < RL; ++r) out[o + r * (N / RL)] = C{u[r].x * scale, u[r].y * scale};
+            } else {
+#pragma unroll
+                for (int r = 0; r < RL; ++r) {
+                    const C a = ap.x[o + r * (N / RL)];
+                    const double vv = (double)ap.v[o + r * (N / RL)];
+                    const double hr = (double)u[r].x + vv * (double)a.x, hi = (double)u[r].y + vv * (double)a.y;
+                    // i * hdt * (hr + i hi) = -hdt hi + i hdt hr
+                    const double orr = (double)a.x - ap.hdt * hi, oi = (double)a.y + ap.hdt * hr;
+                    out[o + r * (N / RL)] = C{(T)orr, (T)oi};
+                    if constexpr (MODE == 1) {
+                        acc[0] += (double)a.x * orr - (double)a.y * oi;
+                        acc[K - 1] += (double)a.x * oi + (double)a.y * orr;
+                    } else if constexpr (MODE == 2) {
+                        acc[0] += orr * orr + oi * oi;
+                    }
+                }
+            }
+        });
+        if (tile + (int)gridDim.x < ntiles) __syncthreads();
+    }
+    if constexpr (MODE == 1 || MODE == 2) {
+        block_sums<K>(acc, ap.partials + (long long)blockIdx.y * gridDim.x * K);
+    }
+}
+
 // ---------------------------------------------------------------- dispatch
-// Tile of the column pass: as many pencils as fit 1024 threads, power of 2,
-// at most 32 (FP32) / 16 (FP64), LDS <= 64 KB; variant v halves it v times.
-template <typename T, int N> constexpr int col_tile() {
-    int t = sizeof(T) == 4 ? 32 : 16;
-    while (t > 1 && (t * SL<N>::tpp > 1024 || (t + 1) * N * 2 * (int)sizeof(T) > 64 * 1024)) t /= 2;
+// Column tile: runs of 128 bytes per element row, or 256 where the workgroup
+// takes that many threads
+template <typename T, int N, int V> constexpr int col_tile_v() {
+    int t = (V == 0 ? 128 : 256) / (2 * (int)sizeof(T));
+    while (t * SL<T, N>::TP > 1024) t /= 2;
     return t;
 }
-template <typename T, int N, int V> constexpr int col_tile_v() {
-    const int t = col_tile<T, N>() >> V;
-    return t < 1 ? 1 : t;
-}
-template <typename T, int N> constexpr int row_pens() {
-    int p = 16;
-    while (p > 1 && (p * SL<N>::tpp > 1024 || (p * (N + 1) + N) * 2 * (int)sizeof(T) > 64 * 1024)) --p;
-    return p;
-}
-template <typename T, int N, int V> constexpr int row_pens_v() {
-    const int p = row_pens<T, N>() >> V;
-    return p < 1 ? 1 : p;
-}
-template <typename T, int N, int NF> constexpr int r2c_pens() {
-    int p = 8;
-    while (p > 1 && (NF * p * SL<N>::tpp > 1024 || (NF * p * (N + 1) + N) * 2 * (int)sizeof(T) + 128 > 64 * 1024))
-        --p;
-    return p;
-}
-template <typename T, int N, int NF, int V> constexpr int r2c_pens_v() {
-    const int p = r2c_pens<T, N, NF>() >> V;
+// Row pairs of a workgroup: about 256 or 128 threads
+template <typename T, int N, int NF, int V> constexpr int pens_v() {
+    int p = (V == 0 ? 256 : 128) / (NF * SL<T, N>::TP);
+    while (p > 1 && (NF * p * (N + 1) + N) * 2 * (int)sizeof(T) > 62 * 1024) --p;
     return p < 1 ? 1 : p;
 }
 
+// workgroups of a tile walk: all tiles at once up to `cap`, else equal rounds
+inline int tile_blocks(long long tiles, long long cap) {
+    if (tiles <= cap) return (int)tiles;
+    const long long rounds = (tiles + cap - 1) / cap;
+    return (int)((tiles + rounds - 1) / rounds);
+}
+
+// the odd variants have the second tile
 #define OFDFT_VARIANT(var, CALL) \
-    switch (var) {               \
-        case 1: CALL(1); break;  \
-        case 2: CALL(2); break;  \
-        default: CALL(0); break; \
-    }
-#define OFDFT_COL_VARIANT(var, CALL) \
-    switch (var) {                   \
-        case 1: CALL(1, 0); break;   \
-        case 2: CALL(2, 0); break;   \
-        case 3: CALL(0, 1); break;   \
-        case 4: CALL(1, 1); break;   \
-        case 5: CALL(2, 1); break;   \
-        default: CALL(0, 0); break;  \
+    if ((var) % kTiles == 1) {        \
+        CALL(1);                 \
+    } else {                     \
+        CALL(0);                 \
     }
 
-template <typename T, int N>
-static void launch_cols(int var, bool inv, const cpx<T> *in, cpx<T> *out, int batch, long long bs, long long ncols,
-                        long long P, long long Q, long long S, long long vp, const cpx<T> *tw, T scale, hipStream_t s,
-                        const double *gate) {
-#define CALL(V, O)                                                                                                 \
-    {                                                                                                              \
-        constexpr int TILE = col_tile_v<T, N, V>();                                                                \
-        dim3 grid((unsigned)((ncols + TILE - 1) / TILE), (unsigned)batch);                                         \
-        if (inv)                                                                                                   \
-            hipLaunchKernelGGL((k_cols_f<T, N, TILE, true, O>), grid, dim3(TILE * SL<N>::tpp), 0, s, in, out, bs,   \
-                               ncols, P, Q, S, vp, tw, scale, gate);                                               \
-        else                                                                                                       \
-            hipLaunchKernelGGL((k_cols_f<T, N, TILE, false, O>), grid, dim3(TILE * SL<N>::tpp), 0, s, in, out, bs,  \
-                               ncols, P, Q, S, vp, tw, scale, gate);                                               \
+template <typename T> struct SizeOps {
+    void (*cols)(int var, bool inv, const cpx<T> *in, cpx<T> *out, int batch, long long bs, long long ncols,
+                 long long P, long long Q, long long S, long long vp, const cpx<T> *tw, T scale, unsigned mask,
+                 hipStream_t s, const double *gate);
+    void (*xfused)(int var, cpx<T> *data, int batch, long long bs, long long ncols, long long pitch, long long vp,
+                   const cpx<T> *tw, const GParams &gp, unsigned mask, hipStream_t s, const double *gate);
+    void (*r2c)(int var, const T *in, cpx<T> *out, int batch, long long in_bs, long long out_bs, long long nrows,
+                long long opitch, const cpx<T> *tw, T scale, const Prologue &pro, double *partials, int sum_slot,
+                hipStream_t s, const double *gate);
+    int (*r2c_tiles)(int var, int batch, long long nrows);  // its workgroups, each with a partial sum
+    void (*c2r)(int var, const cpx<T> *in, T *out, int batch, long long in_bs, long long out_bs, long long nrows,
+                long long ipitch, const cpx<T> *tw, T scale, hipStream_t s, const double *gate);
+    void (*rows_fwd)(const cpx<T> *in, cpx<T> *out, int batch, long long bs, long long nrows, const cpx<T> *tw,
+                     T scale, const CgStep<T> *cg, unsigned mask, hipStream_t s, const double *gate);
+    int (*rows_inv)(int mode, const cpx<T> *in, cpx<T> *out, int batch, long long bs, long long nrows,
+                    const cpx<T> *tw, T scale, const ApplyArgs<T> &ap, int cap, unsigned mask, hipStream_t s,
+                    const double *gate);
+};
+
+template <typename T, int N> struct Launch {
+    using C = cpx<T>;
+    static constexpr int TP = SL<T, N>::TP;
+
+    static void cols(int var, bool inv, const C *in, C *out, int batch, long long bs, long long ncols, long long P,
+                     long long Q, long long S, long long vp, const C *tw, T scale, unsigned mask, hipStream_t s,
+                     const double *gate) {
+#define CALL(V)                                                                                                        \
+    {                                                                                                                  \
+        constexpr int TILE = col_tile_v<T, N, V>();                                                                       \
+        const dim3 grid((unsigned)((ncols + TILE - 1) / TILE), (unsigned)batch);                                       \
+        if (inv)                                                                                                       \
+            hipLaunchKernelGGL((k_cols_f<T, N, TILE, true>), grid, dim3(TILE * TP), 0, s, in, out, bs, (unsigned)ncols, \
+                               (unsigned)P, Q, S, (unsigned)vp, tw, scale, mask, gate);                           \
+        else                                                                                                           \
+            hipLaunchKernelGGL((k_cols_f<T, N, TILE, false>), grid, dim3(TILE * TP), 0, s, in, out, bs,                 \
+                               (unsigned)ncols, (unsigned)P, Q, S, (unsigned)vp, tw, scale, mask, gate);          \
     }
-    OFDFT_COL_VARIANT(var, CALL)
+        OFDFT_VARIANT(var, CALL)
 #undef CALL
-}
-
-template <typename T, int N, int NF>
-static void launch_r2c_nf(int var, const T *in, cpx<T> *out, int nblk, long long in_bs, long long out_bs,
-                          long long nrows, long long opitch, const cpx<T> *tw, T scale, const Prologue &pro,
-                          double *partials, int sum_slot, hipStream_t s, const double *gate) {
-#define CALL(V)                                                                                                \
-    {                                                                                                          \
-        constexpr int NP = r2c_pens_v<T, N, NF, V>();                                                          \
-        const long long tiles = (nrows + 2 * NP - 1) / (2 * NP);                                               \
-        OFDFT_REQUIRE(tiles <= 65535, "too many rows for the R2C pass");                                       \
-        dim3 grid((unsigned)nblk, (unsigned)tiles);                                                            \
-        hipLaunchKernelGGL((k_rows_r2c_f<T, N, NP, NF>), grid, dim3(NF * NP * SL<N>::tpp), 0, s, in, out, in_bs, \
-                           out_bs, nrows, opitch, tw, scale, pro, partials, sum_slot, gate);                   \
     }
-    OFDFT_VARIANT(var, CALL)
+    static void xfused(int var, C *data, int batch, long long bs, long long ncols, long long pitch, long long vp,
+                       const C *tw, const GParams &gp, unsigned mask, hipStream_t s, const double *gate) {
+#define CALL(V)                                                                                                        \
+    {                                                                                                                  \
+        constexpr int TILE = col_tile_v<T, N, V>();                                                                       \
+        const dim3 grid((unsigned)((ncols + TILE - 1) / TILE), (unsigned)batch);                                       \
+        hipLaunchKernelGGL((k_xfused_f<T, N, TILE>), grid, dim3(TILE * TP), 0, s, data, bs, (unsigned)ncols,           \
+                           (unsigned)pitch, (unsigned)vp, tw, gp, mask, gate);                                         \
+    }
+        OFDFT_VARIANT(var, CALL)
 #undef CALL
-}
-
-template <typename T, int N>
-static void launch_r2c(int var, const T *in, cpx<T> *out, int batch, long long in_bs, long long out_bs,
-                       long long nrows, long long opitch, const cpx<T> *tw, T scale, const Prologue &pro,
-                       double *partials, int sum_slot, hipStream_t s, const double *gate) {
-    if (batch == 3)
-        launch_r2c_nf<T, N, 3>(var, in, out, 1, in_bs, out_bs, nrows, opitch, tw, scale, pro, partials, sum_slot, s,
-                               gate);
-    else if (batch == 2)
-        launch_r2c_nf<T, N, 2>(var, in, out, 1, in_bs, out_bs, nrows, opitch, tw, scale, pro, partials, sum_slot, s,
-                               gate);
-    else
-        launch_r2c_nf<T, N, 1>(var, in, out, batch, in_bs, out_bs, nrows, opitch, tw, scale, pro, partials, sum_slot,
-                               s, gate);
-}
-
-template <typename T, int N>
-static void launch_c2r(int var, const cpx<T> *in, T *out, int batch, long long in_bs, long long out_bs,
-                       long long nrows, long long ipitch, const cpx<T> *tw, T scale, hipStream_t s,
-                       const double *gate) {
-#define CALL(V)                                                                                                \
-    {                                                                                                          \
-        constexpr int NP = row_pens_v<T, N, V>();                                                              \
-        const long long tiles = (nrows + 2 * NP - 1) / (2 * NP);                                               \
-        OFDFT_REQUIRE(tiles <= 65535, "too many rows for the C2R pass");                                       \
-        dim3 grid((unsigned)batch, (unsigned)tiles);                                                           \
-        hipLaunchKernelGGL((k_rows_c2r_f<T, N, NP>), grid, dim3(NP * SL<N>::tpp), 0, s, in, out, in_bs, out_bs, \
-                           nrows, ipitch, tw, scale, gate);                                                    \
     }
-    OFDFT_VARIANT(var, CALL)
+    template <int NF>
+    static void r2c_nf(int var, const T *in, C *out, int nblk, long long in_bs, long long out_bs, long long nrows,
+                       long long opitch, const C *tw, T scale, const Prologue &pro, double *partials, int sum_slot,
+                       hipStream_t s, const double *gate) {
+#define CALL(V)                                                                                                      \
+    {                                                                                                                \
+        constexpr int NP = pens_v<T, N, NF, V>();                                                                    \
+        const long long tiles = (nrows + 2 * NP - 1) / (2 * NP);                                                     \
+        const dim3 grid((unsigned)tiles, (unsigned)nblk);                                                            \
+        hipLaunchKernelGGL((k_rows_r2c_f<T, N, NP, NF>), grid, dim3(NF * NP * TP), 0, s, in, out, in_bs, out_bs, nrows, \
+                           (int)opitch, tw, scale, pro, partials, sum_slot, gate);                       \
+    }
+        OFDFT_VARIANT(var, CALL)
 #undef CALL
-}
-
-template <typename T, int N>
-static void launch_xfused(int var, cpx<T> *data, int batch, long long bs, long long ncols, long long pitch,
-                          long long vp, const cpx<T> *tw, const GParams &gp, hipStream_t s, const double *gate) {
-#define CALL(V, O)                                                                                                 \
-    {                                                                                                              \
-        constexpr int TILE = col_tile_v<T, N, V>();                                                                \
-        dim3 grid((unsigned)((ncols + TILE - 1) / TILE), (unsigned)batch);                                         \
-        hipLaunchKernelGGL((k_xfused_f<T, N, TILE, O>), grid, dim3(TILE * SL<N>::tpp), 0, s, data, bs, ncols, pitch, \
-                           vp, tw, gp, gate);                                                                      \
     }
-    OFDFT_COL_VARIANT(var, CALL)
+    static void r2c(int var, const T *in, C *out, int batch, long long in_bs, long long out_bs, long long nrows,
+                    long long opitch, const C *tw, T scale, const Prologue &pro, double *partials, int sum_slot,
+                    hipStream_t s, const double *gate) {
+        if (batch == 3 && in_bs == 0)
+            r2c_nf<3>(var, in, out, 1, in_bs, out_bs, nrows, opitch, tw, scale, pro, partials, sum_slot, s, gate);
+        else if (batch == 2 && in_bs == 0)
+            r2c_nf<2>(var, in, out, 1, in_bs, out_bs, nrows, opitch, tw, scale, pro, partials, sum_slot, s, gate);
+        else
+            r2c_nf<1>(var, in, out, batch, in_bs, out_bs, nrows, opitch, tw, scale, pro, partials, sum_slot, s, gate);
+    }
+    template <int NF> static int r2c_pens(int var) {
+        return var % kTiles == 1 ? pens_v<T, N, NF, 1>() : pens_v<T, N, NF, 0>();
+    }
+    static int r2c_tiles(int var, int batch, long long nrows) {
+        const int np = batch == 3 ? r2c_pens<3>(var) : batch == 2 ? r2c_pens<2>(var) : r2c_pens<1>(var);
+        return (int)((nrows + 2 * np - 1) / (2 * np));
+    }
+    static void c2r(int var, const C *in, T *out, int batch, long long in_bs, long long out_bs, long long nrows,
+                    long long ipitch, const C *tw, T scale, hipStream_t s, const double *gate) {
+#define CALL(V)                                                                                                      \
+    {                                                                                                                \
+        constexpr int NP = pens_v<T, N, 1, V>();                                                                     \
+        const long long tiles = (nrows + 2 * NP - 1) / (2 * NP);                                                     \
+        hipLaunchKernelGGL((k_rows_c2r_f<T, N, NP>), dim3((unsigned)tiles, (unsigned)batch), dim3(NP * TP), 0, s, in, \
+                           out, in_bs, out_bs, nrows, (int)ipitch, tw, scale, gate);                                 \
+    }
+        OFDFT_VARIANT(var, CALL)
 #undef CALL
-}
-
-#define OFDFT_FIXED_SIZES(X) X(32) X(48) X(64) X(72) X(80) X(96) X(100) X(120) X(128) X(144) X(160) X(192) X(200) X(240) X(256)
-
-template <typename T>
-bool xfused_fixed(int n, int var, cpx<T> *data, int batch, long long bs, long long ncols, long long pitch,
-                  long long vp, const void *tw, const GParams &gp, hipStream_t s, const double *gate) {
-    switch (n) {
-#define CASE(N)                                                                                                       \
-    case N:                                                                                                           \
-        launch_xfused<T, N>(var, data, batch, bs, ncols, pitch, vp, reinterpret_cast<const cpx<T> *>(tw), gp, s,       \
-                            gate);                                                                                    \
-        return true;
-        OFDFT_FIXED_SIZES(CASE)
-#undef CASE
-        default: return false;
     }
-}
-
-template <typename T>
-bool cols_fixed(int n, int var, bool inv, const cpx<T> *in, cpx<T> *out, int batch, long long bs, long long ncols,
-                long long P, long long Q, long long S, long long vp, const void *tw, double scale, hipStream_t s,
-                const double *gate) {
-    switch (n) {
-#define CASE(N)                                                                                                        \
-    case N:                                                                                                            \
-        launch_cols<T, N>(var, inv, in, out, batch, bs, ncols, P, Q, S, vp, reinterpret_cast<const cpx<T> *>(tw),      \
-                          (T)scale, s, gate);                                                                         \
-        return true;
-        OFDFT_FIXED_SIZES(CASE)
-#undef CASE
-        default: return false;
+    static void rows_fwd(const C *in, C *out, int batch, long long bs, long long nrows, const C *tw, T scale,
+                         const CgStep<T> *cg, unsigned mask, hipStream_t s, const double *gate) {
+        constexpr int NP = pens_v<T, N, 1, 0>();
+        const dim3 grid((unsigned)((nrows + NP - 1) / NP), (unsigned)batch);
+        if (cg)
+            hipLaunchKernelGGL((k_rows_fwd_f<T, N, NP, true>), grid, dim3(NP * TP), 0, s, in, out, bs, (int)nrows, tw,
+                               scale, *cg, mask, gate);
+        else
+            hipLaunchKernelGGL((k_rows_fwd_f<T, N, NP, false>), grid, dim3(NP * TP), 0, s, in, out, bs, (int)nrows, tw,
+                               scale, CgStep<T>{}, mask, gate);
     }
-}
-
-template <typename T>
-bool r2c_fixed(int n, int var, const T *in, cpx<T> *out, int batch, long long in_bs, long long out_bs,
-               long long nrows, long long opitch, const void *tw, double scale, const Prologue &pro, double *partials,
-               int sum_slot, hipStream_t s, const double *gate) {
-    switch (n) {
-#define CASE(N)                                                                                                       \
-    case N:                                                                                                           \
-        launch_r2c<T, N>(var, in, out, batch, in_bs, out_bs, nrows, opitch, reinterpret_cast<const cpx<T> *>(tw),     \
-                         (T)scale, pro, partials, sum_slot, s, gate);                                                 \
-        return true;
-        OFDFT_FIXED_SIZES(CASE)
-#undef CASE
-        default: return false;
+    template <int MODE>
+    static int inv_mode(const C *in, C *out, int batch, long long bs, long long nrows, const C *tw, T scale,
+                        const ApplyArgs<T> &ap, int cap, unsigned mask, hipStream_t s, const double *gate) {
+        constexpr int NP = pens_v<T, N, 1, 0>();
+        const long long tiles = (nrows + NP - 1) / NP;
+        const int nb = tile_blocks(tiles, cap);
+        hipLaunchKernelGGL((k_rows_inv_f<T, N, NP, MODE>), dim3((unsigned)nb, (unsigned)batch), dim3(NP * TP), 0, s, in,
+                           out, bs, (int)nrows, (int)tiles, tw, scale, ap, mask, gate);
+        return nb;
     }
-}
-
-template <typename T>
-bool c2r_fixed(int n, int var, const cpx<T> *in, T *out, int batch, long long in_bs, long long out_bs,
-               long long nrows, long long ipitch, const void *tw, double scale, hipStream_t s, const double *gate) {
-    switch (n) {
-#define CASE(N)                                                                                                       \
-    case N:                                                                                                           \
-        launch_c2r<T, N>(var, in, out, batch, in_bs, out_bs, nrows, ipitch, reinterpret_cast<const cpx<T> *>(tw),     \
-                         (T)scale, s, gate);                                                                          \
-        return true;
-        OFDFT_FIXED_SIZES(CASE)
-#undef CASE
-        default: return false;
+    static int rows_inv(int mode, const C *in, C *out, int batch, long long bs, long long nrows, const C *tw, T scale,
+                        const ApplyArgs<T> &ap, int cap, unsigned mask, hipStream_t s, const double *gate) {
+        if (mode == 1) return inv_mode<1>(in, out, batch, bs, nrows, tw, scale, ap, cap, mask, s, gate);
+        if (mode == 2) return inv_mode<2>(in, out, batch, bs, nrows, tw, scale, ap, cap, mask, s, gate);
+        if (mode == 3) return inv_mode<3>(in, out, batch, bs, nrows, tw, scale, ap, 1 << 30, mask, s, gate);
+        return inv_mode<0>(in, out, batch, bs, nrows, tw, scale, ap, 1 << 30, mask, s, gate);
     }
-}
+};
 
-#define OFDFT_FIXED_INST(T)                                                                                            \
-    template bool xfused_fixed<T>(int, int, cpx<T> *, int, long long, long long, long long, long long, const void *,   \
-                                  const GParams &, hipStream_t, const double *);                                       \
-    template bool cols_fixed<T>(int, int, bool, const cpx<T> *, cpx<T> *, int, long long, long long, long long,        \
-                                long long, long long, long long, const void *, double, hipStream_t, const double *);   \
-    template bool r2c_fixed<T>(int, int, const T *, cpx<T> *, int, long long, long long, long long, long long,         \
-                               const void *, double, const Prologue &, double *, int, hipStream_t, const double *);    \
-    template bool c2r_fixed<T>(int, int, const cpx<T> *, T *, int, long long, long long, long long, long long,         \
-                               const void *, double, hipStream_t, const double *);
+template <typename T, int N> const SizeOps<T> *size_ops();
+
+#define OFDFT_SIZE_INST(T, N)                                                                                      \
+    template <> const SizeOps<T> *size_ops<T, N>() {                                                               \
+        using L = Launch<T, N>;                                                                                    \
+        static const SizeOps<T> ops{L::cols, L::xfused,   L::r2c,     L::r2c_tiles,                                \
+                                    L::c2r,  L::rows_fwd, L::rows_inv};                                            \
+        return &ops;                                                                                               \
+    }
+
+// the lengths, in groups compiled apart
+#define OFDFT_SIZES_0(X, T) \
+    X(T, 16) X(T, 18) X(T, 20) X(T, 22) X(T, 24) X(T, 26) X(T, 28) X(T, 30) X(T, 32) X(T, 36) X(T, 40) X(T, 42) \
+    X(T, 44) X(T, 48) X(T, 50) X(T, 52) X(T, 54) X(T, 56) X(T, 60) X(T, 64)
+#define OFDFT_SIZES_1(X, T) \
+    X(T, 66) X(T, 70) X(T, 72) X(T, 78) X(T, 80) X(T, 84) X(T, 88) X(T, 90) X(T, 96) X(T, 98) X(T, 100) X(T, 104) \
+    X(T, 108) X(T, 110) X(T, 112) X(T, 120)
+#define OFDFT_SIZES_2(X, T) \
+    X(T, 126) X(T, 128) X(T, 130) X(T, 132) X(T, 140) X(T, 144) X(T, 150) X(T, 154) X(T, 156) X(T, 160) X(T, 162) \
+    X(T, 168) X(T, 176) X(T, 180)
+#define OFDFT_SIZES_3(X, T) \
+    X(T, 182) X(T, 192) X(T, 196) X(T, 198) X(T, 200) X(T, 208) X(T, 210) X(T, 216) X(T, 220) X(T, 224) X(T, 234) \
+    X(T, 240) X(T, 250) X(T, 252) X(T, 256)
+#define OFDFT_SIZES(X, T) OFDFT_SIZES_0(X, T) OFDFT_SIZES_1(X, T) OFDFT_SIZES_2(X, T) OFDFT_SIZES_3(X, T)
+
+// the passes of a length, or null where it has none (fft_fixed.hip)
+template <typename T> const SizeOps<T> *find_ops(int n);
 
 }  // namespace ofdft

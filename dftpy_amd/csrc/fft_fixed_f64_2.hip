@@ -1,0 +1,6 @@
+// Size-specialised FFT passes in double, length group 2.
+#include "fft_fixed.h"
+
+namespace ofdft {
+OFDFT_SIZES_2(OFDFT_SIZE_INST, double)
+}  // namespace ofdft

@@ -11,13 +11,31 @@
 namespace ofdft {
 
 // ------------------------------------------------------------------ Lindhard
+// quotients of the G-space functions, whose operands are normal numbers: the
+// Newton division in FP64 (the library's scales its operands first)
+template <typename T> __device__ __forceinline__ T gdiv(T a, T b) { return fm::div(a, b); }
+template <> __device__ __forceinline__ double gdiv<double>(double a, double b) { return fm::div_n(a, b); }
+
 // Inverse Lindhard function with the reference's branch priority
 // normal < zero (eta < tol) < one (|eta-1| < tol) < large (eta > 3.65).
-// T = double for the FP64 pipeline, float for the FP32 one
+// T = double, or float for FP32 response tables
 template <typename T> __device__ __forceinline__ T lindhard_t(T eta, T lbda, T mu) {
     const T tol = (T)1e-10;
-    if (eta > (T)3.65) {
-        const T inv = fm::rcp(eta * eta);
+    if constexpr (sizeof(T) == 4) {
+        // FP32: 1/f - 1 = x S / f with f = 1 - x S, x = eta^2, S the sum of
+        // x^k / ((2k+1)(2k+3)), which keeps the digits that the difference of
+        // numbers near one loses at small eta (12 terms, 1e-8 at 0.6)
+        if (eta < (T)0.6) {
+            const T x = eta * eta;
+            T sum = (T)0;
+#pragma unroll
+            for (int k = 11; k >= 0; --k) sum = sum * x + (T)(1.0 / ((2 * k + 1) * (2 * k + 3)));
+            return gdiv<T>(x * sum, (T)1 - x * sum) - (T)3 * mu * x + ((T)1 - lbda);
+        }
+    }
+    // the series also from 1.5 in FP32 (1e-8 there; f is a difference that loses digits)
+    if (eta > (sizeof(T) == 4 ? (T)1.5 : (T)3.65)) {
+        const T inv = gdiv<T>((T)1, eta * eta);
         T s = (T)-3.00624946457977689e-3;
         s = (T)-3.38745061493813488e-3 + inv * s;
         s = (T)-3.84763737842981233e-3 + inv * s;
@@ -38,8 +56,8 @@ template <typename T> __device__ __forceinline__ T lindhard_t(T eta, T lbda, T m
     if (fabs(eta - (T)1) < tol) return (T)2 - lbda - (T)3 * mu + (T)20 * (eta - (T)1);
     if (eta < tol) return (T)1 - lbda + eta * eta * ((T)(1.0 / 3.0) - (T)3 * mu);
     // the logarithm stays the library's: its argument tends to 1 as eta -> 0
-    const T lg = log(fm::div((T)1 + eta, fabs((T)1 - eta)));
-    return fm::rcp((T)0.5 + fm::div((T)0.25 * ((T)1 - eta * eta) * lg, eta)) - (T)3 * mu * eta * eta - lbda;
+    const T lg = log(gdiv<T>((T)1 + eta, fabs((T)1 - eta)));
+    return gdiv<T>((T)1, (T)0.5 + gdiv<T>((T)0.25 * ((T)1 - eta * eta) * lg, eta)) - (T)3 * mu * eta * eta - lbda;
 }
 
 __device__ __forceinline__ double lindhard(double eta, double lbda, double mu) { return lindhard_t<double>(eta, lbda, mu); }
@@ -62,7 +80,8 @@ template <typename CT> __device__ __forceinline__ CT resp_k(const RespK &r, CT q
 
 struct GParams {
     double B[9];
-    int kind[4];  // per spectrum slot: 0 vW, 1 WT, 2 Hartree, 3 radial table, -1 none
+    int kind[4];  // per spectrum slot: 0 vW, 1 WT, 2 Hartree, 3 radial table, 4 kinetic (c2c), -1 none
+    int c2c = 0;  // full complex spectra of lock-step runs: every slot has kind[0]
     int nx, ny, nz, nzc;
     int pitch;  // row pitch of the spectra (>= nzc)
     int full;
@@ -116,47 +135,25 @@ __device__ __forceinline__ KVals kernel_vals(const GParams &p, double gg, bool g
 }
 
 
-// value of one kernel (kind 0 vW, 1 WT, 2 Hartree) at |G|^2 = gg; the WT
-// Lindhard function is evaluated in T
-template <typename T>
-__device__ __forceinline__ double kernel_val(const GParams &p, int kind, double gg, bool g0, double tkf, double wtfac) {
+// value of one kernel (kind 0 vW, 1 WT, 2 Hartree, 3 radial table) at |G|^2 = gg
+__device__ __forceinline__ double kernel_val(const GParams &p, int kind, double gg, bool g0, double tkf,
+                                             double wtfac) {
     if (kind == 0) {
         double v = 0.5 * gg;
         if (p.sigma > 0) v *= exp(-gg * p.sigma * p.sigma / 4.0);
         return v;
     }
-    if (kind == 1) return (double)lindhard_t<T>((T)(sqrt(gg) / tkf), (T)p.lbda, (T)1) * wtfac;
-    if (kind == 3) return radial_table(p, sqrt(gg));
-    return g0 ? 0.0 : 4.0 * M_PI / gg;
-}
-
-// multiplier of spectrum kind `kind` at frequency indices (ix, iy, iz) of the
-// half grid, including the full-grid Nyquist averaging and the 1/N scale
-template <typename T>
-__device__ __forceinline__ double gfactor(const GParams &p, int kind, int ix, int iy, int iz, double tkf,
-                                          double wtfac) {
-    int fx = ffreq(ix, p.nx), fy = ffreq(iy, p.ny), fz = iz;
-    const bool g0 = (ix == 0 && iy == 0 && iz == 0);
-    double f;
-    if (p.full) {
-        fz = wrapf(fz, p.nz);
-        const bool nyq = ((p.nx & 1) == 0 && ix == p.nx / 2) || ((p.ny & 1) == 0 && iy == p.ny / 2) ||
-                         ((p.nz & 1) == 0 && iz == p.nz / 2);
-        f = kernel_val<T>(p, kind, gsq(p.B, fx, fy, fz), g0, tkf, wtfac);
-        if (nyq)
-            f = 0.5 * (f + kernel_val<T>(p, kind, gsq(p.B, wrapf(-fx, p.nx), wrapf(-fy, p.ny), wrapf(-fz, p.nz)), g0,
-                                         tkf, wtfac));
-    } else {
-        f = kernel_val<T>(p, kind, gsq(p.B, fx, fy, fz), g0, tkf, wtfac);
-    }
-    return f * p.scale;
+    if (kind == 1) return lindhard(gdiv<double>(fm::sqrt_n(gg), tkf), p.lbda, 1.0) * wtfac;
+    if (kind == 3) return radial_table(p, fm::sqrt_n(gg));
+    return g0 ? 0.0 : gdiv<double>(4.0 * M_PI, gg);
 }
 
 // 2 k_F of rho0 and the WT kernel prefactor (wt.py:66, kernel.py:325-334)
 __device__ __forceinline__ void wt_consts_at(double rho0, double alpha, double beta, double &tkf, double &wtfac) {
     tkf = 2.0 * cbrt(3.0 * rho0 * M_PI * M_PI);
-    const double ctf = 0.3 * pow(3.0 * M_PI * M_PI, 2.0 / 3.0);
-    wtfac = 5.0 / (9.0 * alpha * beta * pow(rho0, alpha + beta - 5.0 / 3.0)) * ctf;
+    const double ctf = 2.871234000188191;  // 3/10 (3 pi^2)^(2/3)
+    const double ex = alpha + beta - 5.0 / 3.0;  // zero up to rounding for alpha = beta = 5/6
+    wtfac = 5.0 / (9.0 * alpha * beta * (fabs(ex) < 1e-15 ? 1.0 : pow(rho0, ex))) * ctf;
 }
 
 __device__ __forceinline__ void wt_consts(const GParams &p, double &tkf, double &wtfac) {

@@ -89,8 +89,9 @@ struct Prologue {
 
 struct LmgpState;  // LMGP nonlocal KEDF tables and workspace (lmgp.hip)
 
-// variants of the size-specialised FFT passes the autotuner times: the row
-// passes have 3 tiles; the column passes 6, tile var % 3 and radix order var / 3
+// variants of the size-specialised FFT passes: two tiles each (variant % 2),
+// which the autotuner times; the ranges accepted by ofdft_plan_set_variants
+constexpr int kTiles = 2;
 constexpr int kTileVariants = 3;
 constexpr int kColVariants = 6;
 
@@ -192,10 +193,11 @@ bool fixed_size(int n);
 template <typename T>
 void fft_c2c(Plan &P, const cpx<T> *in, cpx<T> *out, bool inverse, int batch, long long bs, double scale,
              hipStream_t s);
-// the x/y passes alone (in place allowed), for fused pipelines
+// the x/y passes alone (in place allowed), for fused pipelines; batch entries
+// b < 32 whose bit of mask is clear are left out
 template <typename T>
 void fft_cols(Plan &P, int axis, bool full_grid, bool inverse, const cpx<T> *in, cpx<T> *out, int batch,
-              long long bs, double scale, hipStream_t s, long long pitch = 0);
+              long long bs, double scale, hipStream_t s, long long pitch = 0, unsigned mask = ~0u);
 
 // single passes, for timing
 template <typename T>
@@ -212,8 +214,8 @@ void eval_fields(Plan &P, const T *rho, unsigned calc, T *pot, double *energies,
 // 1 = point-wise post pass), eval.hip
 template <typename T> void bench_eval_stage(Plan &P, int stage, const T *rho, T *pot, hipStream_t s);
 
-// autotuner of the tile variants (fft.hip); times[12]: per pass (r2c, c2r,
-// x cols, y cols) the mean ms of variants 0..2 (optional)
+// autotuner of the tile variants (fft.hip); times[4 * kColVariants]: per pass
+// (r2c, c2r, x cols, y cols) the mean ms of the tiles, -1 where none (optional)
 void plan_autotune(Plan &P, hipStream_t s, float *times);
 
 // reductions (vec.hip)
@@ -231,10 +233,11 @@ void reduce_final(const double *partials, int nblocks, int nterms, double *out, 
 template <typename T>
 void eval(Plan &P, const T *rho, unsigned calc, T *pot, double *energies, hipStream_t s);
 // analytic Hessian-vector product of the residual (V - mu) phi along p
-// (drho = 2 phi p is formed inside the kernels)
+// (drho = 2 phi p is formed inside the kernels); returns the rows of partial
+// sums p . Ap in P.red
 template <typename T>
-void hvp(Plan &P, const T *rho, const T *phi, const T *p, const T *pot, const T *base_a, const T *base_c,
-         const double *mu, T *Ap, int nb, hipStream_t s);
+int hvp(Plan &P, const T *rho, const T *phi, const T *p, const T *pot, const T *base_a, const T *base_c,
+         const double *mu, T *Ap, hipStream_t s);
 void work_slots(const Plan &P, int *slot);
 
 // lmgp.hip: adds the LMGP nonlocal energy (energies[E_NL], E_SUM) and

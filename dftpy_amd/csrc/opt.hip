@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "dcsrch.h"
+#include "fft_fixed.h"
 #include "gspace.h"
 #include "internal.h"
 #include "reduce.h"
@@ -51,10 +52,6 @@ void plan_aux_free(Plan &P) {
 
 template <typename T> static T *fld(Plan &P, int f) { return reinterpret_cast<T *>(P.aux) + (size_t)f * P.N; }
 
-
-template <typename T>
-bool xfused_fixed(int n, int var, cpx<T> *data, int batch, long long bs, long long ncols, long long pitch,
-                  long long vp, const void *tw, const GParams &gp, hipStream_t s, const double *gate);
 
 // ------------------------------------------------------------------ kernels
 // Streaming kernels: template VEC (4 consecutive elements per thread when the
@@ -787,10 +784,10 @@ struct Ctx {
     }
     // pub_n > 0: the same launch then publishes scal[pub_slot..pub_slot+pub_n)
     // to the pinned host buffer, read by published()
-    void reduce_final_cols(int K, int slot, int pub_n = 0, int pub_slot = 0, int pub_off = 0) {
-        // partials laid out [block][K]
+    void reduce_final_cols(int K, int slot, int pub_n = 0, int pub_slot = 0, int pub_off = 0, int rows = 0) {
+        // partials laid out [block][K], of nb blocks unless the kernel had its own number
         std::vector<double> ones(K, 1.0);
-        reduce_final(P.red, nb, K, P.scal + slot, ones.data(), s, P.gate, pub_n ? P.scal + pub_slot : nullptr,
+        reduce_final(P.red, rows ? rows : nb, K, P.scal + slot, ones.data(), s, P.gate, pub_n ? P.scal + pub_slot : nullptr,
                      pub_n ? P.pinned_dev + pub_off : nullptr, pub_n);
     }
     // the scalars the last publishing reduction sent, once the stream is done
@@ -818,6 +815,13 @@ struct Ctx {
     } while (0)
 #define PW_RED(K, ...) PW_LAUNCH_(K, C.nb, __VA_ARGS__)
 #define PW_STREAM(K, ...) PW_LAUNCH_(K, C.nbw, __VA_ARGS__)
+
+// lengths the device-driven iteration is accepted for
+static bool graph_size(int n) {
+    for (int m : {32, 48, 64, 72, 80, 96, 100, 120, 128, 144, 160, 192, 200, 240, 256})
+        if (n == m) return true;
+    return false;
+}
 
 template <typename T> struct Opt {
     Plan &P;
@@ -877,9 +881,8 @@ template <typename T> struct Opt {
             gp.tab_n = P.tn_pre_n;
             gp.tab_inv_dq = 1.0 / P.tn_pre_dq;
             fft_r2c<T>(P, in, spec, 1, 0, ncp, 1.0, nullptr, nullptr, C.s, pitch, true);
-            OFDFT_REQUIRE(xfused_fixed<T>(P.nr[0], P.var_cols[0], spec, 1, ncp, (long long)P.nr[1] * pitch, pitch,
-                                          P.nzc, P.tw[0], gp, C.s, P.gate),
-                          "fused x pass unavailable");
+            find_ops<T>(P.nr[0])->xfused(P.var_cols[0], spec, 1, ncp, (long long)P.nr[1] * pitch, pitch, P.nzc,
+                                         reinterpret_cast<const cpx<T> *>(P.tw[0]), gp, ~0u, C.s, P.gate);
             OFDFT_HIP(hipGetLastError());
             fft_c2r<T>(P, spec, spec, out, 1, ncp, ncp, P.N, 1.0, C.s, pitch, true);
             return;
@@ -934,8 +937,9 @@ template <typename T> struct Opt {
         std::vector<double> rl{1e10};
         int it = 0;
         for (it = 0; it < maxfun; ++it) {
+            int rows = C.nb;
             if (hvp_mode) {
-                hvp<T>(P, F(F_RHO), F(F_PHI), tp, F(F_POT), F(F_BASE_A), F(F_BASE_C), P.scal + 2, Ap, C.nb, C.s);
+                rows = hvp<T>(P, F(F_RHO), F(F_PHI), tp, F(F_POT), F(F_BASE_A), F(F_BASE_C), P.scal + 2, Ap, C.s);
                 ++n_v;
             } else {
                 PW_STREAM(k_tn_shift, F(F_PHI), tp, eps, phi1, rho1, n);
@@ -946,7 +950,7 @@ template <typename T> struct Opt {
             // pAp -> scal[16]; the update takes alpha = r.z / pAp from the
             // device (r.z of the start, then of the previous iteration);
             // r1 -> scal[17]; r1.z1 -> scal[18]
-            C.reduce_final_cols(1, 16);
+            C.reduce_final_cols(1, 16, 0, 0, 0, rows);
             const int rz_slot = it == 0 ? (pre ? 26 : 25) : (pre ? 18 : 17);
             PW_RED(k_tn_update_dev, dir, tres, tp, Ap, P.scal + rz_slot,
                                P.scal + 16, n, P.red);
@@ -1158,14 +1162,15 @@ template <typename T> struct Opt {
         }
         for (int k = 0; k < G; ++k) {
             gate(G_CG);
+            int rows = C.nb;
             if (hvp_mode) {
-                hvp<T>(P, F(F_RHO), F(F_PHI), tp, F(F_POT), F(F_BASE_A), F(F_BASE_C), P.scal + 2, Ap, C.nb, C.s);
+                rows = hvp<T>(P, F(F_RHO), F(F_PHI), tp, F(F_POT), F(F_BASE_A), F(F_BASE_C), P.scal + 2, Ap, C.s);
             } else {
                 PW_STREAM(k_tn_shift, F(F_PHI), tp, eps, phi1, rho1, n);
                 eval<T>(P, rho1, OFDFT_CALC_V, pot1, nullptr, C.s);
                 PW_RED(k_tn_ap, pot1, phi1, F(F_RES), tp, P.scal + 2, eps, Ap, n, P.red);
             }
-            C.reduce_final_cols(1, 16);
+            C.reduce_final_cols(1, 16, 0, 0, 0, rows);
             PW_RED(k_tn_update_dev, dir, tres, tp, Ap, P.scal + T_RZCUR, P.scal + 16, n, P.red);
             if (pre) {
                 C.reduce_final_cols(1, 17);
@@ -1292,7 +1297,7 @@ template <typename T> struct Opt {
         OFDFT_REQUIRE(G >= 1 && G <= 64 && L >= 1 && L <= 64, "optimize_tn_graph: steps per superstep out of range");
         OFDFT_REQUIRE(!(P.terms & OFDFT_TERM_LMGP), "optimize_tn_graph: LMGP is not supported");
         for (int d = 0; d < 3; ++d)
-            OFDFT_REQUIRE(P.use_fixed && (P.nr[d] == 1 || fixed_size(P.nr[d])),
+            OFDFT_REQUIRE(P.use_fixed && (P.nr[d] == 1 || graph_size(P.nr[d])),
                           "optimize_tn_graph: every axis needs a size-specialised FFT pass (2/3/5-smooth sizes of "
                           "the fixed table)");
         const double econv = opts[0];

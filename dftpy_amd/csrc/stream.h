@@ -98,6 +98,23 @@ template <int VEC, typename F> __device__ __forceinline__ void pw_groups(long lo
     for (long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x; g < ng; g += stride) body(g * VEC);
 }
 
+// G groups of the calling thread, one launch covering the field: unrolled
+// without a loop, around which the compiler would keep the constants of FP64
+// functions in 100 registers.  G = 0: the loop of pw_groups.
+template <int VEC, int G, typename F> __device__ __forceinline__ void pw_each(long long n, F &&body) {
+    if constexpr (G == 0) {
+        pw_groups<VEC>(n, body);
+        return;
+    }
+    const long long ng = VEC == 4 ? (n >> 2) : n;
+    const long long g0 = (long long)blockIdx.x * (blockDim.x * G) + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < G; ++k) {
+        const long long g = g0 + (long long)k * blockDim.x;
+        if (g < ng) body(g * VEC);
+    }
+}
+
 // host side: element width of a launch and the block count of a
 // non-reducing streaming kernel of 256 threads
 inline int pw_vec(long long n) { return (n & 3) == 0 ? 4 : 1; }

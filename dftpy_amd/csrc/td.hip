@@ -10,8 +10,10 @@
 #include <tuple>
 #include <vector>
 
+#include "fft_fixed.h"
 #include "internal.h"
 #include "reduce.h"
+#include "stream.h"
 
 namespace ofdft {
 
@@ -29,27 +31,8 @@ template <int K> __device__ __forceinline__ void td_partials(double *acc, double
 
 __device__ __forceinline__ int ffreq_td(int i, int n) { return i <= (n - 1) / 2 ? i : i - n; }
 
-// spec *= 1/2 G^2 exp(-G^2 sigma^2 / 2) / N   (full grid, fftfreq on all axes)
-template <typename T>
-__global__ void k_td_gmul(cpx<T> *spec, long long n, int nx, int ny, int nz, double B0, double B1, double B2,
-                          double B3, double B4, double B5, double B6, double B7, double B8, double sigma,
-                          double scale) {
-    GRID_LOOP(i, n) {
-        const int iz = (int)(i % nz);
-        const long long r = i / nz;
-        const int iy = (int)(r % ny), ix = (int)(r / ny);
-        const int fx = ffreq_td(ix, nx), fy = ffreq_td(iy, ny), fz = ffreq_td(iz, nz);
-        const double gx = fx * B0 + fy * B3 + fz * B6;
-        const double gy = fx * B1 + fy * B4 + fz * B7;
-        const double gz = fx * B2 + fy * B5 + fz * B8;
-        const double gg = gx * gx + gy * gy + gz * gz;
-        const double f = 0.5 * gg * exp(-gg * sigma * sigma / 2.0) * scale;
-        cpx<T> v = spec[i];
-        spec[i] = cpx<T>{(T)(v.x * f), (T)(v.y * f)};
-    }
-}
-
-// batched form: element i of the stacked runs has grid index i % n
+// spec *= 1/2 G^2 exp(-G^2 sigma^2 / 2) / N (full grid, fftfreq on all axes);
+// element j of the stacked runs has grid index j % n
 template <typename T>
 __global__ void k_td_gmul_b(cpx<T> *spec, long long tot, long long n, int nx, int ny, int nz, double B0, double B1,
                             double B2, double B3, double B4, double B5, double B6, double B7, double B8, double sigma,
@@ -70,17 +53,39 @@ __global__ void k_td_gmul_b(cpx<T> *spec, long long tot, long long n, int nx, in
     }
 }
 
-// out = x + sgn * i (dt/2) (kin + v x)   with kin = -1/2 lap x already in `kin`
-// sums: (mode 1) p.out complex (no conj)   (mode 2) |out|^2
+#undef GRID_LOOP
+
+// ---------------------------------------------------------------- batched
+// nb independent runs (each its own psi, v and CG scalars; a single step is
+// the batch of one) advance in lock step: every Hamiltonian application is one batched C2C transform pair and
+// one launch over all runs (blockIdx.y = run); per-run FP64 partial sums are
+// laid out partials[(run * nblk + block) * K + t].  Runs that have converged
+// stop updating; the loop ends when all have.
+template <int K> __device__ __forceinline__ void run_partials(double *acc, double *partials) {
+    __shared__ double sm[16];
+#pragma unroll
+    for (int t = 0; t < K; ++t) {
+        const double s = block_sum(acc[t], sm);
+        if (threadIdx.x == 0) partials[((long long)blockIdx.y * gridDim.x + blockIdx.x) * K + t] = s;
+    }
+}
+
+#define RUN_LOOP(i, n) \
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < (n); i += (long long)gridDim.x * blockDim.x)
+
 template <typename T, int MODE>
-__global__ void k_td_apply(const cpx<T> *x, const cpx<T> *kin, const T *v, double hdt, cpx<T> *out, long long n,
-                           double *partials) {
+__global__ void k_tdb_apply(const cpx<T> *x, const cpx<T> *kin, const T *v, double hdt, cpx<T> *out, long long n,
+                            double *partials) {
+    const long long o = (long long)blockIdx.y * n;
+    x += o;
+    kin += o;
+    v += o;
+    out += o;
     double acc[2] = {0, 0};
-    GRID_LOOP(i, n) {
+    RUN_LOOP(i, n) {
         const cpx<T> a = x[i], k = kin[i];
         const double vv = (double)v[i];
         const double hr = (double)k.x + vv * (double)a.x, hi = (double)k.y + vv * (double)a.y;
-        // i * hdt * (hr + i hi) = -hdt hi + i hdt hr
         const double orr = (double)a.x - hdt * hi, oi = (double)a.y + hdt * hr;
         out[i] = cpx<T>{(T)orr, (T)oi};
         if (MODE == 1) {
@@ -90,140 +95,306 @@ __global__ void k_td_apply(const cpx<T> *x, const cpx<T> *kin, const T *v, doubl
             acc[0] += orr * orr + oi * oi;
         }
     }
-    if (MODE == 1) td_partials<2>(acc, partials);
-    if (MODE == 2) td_partials<1>(acc, partials);
+    if (MODE == 1) run_partials<2>(acc, partials);
+    if (MODE == 2) run_partials<1>(acc, partials);
 }
 
-// res = b - res (res holds A x0) ; p = res ; sums res.res (complex), |res|^2
 template <typename T>
-__global__ void k_td_init(const cpx<T> *b, cpx<T> *res, cpx<T> *p, long long n, double *partials) {
+__global__ void k_tdb_init(const cpx<T> *b, cpx<T> *res, cpx<T> *p, long long n, double *partials) {
+    const long long o = (long long)blockIdx.y * n;
     double acc[3] = {0, 0, 0};
-    GRID_LOOP(i, n) {
-        const cpx<T> bb = b[i], ax = res[i];
+    RUN_LOOP(i, n) {
+        const cpx<T> bb = b[o + i], ax = res[o + i];
         const cpx<T> r{bb.x - ax.x, bb.y - ax.y};
-        res[i] = r;
-        p[i] = r;
+        res[o + i] = r;
+        p[o + i] = r;
         acc[0] += (double)r.x * r.x - (double)r.y * r.y;
         acc[1] += 2.0 * (double)r.x * r.y;
         acc[2] += (double)r.x * r.x + (double)r.y * r.y;
     }
-    td_partials<3>(acc, partials);
+    run_partials<3>(acc, partials);
 }
 
-// x += a p ; res -= a v ; sums res.res (complex), |res|^2
-template <typename T>
-__global__ void k_td_update(cpx<T> *x, cpx<T> *res, const cpx<T> *p, const cpx<T> *v, double ar, double ai, long long n,
-                            double *partials) {
+// res -= a v ; sums res.res (complex), |res|^2.  X: also x += a p
+template <typename T, bool X>
+__global__ void k_tdb_update(cpx<T> *x, cpx<T> *res, const cpx<T> *p, const cpx<T> *v, RunScalars rs, long long n,
+                             double *partials) {
+    const int run = blockIdx.y;
+    const long long o = (long long)run * n;
     double acc[3] = {0, 0, 0};
-    GRID_LOOP(i, n) {
-        const cpx<T> pp = p[i], vv = v[i], xx = x[i], rr = res[i];
-        x[i] = cpx<T>{(T)(xx.x + ar * pp.x - ai * pp.y), (T)(xx.y + ar * pp.y + ai * pp.x)};
-        const double r0 = rr.x - (ar * vv.x - ai * vv.y), r1 = rr.y - (ar * vv.y + ai * vv.x);
-        res[i] = cpx<T>{(T)r0, (T)r1};
-        acc[0] += r0 * r0 - r1 * r1;
-        acc[1] += 2.0 * r0 * r1;
-        acc[2] += r0 * r0 + r1 * r1;
+    if (rs.active[run]) {
+        const double ar = rs.ar[run], ai = rs.ai[run];
+        RUN_LOOP(i, n) {
+            const cpx<T> vv = v[o + i], rr = res[o + i];
+            if constexpr (X) {
+                const cpx<T> pp = p[o + i], xx = x[o + i];
+                x[o + i] = cpx<T>{(T)(xx.x + ar * pp.x - ai * pp.y), (T)(xx.y + ar * pp.y + ai * pp.x)};
+            }
+            const double r0 = rr.x - (ar * vv.x - ai * vv.y), r1 = rr.y - (ar * vv.y + ai * vv.x);
+            res[o + i] = cpx<T>{(T)r0, (T)r1};
+            acc[0] += r0 * r0 - r1 * r1;
+            acc[1] += 2.0 * r0 * r1;
+            acc[2] += r0 * r0 + r1 * r1;
+        }
     }
-    td_partials<3>(acc, partials);
+    run_partials<3>(acc, partials);
 }
 
-// p = res + beta p
-template <typename T> __global__ void k_td_pupd(const cpx<T> *res, cpx<T> *p, double br, double bi, long long n) {
-    GRID_LOOP(i, n) {
-        const cpx<T> pp = p[i], rr = res[i];
-        p[i] = cpx<T>{(T)(rr.x + br * pp.x - bi * pp.y), (T)(rr.y + br * pp.y + bi * pp.x)};
+// x += a p
+template <typename T> __global__ void k_tdb_xupd(cpx<T> *x, const cpx<T> *p, RunScalars rs, long long n) {
+    const int run = blockIdx.y;
+    if (!rs.active[run]) return;
+    const long long o = (long long)run * n;
+    const double ar = rs.ar[run], ai = rs.ai[run];
+    RUN_LOOP(i, n) {
+        const cpx<T> pp = p[o + i], xx = x[o + i];
+        x[o + i] = cpx<T>{(T)(xx.x + ar * pp.x - ai * pp.y), (T)(xx.y + ar * pp.y + ai * pp.x)};
     }
 }
 
-template <typename T> __global__ void k_td_copy(const cpx<T> *a, cpx<T> *b, long long n) {
-    GRID_LOOP(i, n) b[i] = a[i];
+// p = res + b p
+template <typename T> __global__ void k_tdb_pupd(const cpx<T> *res, cpx<T> *p, RunScalars rs, long long n) {
+    const int run = blockIdx.y;
+    if (!rs.active[run]) return;
+    const long long o = (long long)run * n;
+    const double br = rs.br[run], bi = rs.bi[run];
+    RUN_LOOP(i, n) {
+        const cpx<T> pp = p[o + i], rr = res[o + i];
+        p[o + i] = cpx<T>{(T)(rr.x + br * pp.x - bi * pp.y), (T)(rr.y + br * pp.y + bi * pp.x)};
+    }
 }
 
-#undef GRID_LOOP
+// out[run * K + t] = sum_b partials[(run * nblk + b) * K + t]
+// one workgroup per (run, term); pub (the device view of pinned host memory,
+// or null) receives a copy for the host
+__global__ void k_tdb_reduce(const double *partials, int nblk, int K, double *out, double *pub) {
+    __shared__ double sm[16];
+    const int run = blockIdx.x / K, t = blockIdx.x % K;
+    double acc = 0.0;
+    for (int b = threadIdx.x; b < nblk; b += blockDim.x) acc += partials[((long long)run * nblk + b) * K + t];
+    acc = block_sum(acc, sm);
+    if (threadIdx.x == 0) {
+        out[blockIdx.x] = acc;
+        if (pub) pub[blockIdx.x] = acc;
+    }
+}
 
+#undef RUN_LOOP
+
+// The Hamiltonian product A x = x + i hdt (-1/2 lap_sigma x + v x) of nb
+// stacked runs.  Where the axes have size-specialised passes the kinetic
+// multiply is part of the x pass and the rest of the product (and its sums)
+// part of the inverse z pass; a CgStep, if given, is applied by the forward z
+// pass.  Else the complete transforms and separate kernels run.
+template <typename T> struct KinOp {
+    Plan &P;
+    hipStream_t s;
+    long long n;
+    int nb;      // runs
+    int nblk;    // workgroups per run of the streaming kernels
+    double sigma;
+    cpx<T> *kin;
+    const SizeOps<T> *zo, *xo;  // null: no size-specialised pass
+    KinOp(Plan &p, hipStream_t st, double sg, int runs, cpx<T> *k)
+        : P(p), s(st), n(p.N), nb(runs), sigma(sg), kin(k) {
+        nblk = std::max(1, std::min(reduce_blocks(n), nb == 1 ? 1024 : 256));
+        zo = P.use_fixed ? find_ops<T>(P.nr[2]) : nullptr;
+        xo = P.use_fixed && P.nr[0] * P.nr[1] > 1 ? find_ops<T>(P.nr[0]) : nullptr;
+        if (xo && P.nr[1] > 1 && !find_ops<T>(P.nr[1])) xo = nullptr;
+        if (P.nr[0] * P.nr[1] == 1) zo = nullptr;
+    }
+    bool steps() const { return zo != nullptr; }
+    // product into out; MODE 1 sums x . out, MODE 2 |out|^2 into P.red;
+    // returns the rows of partial sums per run
+    template <int MODE>
+    int apply(const cpx<T> *x, const T *v, double hdt, cpx<T> *out, const CgStep<T> *cg, unsigned mask) {
+        const unsigned m = xo ? mask : ~0u;  // generic passes take every run
+        if (zo) {
+            const long long nrows = (long long)P.nr[0] * P.nr[1];
+            const cpx<T> *tz = reinterpret_cast<const cpx<T> *>(P.tw[2]);
+            zo->rows_fwd(x, kin, nb, n, nrows, tz, (T)1, cg, mask, s, nullptr);
+            fft_cols<T>(P, 1, true, false, kin, kin, nb, n, 1.0, s, P.nr[2], m);
+            if (xo) {
+                GParams gp{};
+                for (int i = 0; i < 9; ++i) gp.B[i] = P.B[i];
+                gp.kind[0] = 4;
+                gp.c2c = 1;
+                gp.nx = P.nr[0];
+                gp.ny = P.nr[1];
+                gp.nz = P.nr[2];
+                gp.scale = 1.0 / (double)n;
+                gp.sigma = sigma;
+                xo->xfused(P.var_cols[0], kin, nb, n, (long long)P.nr[1] * P.nr[2], P.nr[2], P.nr[2],
+                           reinterpret_cast<const cpx<T> *>(P.tw[0]), gp, mask, s, nullptr);
+            } else {
+                fft_cols<T>(P, 0, true, false, kin, kin, nb, n, 1.0, s, P.nr[2]);
+                gmul();
+                fft_cols<T>(P, 0, true, true, kin, kin, nb, n, 1.0, s, P.nr[2]);
+            }
+            fft_cols<T>(P, 1, true, true, kin, kin, nb, n, 1.0, s, P.nr[2], m);
+            const ApplyArgs<T> ap{x, v, hdt, P.red};
+            const int rows = zo->rows_inv(MODE == 0 ? 3 : MODE, kin, out, nb, n, nrows, tz, (T)1, ap,
+                                          std::min(1024, 32768 / nb), mask, s, nullptr);
+            OFDFT_HIP(hipGetLastError());
+            return rows;
+        }
+        fft_c2c<T>(P, x, kin, false, nb, n, 1.0, s);
+        gmul();
+        fft_c2c<T>(P, kin, kin, true, nb, n, 1.0, s);
+        hipLaunchKernelGGL((k_tdb_apply<T, MODE>), dim3(nblk, nb), dim3(256), 0, s, x, kin, v, hdt, out, n, P.red);
+        OFDFT_HIP(hipGetLastError());
+        return nblk;
+    }
+    void gmul() {
+        const long long tot = (long long)nb * n;
+        hipLaunchKernelGGL((k_td_gmul_b<T>), dim3(std::min<long long>((tot + 255) / 256, 8192)), dim3(256), 0, s, kin,
+                           tot, n, P.nr[0], P.nr[1], P.nr[2], P.B[0], P.B[1], P.B[2], P.B[3], P.B[4], P.B[5], P.B[6],
+                           P.B[7], P.B[8], sigma, 1.0 / (double)n);
+        OFDFT_HIP(hipGetLastError());
+    }
+};
+
+// the operator and reductions of one run, for the Krylov solvers below
 template <typename T> struct CN {
     Plan &P;
     hipStream_t s;
     long long n;
-    int nb;
-    double *host;
-    double sigma;
-    cpx<T> *kin, *tmp;
-    CN(Plan &p, hipStream_t st, double sg) : P(p), s(st), n(p.N), sigma(sg) {
+    int nb;  // workgroups of the streaming kernels
+    KinOp<T> H;
+    CN(Plan &p, hipStream_t st, double sg)
+        : P(p), s(st), n(p.N), H(p, st, sg, 1, reinterpret_cast<cpx<T> *>(p.spec)) {
         nb = std::min(reduce_blocks(n), 1024);
-        host = P.pinned;
-        kin = reinterpret_cast<cpx<T> *>(P.spec);
     }
-
-    // the K sums, published by the reduction itself to the pinned buffer
-    const double *fetch(int K) {
+    // the K sums over `rows` partial rows, published by the reduction itself to the pinned buffer
+    const double *fetch(int K, int rows = 0) {
         std::vector<double> ones(K, 1.0);
-        reduce_final(P.red, nb, K, P.scal + 64, ones.data(), s, nullptr, P.scal + 64, P.pinned_dev, K);
+        reduce_final(P.red, rows ? rows : nb, K, P.scal + 64, ones.data(), s, nullptr, P.scal + 64, P.pinned_dev, K);
         stream_wait(s);
-        return host;
+        return P.pinned;
     }
-    // kin = -1/2 lap_sigma(x)
-    void kinetic(const cpx<T> *x) {
-        fft_c2c<T>(P, x, kin, false, 1, n, 1.0, s);
-        hipLaunchKernelGGL((k_td_gmul<T>), dim3(std::min<long long>((n + 255) / 256, 4096)), dim3(256), 0, s, kin, n,
-                           P.nr[0], P.nr[1], P.nr[2], P.B[0], P.B[1], P.B[2], P.B[3], P.B[4], P.B[5], P.B[6], P.B[7],
-                           P.B[8], sigma, 1.0 / (double)n);
-        OFDFT_HIP(hipGetLastError());
-        fft_c2c<T>(P, kin, kin, true, 1, n, 1.0, s);
+    template <int MODE> int apply(const cpx<T> *x, const T *v, double hdt, cpx<T> *out) {
+        return H.template apply<MODE>(x, v, hdt, out, nullptr, ~0u);
     }
-    template <int MODE> void apply(const cpx<T> *x, const T *v, double hdt, cpx<T> *out) {
-        kinetic(x);
-        hipLaunchKernelGGL((k_td_apply<T, MODE>), dim3(nb), dim3(256), 0, s, x, kin, v, hdt, out, n, P.red);
-        OFDFT_HIP(hipGetLastError());
+};
+
+template <typename T> struct CNBatch {
+    Plan &P;
+    hipStream_t s;
+    long long n;
+    int nb, nblk;
+    KinOp<T> H;
+    cpx<T> *b, *res, *p, *Ap;
+    // kin, b, res, p, Ap: nb stacked fields each
+    CNBatch(Plan &pl, hipStream_t st, double sg, int nruns, cpx<T> *kin, cpx<T> *work)
+        : P(pl), s(st), n(pl.N), nb(nruns), H(pl, st, sg, nruns, kin) {
+        nblk = H.nblk;
+        OFDFT_REQUIRE((long long)nb * nblk * 3 <= 4096LL * 16, "cn_step_batch: too many runs for the partials");
+        b = work;
+        res = work + (long long)nb * n;
+        p = work + 2LL * nb * n;
+        Ap = work + 3LL * nb * n;
     }
 
+    const double *fetch(int K, int rows) {
+        OFDFT_REQUIRE(nb * K <= 128, "cn_step_batch: read-back larger than the pinned buffer");
+        hipLaunchKernelGGL(k_tdb_reduce, dim3(nb * K), dim3(256), 0, s, P.red, rows, K, P.scal + 128, P.pinned_dev);
+        OFDFT_HIP(hipGetLastError());
+        stream_wait(s);
+        return P.pinned;
+    }
+    // The conjugate gradients of linear_solver.py:24-47, run by run.  With
+    // H.steps() the residual is updated alone after each product, and x and p
+    // by the next product's forward z pass (one read of p and one launch less
+    // per iteration); a run's last x is then updated by a kernel of its own.
     void step(const cpx<T> *psi0, const T *v, double dt, double tol, int maxiter, cpx<T> *x, double *info) {
-        cpx<T> *base = reinterpret_cast<cpx<T> *>(P.aux);
-        cpx<T> *b = base, *res = base + n, *p = base + 2 * n, *Ap = base + 3 * n;
-        // b = psi0 - i dt/2 H psi0, ||b||
-        apply<2>(psi0, v, -0.5 * dt, b);
-        const double bn = std::sqrt(fetch(1)[0]);
-        const double atol = bn == 0.0 ? tol : tol * bn;
-        // x = psi0 ; res = b - A x
-        if (x != psi0) hipLaunchKernelGGL((k_td_copy<T>), dim3(nb), dim3(256), 0, s, psi0, x, n);
-        apply<0>(x, v, 0.5 * dt, res);
-        hipLaunchKernelGGL((k_td_init<T>), dim3(nb), dim3(256), 0, s, b, res, p, n, P.red);
-        const double *h = fetch(3);
-        double rr_r = h[0], rr_i = h[1];
-        double rnorm = std::sqrt(h[2]);
-        int status = 1, k = 0;
-        if (rnorm < atol) {
-            status = 0;
-        } else {
-            while (k < maxiter) {
-                apply<1>(p, v, 0.5 * dt, Ap);
-                h = fetch(2);
-                const double pv_r = h[0], pv_i = h[1];
+        unsigned mask = ~0u;
+        int rows = H.template apply<2>(psi0, v, -0.5 * dt, b, nullptr, mask);
+        const double *h = fetch(1, rows);
+        double atol[kMaxRuns], rr_r[kMaxRuns], rr_i[kMaxRuns], rnorm[kMaxRuns];
+        int status[kMaxRuns], iters[kMaxRuns];
+        for (int r = 0; r < nb; ++r) {
+            const double bn = std::sqrt(h[r]);
+            atol[r] = bn == 0.0 ? tol : tol * bn;
+        }
+        if (x != psi0)
+            OFDFT_HIP(hipMemcpyAsync(x, psi0, (size_t)nb * n * sizeof(cpx<T>), hipMemcpyDeviceToDevice, s));
+        H.template apply<0>(x, v, 0.5 * dt, res, nullptr, mask);
+        hipLaunchKernelGGL((k_tdb_init<T>), dim3(nblk, nb), dim3(256), 0, s, b, res, p, n, P.red);
+        OFDFT_HIP(hipGetLastError());
+        h = fetch(3, nblk);
+        CgStep<T> cg{x, p, res, {}};
+        RunScalars &sc = cg.s;
+        int nactive = 0;
+        for (int r = 0; r < nb; ++r) {
+            rr_r[r] = h[3 * r];
+            rr_i[r] = h[3 * r + 1];
+            rnorm[r] = std::sqrt(h[3 * r + 2]);
+            iters[r] = 0;
+            status[r] = rnorm[r] < atol[r] ? 0 : 1;
+            sc.active[r] = status[r];
+            nactive += status[r];
+        }
+        for (int k = 0; k < maxiter && nactive > 0; ++k) {
+            mask = 0;
+            for (int r = 0; r < nb; ++r)
+                if (sc.active[r]) mask |= 1u << r;
+            rows = H.template apply<1>(p, v, 0.5 * dt, Ap, H.steps() && k > 0 ? &cg : nullptr, mask);
+            h = fetch(2, rows);
+            for (int r = 0; r < nb; ++r) {
+                if (!sc.active[r]) continue;
+                const double pv_r = h[2 * r], pv_i = h[2 * r + 1];
                 const double den = pv_r * pv_r + pv_i * pv_i;
-                const double ar = (rr_r * pv_r + rr_i * pv_i) / den, ai = (rr_i * pv_r - rr_r * pv_i) / den;
-                hipLaunchKernelGGL((k_td_update<T>), dim3(nb), dim3(256), 0, s, x, res, p, Ap, ar, ai, n, P.red);
-                h = fetch(3);
-                const double nr_r = h[0], nr_i = h[1];
-                rnorm = std::sqrt(h[2]);
-                ++k;
-                if (rnorm < atol) {
-                    status = 0;
-                    break;
-                }
-                const double d2 = rr_r * rr_r + rr_i * rr_i;
-                const double br = (nr_r * rr_r + nr_i * rr_i) / d2, bi = (nr_i * rr_r - nr_r * rr_i) / d2;
-                hipLaunchKernelGGL((k_td_pupd<T>), dim3(nb), dim3(256), 0, s, res, p, br, bi, n);
-                rr_r = nr_r;
-                rr_i = nr_i;
+                sc.ar[r] = (rr_r[r] * pv_r + rr_i[r] * pv_i) / den;
+                sc.ai[r] = (rr_i[r] * pv_r - rr_r[r] * pv_i) / den;
             }
+            if (H.steps())
+                hipLaunchKernelGGL((k_tdb_update<T, false>), dim3(nblk, nb), dim3(256), 0, s, x, res, p, Ap, sc, n,
+                                   P.red);
+            else
+                hipLaunchKernelGGL((k_tdb_update<T, true>), dim3(nblk, nb), dim3(256), 0, s, x, res, p, Ap, sc, n,
+                                   P.red);
+            OFDFT_HIP(hipGetLastError());
+            h = fetch(3, nblk);
+            RunScalars last = sc;  // the runs that end here
+            bool ends = false;
+            nactive = 0;
+            for (int r = 0; r < nb; ++r) {
+                last.active[r] = 0;
+                if (!sc.active[r]) continue;
+                const double nr_r = h[3 * r], nr_i = h[3 * r + 1];
+                rnorm[r] = std::sqrt(h[3 * r + 2]);
+                iters[r] = k + 1;
+                if (rnorm[r] < atol[r]) status[r] = 0;
+                if (status[r] == 0 || k + 1 == maxiter) {
+                    last.active[r] = 1;
+                    ends = true;
+                }
+                if (status[r] == 0) {
+                    sc.active[r] = 0;
+                    continue;
+                }
+                const double d2 = rr_r[r] * rr_r[r] + rr_i[r] * rr_i[r];
+                sc.br[r] = (nr_r * rr_r[r] + nr_i * rr_i[r]) / d2;
+                sc.bi[r] = (nr_i * rr_r[r] - nr_r * rr_i[r]) / d2;
+                rr_r[r] = nr_r;
+                rr_i[r] = nr_i;
+                ++nactive;
+            }
+            if (H.steps()) {
+                if (ends) hipLaunchKernelGGL((k_tdb_xupd<T>), dim3(nblk, nb), dim3(256), 0, s, x, p, last, n);
+            } else if (nactive > 0) {
+                hipLaunchKernelGGL((k_tdb_pupd<T>), dim3(nblk, nb), dim3(256), 0, s, res, p, sc, n);
+            }
+            OFDFT_HIP(hipGetLastError());
         }
         stream_wait(s);
-        if (info) {
-            info[0] = status;
-            info[1] = k;
-            info[2] = rnorm;
-            info[3] = atol;
-        }
+        if (info)
+            for (int r = 0; r < nb; ++r) {
+                info[4 * r] = status[r];
+                info[4 * r + 1] = iters[r];
+                info[4 * r + 2] = rnorm[r];
+                info[4 * r + 3] = atol[r];
+            }
     }
 };
 
@@ -519,8 +690,8 @@ template <typename T> struct CNK : CN<T> {
     void solve(int solver, int restart, const C *psi0, const T *v, double dt, double tol, int maxiter, C *x,
                double *info) {
         C *b = field(0);
-        this->template apply<2>(psi0, v, -0.5 * dt, b);
-        const double bn = std::sqrt(this->fetch(1)[0]);
+        const int rows = this->template apply<2>(psi0, v, -0.5 * dt, b);
+        const double bn = std::sqrt(this->fetch(1, rows)[0]);
         const double atol = bn == 0.0 ? tol : tol * bn;
         if (x != psi0) lin(psi0, 1.0, nullptr, 0.0, x);
         int k = 0, st = 1;
@@ -538,238 +709,6 @@ template <typename T> struct CNK : CN<T> {
             info[2] = rn;
             info[3] = atol;
         }
-    }
-};
-
-// ---------------------------------------------------------------- batched
-// nb independent runs (each its own psi, v and CG scalars) advance in lock
-// step: every Hamiltonian application is one batched C2C transform pair and
-// one launch over all runs (blockIdx.y = run); per-run FP64 partial sums are
-// laid out partials[(run * nblk + block) * K + t].  Runs that have converged
-// stop updating; the loop ends when all have.
-constexpr int kMaxRuns = 16;
-
-struct RunScalars {
-    double ar[kMaxRuns], ai[kMaxRuns];
-    int active[kMaxRuns];
-};
-
-template <int K> __device__ __forceinline__ void run_partials(double *acc, double *partials) {
-    __shared__ double sm[16];
-#pragma unroll
-    for (int t = 0; t < K; ++t) {
-        const double s = block_sum(acc[t], sm);
-        if (threadIdx.x == 0) partials[((long long)blockIdx.y * gridDim.x + blockIdx.x) * K + t] = s;
-    }
-}
-
-#define RUN_LOOP(i, n) \
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < (n); i += (long long)gridDim.x * blockDim.x)
-
-template <typename T, int MODE>
-__global__ void k_tdb_apply(const cpx<T> *x, const cpx<T> *kin, const T *v, double hdt, cpx<T> *out, long long n,
-                            double *partials) {
-    const long long o = (long long)blockIdx.y * n;
-    x += o;
-    kin += o;
-    v += o;
-    out += o;
-    double acc[2] = {0, 0};
-    RUN_LOOP(i, n) {
-        const cpx<T> a = x[i], k = kin[i];
-        const double vv = (double)v[i];
-        const double hr = (double)k.x + vv * (double)a.x, hi = (double)k.y + vv * (double)a.y;
-        const double orr = (double)a.x - hdt * hi, oi = (double)a.y + hdt * hr;
-        out[i] = cpx<T>{(T)orr, (T)oi};
-        if (MODE == 1) {
-            acc[0] += (double)a.x * orr - (double)a.y * oi;
-            acc[1] += (double)a.x * oi + (double)a.y * orr;
-        } else if (MODE == 2) {
-            acc[0] += orr * orr + oi * oi;
-        }
-    }
-    if (MODE == 1) run_partials<2>(acc, partials);
-    if (MODE == 2) run_partials<1>(acc, partials);
-}
-
-template <typename T>
-__global__ void k_tdb_init(const cpx<T> *b, cpx<T> *res, cpx<T> *p, long long n, double *partials) {
-    const long long o = (long long)blockIdx.y * n;
-    double acc[3] = {0, 0, 0};
-    RUN_LOOP(i, n) {
-        const cpx<T> bb = b[o + i], ax = res[o + i];
-        const cpx<T> r{bb.x - ax.x, bb.y - ax.y};
-        res[o + i] = r;
-        p[o + i] = r;
-        acc[0] += (double)r.x * r.x - (double)r.y * r.y;
-        acc[1] += 2.0 * (double)r.x * r.y;
-        acc[2] += (double)r.x * r.x + (double)r.y * r.y;
-    }
-    run_partials<3>(acc, partials);
-}
-
-template <typename T>
-__global__ void k_tdb_update(cpx<T> *x, cpx<T> *res, const cpx<T> *p, const cpx<T> *v, RunScalars rs, long long n,
-                             double *partials) {
-    const int run = blockIdx.y;
-    const long long o = (long long)run * n;
-    double acc[3] = {0, 0, 0};
-    if (rs.active[run]) {
-        const double ar = rs.ar[run], ai = rs.ai[run];
-        RUN_LOOP(i, n) {
-            const cpx<T> pp = p[o + i], vv = v[o + i], xx = x[o + i], rr = res[o + i];
-            x[o + i] = cpx<T>{(T)(xx.x + ar * pp.x - ai * pp.y), (T)(xx.y + ar * pp.y + ai * pp.x)};
-            const double r0 = rr.x - (ar * vv.x - ai * vv.y), r1 = rr.y - (ar * vv.y + ai * vv.x);
-            res[o + i] = cpx<T>{(T)r0, (T)r1};
-            acc[0] += r0 * r0 - r1 * r1;
-            acc[1] += 2.0 * r0 * r1;
-            acc[2] += r0 * r0 + r1 * r1;
-        }
-    }
-    run_partials<3>(acc, partials);
-}
-
-template <typename T> __global__ void k_tdb_pupd(const cpx<T> *res, cpx<T> *p, RunScalars rs, long long n) {
-    const int run = blockIdx.y;
-    if (!rs.active[run]) return;
-    const long long o = (long long)run * n;
-    const double br = rs.ar[run], bi = rs.ai[run];
-    RUN_LOOP(i, n) {
-        const cpx<T> pp = p[o + i], rr = res[o + i];
-        p[o + i] = cpx<T>{(T)(rr.x + br * pp.x - bi * pp.y), (T)(rr.y + br * pp.y + bi * pp.x)};
-    }
-}
-
-// out[run * K + t] = sum_b partials[(run * nblk + b) * K + t]
-// one workgroup per (run, term); pub (the device view of pinned host memory,
-// or null) receives a copy for the host
-__global__ void k_tdb_reduce(const double *partials, int nblk, int K, double *out, double *pub) {
-    __shared__ double sm[16];
-    const int run = blockIdx.x / K, t = blockIdx.x % K;
-    double acc = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) acc += partials[((long long)run * nblk + b) * K + t];
-    acc = block_sum(acc, sm);
-    if (threadIdx.x == 0) {
-        out[blockIdx.x] = acc;
-        if (pub) pub[blockIdx.x] = acc;
-    }
-}
-
-#undef RUN_LOOP
-
-template <typename T> struct CNBatch {
-    Plan &P;
-    hipStream_t s;
-    long long n;
-    int nb, nblk;
-    double *host;
-    double sigma;
-    cpx<T> *kin, *b, *res, *p, *Ap;
-    CNBatch(Plan &pl, hipStream_t st, double sg, int nruns, void *work)
-        : P(pl), s(st), n(pl.N), nb(nruns), sigma(sg) {
-        nblk = std::max(1, std::min(reduce_blocks(n), 256));
-        OFDFT_REQUIRE((long long)nb * nblk * 3 <= 4096LL * 16, "cn_step_batch: too many runs for the partials");
-        host = P.pinned;
-        cpx<T> *w = reinterpret_cast<cpx<T> *>(work);
-        kin = w;
-        b = w + (long long)nb * n;
-        res = w + 2LL * nb * n;
-        p = w + 3LL * nb * n;
-        Ap = w + 4LL * nb * n;
-    }
-
-    const double *fetch(int K) {
-        OFDFT_REQUIRE(nb * K <= 128, "cn_step_batch: read-back larger than the pinned buffer");
-        hipLaunchKernelGGL(k_tdb_reduce, dim3(nb * K), dim3(256), 0, s, P.red, nblk, K, P.scal + 128, P.pinned_dev);
-        OFDFT_HIP(hipGetLastError());
-        stream_wait(s);
-        return host;
-    }
-    void kinetic(const cpx<T> *x) {
-        fft_c2c<T>(P, x, kin, false, nb, n, 1.0, s);
-        const long long tot = (long long)nb * n;
-        hipLaunchKernelGGL((k_td_gmul_b<T>), dim3(std::min<long long>((tot + 255) / 256, 8192)), dim3(256), 0, s, kin,
-                           tot, n, P.nr[0], P.nr[1], P.nr[2], P.B[0], P.B[1], P.B[2], P.B[3], P.B[4], P.B[5], P.B[6],
-                           P.B[7], P.B[8], sigma, 1.0 / (double)n);
-        OFDFT_HIP(hipGetLastError());
-        fft_c2c<T>(P, kin, kin, true, nb, n, 1.0, s);
-    }
-    template <int MODE> void apply(const cpx<T> *x, const T *v, double hdt, cpx<T> *out) {
-        kinetic(x);
-        hipLaunchKernelGGL((k_tdb_apply<T, MODE>), dim3(nblk, nb), dim3(256), 0, s, x, kin, v, hdt, out, n, P.red);
-        OFDFT_HIP(hipGetLastError());
-    }
-    void step(const cpx<T> *psi0, const T *v, double dt, double tol, int maxiter, cpx<T> *x, double *info) {
-        apply<2>(psi0, v, -0.5 * dt, b);
-        const double *h = fetch(1);
-        double atol[kMaxRuns], rr_r[kMaxRuns], rr_i[kMaxRuns], rnorm[kMaxRuns];
-        int status[kMaxRuns], iters[kMaxRuns];
-        for (int r = 0; r < nb; ++r) {
-            const double bn = std::sqrt(h[r]);
-            atol[r] = bn == 0.0 ? tol : tol * bn;
-        }
-        OFDFT_HIP(hipMemcpyAsync(x, psi0, (size_t)nb * n * sizeof(cpx<T>), hipMemcpyDeviceToDevice, s));
-        apply<0>(x, v, 0.5 * dt, res);
-        hipLaunchKernelGGL((k_tdb_init<T>), dim3(nblk, nb), dim3(256), 0, s, b, res, p, n, P.red);
-        OFDFT_HIP(hipGetLastError());
-        h = fetch(3);
-        RunScalars sc{};
-        int nactive = 0;
-        for (int r = 0; r < nb; ++r) {
-            rr_r[r] = h[3 * r];
-            rr_i[r] = h[3 * r + 1];
-            rnorm[r] = std::sqrt(h[3 * r + 2]);
-            iters[r] = 0;
-            status[r] = rnorm[r] < atol[r] ? 0 : 1;
-            sc.active[r] = status[r];
-            nactive += status[r];
-        }
-        for (int k = 0; k < maxiter && nactive > 0; ++k) {
-            apply<1>(p, v, 0.5 * dt, Ap);
-            h = fetch(2);
-            for (int r = 0; r < nb; ++r) {
-                if (!sc.active[r]) continue;
-                const double pv_r = h[2 * r], pv_i = h[2 * r + 1];
-                const double den = pv_r * pv_r + pv_i * pv_i;
-                sc.ar[r] = (rr_r[r] * pv_r + rr_i[r] * pv_i) / den;
-                sc.ai[r] = (rr_i[r] * pv_r - rr_r[r] * pv_i) / den;
-            }
-            hipLaunchKernelGGL((k_tdb_update<T>), dim3(nblk, nb), dim3(256), 0, s, x, res, p, Ap, sc, n, P.red);
-            OFDFT_HIP(hipGetLastError());
-            h = fetch(3);
-            RunScalars bs = sc;
-            for (int r = 0; r < nb; ++r) {
-                if (!sc.active[r]) continue;
-                const double nr_r = h[3 * r], nr_i = h[3 * r + 1];
-                rnorm[r] = std::sqrt(h[3 * r + 2]);
-                iters[r] = k + 1;
-                if (rnorm[r] < atol[r]) {
-                    status[r] = 0;
-                    bs.active[r] = 0;
-                    continue;
-                }
-                const double d2 = rr_r[r] * rr_r[r] + rr_i[r] * rr_i[r];
-                bs.ar[r] = (nr_r * rr_r[r] + nr_i * rr_i[r]) / d2;
-                bs.ai[r] = (nr_i * rr_r[r] - nr_r * rr_i[r]) / d2;
-                rr_r[r] = nr_r;
-                rr_i[r] = nr_i;
-            }
-            hipLaunchKernelGGL((k_tdb_pupd<T>), dim3(nblk, nb), dim3(256), 0, s, res, p, bs, n);
-            OFDFT_HIP(hipGetLastError());
-            nactive = 0;
-            for (int r = 0; r < nb; ++r) {
-                sc.active[r] = bs.active[r];
-                nactive += bs.active[r];
-            }
-        }
-        stream_wait(s);
-        if (info)
-            for (int r = 0; r < nb; ++r) {
-                info[4 * r] = status[r];
-                info[4 * r + 1] = iters[r];
-                info[4 * r + 2] = rnorm[r];
-                info[4 * r + 3] = atol[r];
-            }
     }
 };
 
@@ -794,10 +733,12 @@ extern "C" int ofdft_cn_step_batch(ofdft_plan *plan, int nb, const void *psi0, c
         OFDFT_REQUIRE(work_bytes >= ofdft_cn_batch_workspace_bytes(plan, nb), "cn_step_batch: workspace too small");
         hipStream_t s = reinterpret_cast<hipStream_t>(stream);
         if (P->prec == OFDFT_FP64) {
-            CNBatch<double> c(*P, s, sigma, nb, work);
+            double2 *w = reinterpret_cast<double2 *>(work);
+            CNBatch<double> c(*P, s, sigma, nb, w, w + (long long)nb * P->N);
             c.step((const double2 *)psi0, (const double *)v, dt, tol, maxiter, (double2 *)psi1, info);
         } else {
-            CNBatch<float> c(*P, s, sigma, nb, work);
+            float2 *w = reinterpret_cast<float2 *>(work);
+            CNBatch<float> c(*P, s, sigma, nb, w, w + (long long)nb * P->N);
             c.step((const float2 *)psi0, (const float *)v, dt, tol, maxiter, (float2 *)psi1, info);
         }
         return 0;
@@ -827,10 +768,10 @@ extern "C" int ofdft_cn_step_solver(ofdft_plan *plan, int solver, int restart, c
         if (solver == CN_CG) {
             OFDFT_REQUIRE(P->aux_bytes >= (size_t)4 * P->N * (P->prec == OFDFT_FP64 ? 16 : 8), "cn_step: workspace");
             if (P->prec == OFDFT_FP64) {
-                CN<double> c(*P, s, sigma);
+                CNBatch<double> c(*P, s, sigma, 1, (double2 *)P->spec, (double2 *)P->aux);
                 c.step((const double2 *)psi0, (const double *)v, dt, tol, maxiter, (double2 *)psi1, info);
             } else {
-                CN<float> c(*P, s, sigma);
+                CNBatch<float> c(*P, s, sigma, 1, (float2 *)P->spec, (float2 *)P->aux);
                 c.step((const float2 *)psi0, (const float *)v, dt, tol, maxiter, (float2 *)psi1, info);
             }
             return 0;
@@ -863,10 +804,10 @@ extern "C" int ofdft_cn_step(ofdft_plan *plan, const void *psi0, const void *v, 
         OFDFT_REQUIRE(P->aux_bytes >= (size_t)4 * P->N * (P->prec == OFDFT_FP64 ? 16 : 8), "cn_step: workspace");
         hipStream_t s = reinterpret_cast<hipStream_t>(stream);
         if (P->prec == OFDFT_FP64) {
-            CN<double> c(*P, s, sigma);
+            CNBatch<double> c(*P, s, sigma, 1, (double2 *)P->spec, (double2 *)P->aux);
             c.step((const double2 *)psi0, (const double *)v, dt, tol, maxiter, (double2 *)psi1, info);
         } else {
-            CN<float> c(*P, s, sigma);
+            CNBatch<float> c(*P, s, sigma, 1, (float2 *)P->spec, (float2 *)P->aux);
             c.step((const float2 *)psi0, (const float *)v, dt, tol, maxiter, (float2 *)psi1, info);
         }
         return 0;

@@ -32,8 +32,7 @@ class Plan:
             self.autotune()
 
     def autotune(self):
-        """Pick the fastest variant of each FFT pass (ofdft_plan_autotune): tiles
-        of the row passes; tiles and radix orders of the column passes."""
+        """Pick the faster of two tiles for each FFT pass (ofdft_plan_autotune)."""
         v = np.zeros(4, dtype=np.int32)
         t = np.zeros(24, dtype=np.float32)
         _lib.check(_lib.lib.ofdft_plan_autotune(self.handle, _lib.iptr(v), t.ctypes.data_as(ctypes.POINTER(ctypes.c_float)),

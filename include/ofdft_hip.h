@@ -77,13 +77,13 @@ int ofdft_plan_set_lattice(ofdft_plan *plan, const double lattice[9]);
  * 0 forces the generic mixed-radix kernels everywhere. */
 int ofdft_plan_set_fft_kernels(ofdft_plan *plan, int fixed);
 /* FFT autotuner (no counterpart in the reference): times the variants of each
- * size-specialised pass on the plan's shapes and keeps the fastest.  The z
- * R2C and C2R row passes have 3 (0..2: default tile, halved, quartered); the
- * x and y column passes 6: tile v % 3 with the radix order v / 3 (0: radix
- * 8s first, as the length factorises; 1: reversed, odd radices first).
+ * size-specialised pass on the plan's shapes and keeps the fastest: two tiles
+ * a pass.  Variants 0..2 of the z R2C and C2R row passes and 0..5 of the x and
+ * y column passes are accepted; variant v has tile v % 2 and all give the same
+ * results.
  * variants (optional, 4 ints): chosen variant of the z R2C, z C2R, x and y
  * passes; times (optional, 24 floats): mean ms of each variant, 6 per pass
- * in that order (-1 where a pass has fewer).  The choice for a grid shape and
+ * in that order (-1 for those not timed).  The choice for a grid shape and
  * precision is kept for the process: later plans of that shape take it
  * without timing (times all -1), so every plan of a shape gives identical
  * transforms.  Synchronises stream. */

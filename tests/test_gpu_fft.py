@@ -144,3 +144,99 @@ def test_tile_variants_agree(shape, dtype):
         assert np.max(np.abs(F - tiles[0][0])) <= tol * np.max(np.abs(tiles[0][0]))
         assert abs(e - tiles[0][1]) <= tol * abs(tiles[0][1])
         assert np.max(np.abs(p - tiles[0][2])) <= tol * np.max(np.abs(tiles[0][2]))
+
+
+# every length with size-specialised passes (16 to 256, even, primes up to 13),
+# beside odd and generic lengths on the other axes
+def _smooth(n):
+    for p in (2, 3, 5, 7, 11, 13):
+        while n % p == 0:
+            n //= p
+    return n == 1
+
+
+LENGTHS = [n for n in range(16, 257, 2) if _smooth(n)]
+
+
+@pytest.mark.parametrize("n", LENGTHS)
+def test_each_length_on_each_axis(n):
+    from dftpy_amd import DirectField
+    for dtype in (torch.float64, torch.float32):
+        for shape in ((n, 5, 18), (7, n, 20), (3, 5, n)):
+            rng = np.random.default_rng(n)
+            f = rng.standard_normal(shape)
+            g = _grid(shape, dtype)
+            F = DirectField(g, data=f).fft()
+            ref = np.fft.rfftn(f) * g.dV
+            assert np.max(np.abs(F.data.cpu().numpy() - ref)) <= _tol(dtype) * np.max(np.abs(ref)) * 4
+            assert np.max(np.abs(F.ifft().data.cpu().numpy() - f)) <= _tol(dtype) * np.max(np.abs(f)) * 8
+            gc = _grid(shape, dtype, full=True)
+            z = f + 1j * rng.standard_normal(shape)
+            fld = DirectField(gc, data=torch.as_tensor(z), cplx=True)
+            C = fld.fft()
+            ref = np.fft.fftn(z) * gc.dV
+            assert np.max(np.abs(C.data.cpu().numpy() - ref)) <= _tol(dtype) * np.max(np.abs(ref)) * 4
+            assert np.max(np.abs(C.ifft().data.cpu().numpy() - z)) <= _tol(dtype) * np.max(np.abs(z)) * 8
+
+
+@pytest.mark.parametrize("shape", [(16, 18, 20), (22, 26, 28), (52, 78, 104), (36, 15, 98), (27, 32, 40), (162, 20, 30)])
+@pytest.mark.parametrize("full", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_evaluation_on_fixed_and_generic_passes(shape, full, dtype):
+    """TF + vW + WT + LDA + Hartree with the size-specialised passes (the x
+    pass with the multiply) and with the generic kernels.  FP64 to the
+    transforms' rounding, which vW's G^2 multiplies: G_max^2 / 2 times a few
+    ulps of sqrt(rho) over sqrt(rho), 1e-12 of the potential here; FP32
+    likewise, 4e-4."""
+    from dftpy_amd import DirectField, _lib
+    from dftpy_amd.functional import Functional, TotalFunctional
+    g = _grid(shape, dtype, full)
+    rng = np.random.default_rng(2)
+    rho = DirectField(g, data=0.02 + 0.01 * rng.random(shape))
+    ev = TotalFunctional(KE=Functional(type="KEDF", name="WT"), XC=Functional(type="XC", name="LDA"),
+                         H=Functional(type="HARTREE"))
+    out = []
+    for fixed in (1, 0):
+        _lib.check(_lib.lib.ofdft_plan_set_fft_kernels(g.plan().handle, fixed))
+        o = ev(rho)
+        out.append((o.energy, o.potential.numpy().astype(np.float64), ev(rho, calcType={"E"}).energy))
+    (e1, v1, x1), (e0, v0, x0) = out
+    tol = 1e-12 if dtype == torch.float64 else 4e-4
+    assert np.max(np.abs(v1 - v0)) <= tol * np.max(np.abs(v0))
+    etol = 1e-12 if dtype == torch.float64 else 1e-5
+    assert abs(e1 - e0) <= etol * abs(e0) and abs(x1 - x0) <= etol * abs(x0) and abs(x1 - e1) <= etol * abs(e1)
+
+
+@pytest.mark.parametrize("shape", [(16, 18, 20), (26, 50, 52), (22, 15, 30), (27, 32, 40), (1, 24, 36)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("maxiter", [100, 3])
+def test_cn_batch_on_fixed_and_generic_passes(shape, dtype, maxiter):
+    """Lock-step Crank-Nicolson solves with the fused passes and with the
+    generic kernels: three runs that need different numbers of iterations (one
+    of them a constant), and a stop at maxiter.  Converged runs: both residuals
+    are within atol and |A^-1| <= 1 (H is Hermitian), so the solutions differ
+    by 2 atol in the 2-norm at most, besides the rounding of the recursion;
+    after three steps, which amplify nothing much, by rounding alone."""
+    from dftpy_amd import _lib
+    from dftpy_amd.td import CrankNicholsonBatch
+    g = _grid(shape, dtype, full=True)
+    ct = torch.complex128 if dtype == torch.float64 else torch.complex64
+    rng = np.random.default_rng(4)
+    psi = torch.as_tensor(np.stack([np.full(shape, 0.1 + 0.0j),
+                                    rng.standard_normal(shape) + 1j * rng.standard_normal(shape),
+                                    0.1 + 0.01 * rng.standard_normal(shape)])).to(ct).cuda()
+    v = torch.as_tensor(np.stack([np.full(shape, 0.3), rng.random(shape), 0.1 * rng.random(shape)])).to(dtype).cuda()
+    tol = 1e-9 if dtype == torch.float64 else 1e-5
+    out = []
+    for fixed in (1, 0):
+        _lib.check(_lib.lib.ofdft_plan_set_fft_kernels(g.plan().handle, fixed))
+        cn = CrankNicholsonBatch(0.005, tol=tol, maxiter=maxiter)
+        y, status = cn(g, psi, v)
+        out.append((y.clone(), status, [d["iterations"] for d in cn.last_info]))
+    (y1, s1, k1), (y0, s0, k0) = out
+    assert s1 == s0 and all(abs(a - b) <= 1 for a, b in zip(k1, k0))
+    eps = torch.finfo(dtype).eps
+    for r in range(3):
+        diff = float((y1[r] - y0[r]).abs().square().sum().sqrt())
+        size = float(y0[r].abs().square().sum().sqrt())
+        assert diff <= (2 * cn.last_info[r]["atol"] if s0[r] == 0 else 0.0) + 100 * eps * size
