@@ -29,6 +29,7 @@
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
+typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 
 namespace ofdft {
 
@@ -1029,245 +1030,351 @@ __global__ void __launch_bounds__(OUTW_THREADS) k_cnn_out_walk(Geo g, OutWalk wk
     }
 }
 
-// dh[q][c] = sum_t W6[t][c] dout[q - off_t];  g = mask > 0 ? dh : 0 (bf16)
+// dh[q][c] = sum_t W6[t][c] dout[q - off_t];  g = mask > 0 ? dh : 0 (bf16).
+// FP32 matrix instructions (32 points x 32 channels x 2 taps, 14 of them, a
+// zero 28th tap): the weights stay in registers and a row of 32 channels leaves
+// as whole lines.  Bound by its 256 bytes per point.  96^3: 58 us, 86 with a
+// thread per point and the weights read from LDS for each.
 __global__ void __launch_bounds__(256) k_cnn_out_bwd(Geo g, const float *__restrict__ dout,
                                                      const float *__restrict__ w, const __bf16 *__restrict__ mask,
                                                      float *__restrict__ dh, __bf16 *__restrict__ gout) {
-    __shared__ float ws[KOUT];
-    for (int i = threadIdx.x; i < KOUT; i += blockDim.x) ws[i] = w[i];
-    __syncthreads();
-    const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= g.n) return;
-    int x, y, z;
-    decompose(g, p, x, y, z);
-    Nbr nb;
-    nb.init(g, x, y, z);
-    float acc[CH];
+    const int lane = threadIdx.x & 63, half = lane >> 5, c = lane & 31;
+    float wr[14];
 #pragma unroll
-    for (int c = 0; c < CH; ++c) acc[c] = 0.0f;
-#pragma unroll 3
-    for (int t = 0; t < NTAP; ++t) {
-        const float dv = dout[nb.at(NTAP - 1 - t)];  // q - off_t = q + off_{26-t}
-#pragma unroll
-        for (int c = 0; c < CH; ++c) acc[c] += ws[t * CH + c] * dv;
+    for (int s = 0; s < 14; ++s) {
+        const int t = 2 * s + half;
+        wr[s] = t < NTAP ? w[t * CH + c] : 0.0f;
     }
-    float4 *dd = reinterpret_cast<float4 *>(dh + p * CH);
+    const int ntiles = (int)((g.n + 31) / 32);
+    for (int tile = blockIdx.x * 4 + (threadIdx.x >> 6); tile < ntiles; tile += gridDim.x * 4) {
+        const long long p0 = (long long)tile * 32;
+        int x, y, z;
+        decompose(g, min(p0 + c, g.n - 1), x, y, z);  // lane's point
+        Nbr nb;
+        nb.init(g, x, y, z);
+        float dv[14];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) dd[q] = make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
-    const bf16x8 *mv = reinterpret_cast<const bf16x8 *>(mask + p * CH);
-    bf16x8 *gv = reinterpret_cast<bf16x8 *>(gout + p * CH);
+        for (int s = 0; s < 14; ++s) {  // q - off_t = q + off_{26-t}
+            const int t0 = NTAP - 1 - 2 * s, t1 = t0 > 0 ? t0 - 1 : 0;
+            dv[s] = dout[half ? nb.at(t1) : nb.at(t0)];
+        }
+        if (half) dv[13] = 0.0f;
+        float mk[16];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const bf16x8 mk = mv[q];
-        bf16x8 o;
+        for (int i = 0; i < 16; ++i) {
+            const long long p = p0 + half * 4 + (i & 3) + 8 * (i >> 2);
+            mk[i] = (float)mask[min(p, g.n - 1) * CH + c];
+        }
+        floatx16 acc;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = (float)mk[e] > 0.0f ? (__bf16)acc[q * 8 + e] : (__bf16)0.0f;
-        gv[q] = o;
+        for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < 14; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(dv[s], wr[s], acc, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const long long p = p0 + half * 4 + (i & 3) + 8 * (i >> 2);
+            if (p >= g.n) continue;
+            dh[p * CH + c] = acc[i];
+            gout[p * CH + c] = mk[i] > 0.0f ? (__bf16)acc[i] : (__bf16)0.0f;
+        }
     }
 }
 
 // --------------------------------------------------------- weight gradients
-constexpr int WG_CHUNK = 256;  // points per chunk
+// Gradients of the first and the last layer: D[c][col] = sum_p H[p][c] S[col][p],
+// H the 32 hidden channels, S the FP32 field(s) at the taps:
+//   IN   dW1[t][ch][co] = sum_p g[p][co] x0[ch][p + off_t]   (54 columns, and
+//        ones in column 54 for the bias)
+//   else dW6[t][c] = sum_q h[q][c] dout[q - off_t]           (27 columns; the
+//        bias sums dout on the way)
+// on FP32 matrix instructions (32 x 32 x 2): products and sums stay FP32 (the
+// BF16 operand is exact in it).  Every wave works alone: it gathers the columns
+// of 64 points into its part of the LDS (rows of the fields, so the loads are
+// coalesced) and contracts them there.  Bound by the matrix units: 64 cycles
+// per instruction, one or two per pair of points.  96^3 with the final sum: IN
+// 53 us, before (a thread per 8 outputs, 8 FMAs per gathered load) 1400; else
+// 35 and 877.  Loading the next chunk ahead gains nothing.
+constexpr int WF_POINTS = 64;           // points of a wave's chunk
+constexpr int WF_PITCH = WF_POINTS + 4;  // floats per column: 16-byte reads, 16 lanes in distinct banks
+constexpr int WF_WAVES = 4;
 
-// dW6[t][c] = sum_p dout[p] h[p + off_t][c]; db6 = sum_p dout[p].
-// 128 threads: thread j < 108 owns (t = j / 4, channels 8*(j%4)..+8); j == 108
-// the bias.  Grid-stride over chunks; partials[block][KOUT + 1].
-__global__ void __launch_bounds__(128) k_cnn_wgrad_out(Geo g, const float *__restrict__ dout,
-                                                       const __bf16 *__restrict__ h, float *__restrict__ partials) {
-    __shared__ float ds[WG_CHUNK];
-    const int j = threadIdx.x;
-    const int t = j / 4, cg = j % 4;
-    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    float accb = 0.0f;
-    const bf16x8 *hv = reinterpret_cast<const bf16x8 *>(h);
-    const long long nchunk = (g.n + WG_CHUNK - 1) / WG_CHUNK;
-    for (long long ck = blockIdx.x; ck < nchunk; ck += gridDim.x) {
-        const long long p0 = ck * WG_CHUNK;
-        __syncthreads();
-        for (int i = j; i < WG_CHUNK; i += 128) ds[i] = (p0 + i < g.n) ? dout[p0 + i] : 0.0f;
-        __syncthreads();
-        const int np = (int)min((long long)WG_CHUNK, g.n - p0);
-        if (j < 108) {
-            int x, y, z;
-            decompose(g, p0, x, y, z);
-            for (int i = 0; i < np; ++i) {
-                Nbr nb;
-                nb.init(g, x, y, z);
-                const bf16x8 v = hv[(long long)nb.at(t) * 4 + cg];
-                const float dv = ds[i];
+template <bool IN>
+__global__ void __launch_bounds__(64 * WF_WAVES) k_cnn_wgrad_f32(Geo g, const __bf16 *__restrict__ hid,
+                                                                 const float *__restrict__ fld,
+                                                                 float *__restrict__ partials) {
+    constexpr int NCT = IN ? 2 : 1, NF = IN ? 2 : 1, COLS = NTAP * NF, NCOL = COLS + 1;
+    __shared__ __attribute__((aligned(16))) float cols[WF_WAVES][NCOL * WF_PITCH];
+    __shared__ __attribute__((aligned(16))) __bf16 hs[WF_WAVES][WF_POINTS * CH];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float *cw = cols[wave];
+    bf16x8 *hw = reinterpret_cast<bf16x8 *>(hs[wave]);
+    const bf16x8 *hv = reinterpret_cast<const bf16x8 *>(hid);
+    floatx16 acc[NCT];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) acc[e] += dv * (float)v[e];
-                if (++z == g.nz) {
-                    z = 0;
-                    if (++y == g.ny) {
-                        y = 0;
-                        ++x;
-                    }
-                }
-            }
-        } else if (j == 108) {
-            for (int i = 0; i < np; ++i) accb += ds[i];
-        }
-    }
-    float *pp = partials + (long long)blockIdx.x * (KOUT + 1);
-    if (j < 108) {
+    for (int q = 0; q < NCT; ++q)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) pp[t * CH + cg * 8 + e] = acc[e];
-    } else if (j == 108) {
-        pp[KOUT] = accb;
-    }
-}
-
-// dW1[t][c][co] = sum_p g[p][co] x0[c][p + off_t]; db1[co] = sum_p g[p][co].
-// 256 threads: j < 216 owns (t = j / 8, c = (j / 4) % 2, co group j % 4);
-// 216 <= j < 220 the bias of co group j - 216.  partials[block][KIN + 32].
-__global__ void __launch_bounds__(256) k_cnn_wgrad_in(Geo g, const __bf16 *__restrict__ gin,
-                                                      const float *__restrict__ x0, float *__restrict__ partials) {
-    __shared__ bf16x8 gs[WG_CHUNK * 4];
-    const int j = threadIdx.x;
-    const int t = j / 8, c = (j / 4) % 2, cg = j % 4;
-    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    const bf16x8 *gv = reinterpret_cast<const bf16x8 *>(gin);
-    const long long nchunk = (g.n + WG_CHUNK - 1) / WG_CHUNK;
-    const bf16x8 zero8 = {};
-    for (long long ck = blockIdx.x; ck < nchunk; ck += gridDim.x) {
-        const long long p0 = ck * WG_CHUNK;
-        __syncthreads();
-        for (int i = j; i < WG_CHUNK * 4; i += 256) gs[i] = (p0 + i / 4 < g.n) ? gv[p0 * 4 + i] : zero8;
-        __syncthreads();
-        const int np = (int)min((long long)WG_CHUNK, g.n - p0);
-        if (j < 216) {
-            int x, y, z;
-            decompose(g, p0, x, y, z);
-            const float *xc = x0 + (long long)c * g.n;
-            for (int i = 0; i < np; ++i) {
-                Nbr nb;
-                nb.init(g, x, y, z);
-                const float xv = xc[nb.at(t)];
-                const bf16x8 gg = gs[i * 4 + cg];
+        for (int i = 0; i < 16; ++i) acc[q][i] = 0.0f;
+    float bias = 0.0f;
+    // the column past the taps: ones for the bias of IN; the lanes of further
+    // columns repeat it
+    cw[COLS * WF_PITCH + lane] = 1.0f;
+    const long long nchunk = (g.n + WF_POINTS - 1) / WF_POINTS;
+    const long long stride = (long long)gridDim.x * WF_WAVES;
+    for (long long ck = (long long)blockIdx.x * WF_WAVES + wave; ck < nchunk; ck += stride) {
+        const long long p0 = ck * WF_POINTS;
+        const bool valid = p0 + lane < g.n;
+        float v[COLS];
+        bf16x8 hr[4];
+        // addresses clamped: the tail is zeroed at the stores
 #pragma unroll
-                for (int e = 0; e < 8; ++e) acc[e] += xv * (float)gg[e];
-                if (++z == g.nz) {
-                    z = 0;
-                    if (++y == g.ny) {
-                        y = 0;
-                        ++x;
-                    }
-                }
-            }
-        } else if (j < 220) {
-            for (int i = 0; i < np; ++i) {
-                const bf16x8 gg = gs[i * 4 + (j - 216)];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) acc[e] += (float)gg[e];
-            }
-        }
-    }
-    float *pp = partials + (long long)blockIdx.x * (KIN + CH);
-    if (j < 216) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) pp[(t * 2 + c) * CH + cg * 8 + e] = acc[e];
-    } else if (j < 220) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) pp[KIN + (j - 216) * 8 + e] = acc[e];
-    }
-}
-
-// Mid-layer weight gradient with MFMA: dW[t][co][ci] = sum_p g[p][co] x[p+off_t][ci].
-// 4 waves; wave w owns the 16x16 block (co block w>>1, ci block w&1) of all 27
-// taps.  Per chunk of 256 points: g is staged transposed in LDS (gT[co][p])
-// once, and for each tap the shifted x rows are staged transposed (xT[ci][p]);
-// the MFMA K dimension runs over points.  partials[block][KMID + 32].
-constexpr int WG_PITCH = WG_CHUNK + 8;  // bf16 elements per LDS row (16-byte aligned)
-
-__global__ void __launch_bounds__(256) k_cnn_wgrad_mid(Geo g, const __bf16 *__restrict__ gin,
-                                                       const __bf16 *__restrict__ xin, float *__restrict__ partials) {
-    __shared__ __attribute__((aligned(16))) __bf16 gT[CH * WG_PITCH];
-    __shared__ __attribute__((aligned(16))) __bf16 xT[CH * WG_PITCH];
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int m = lane & 15, kq = lane >> 4;
-    const int mt = wave >> 1, nt = wave & 1;
-    floatx4 acc[NTAP];
-#pragma unroll
-    for (int t = 0; t < NTAP; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-    float dbacc = 0.0f;
-    const bf16x8 *gv = reinterpret_cast<const bf16x8 *>(gin);
-    const bf16x8 *xv = reinterpret_cast<const bf16x8 *>(xin);
-    const long long nchunk = (g.n + WG_CHUNK - 1) / WG_CHUNK;
-    const bf16x8 zero8 = {};
-    for (long long ck = blockIdx.x; ck < nchunk; ck += gridDim.x) {
-        const long long p = ck * WG_CHUNK + tid;  // this thread's point
-        const bool valid = p < g.n;
+        for (int q = 0; q < 4; ++q) hr[q] = hv[min(p0 * 4 + q * 64 + lane, g.n * 4 - 1)];
         int x, y, z;
-        decompose(g, valid ? p : 0, x, y, z);
+        decompose(g, min(p0 + lane, g.n - 1), x, y, z);
         Nbr nb;
         nb.init(g, x, y, z);
-        __syncthreads();
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const bf16x8 v = valid ? gv[p * 4 + q] : zero8;
+        for (int t = 0; t < NTAP; ++t)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) gT[(q * 8 + e) * WG_PITCH + tid] = v[e];
-        }
-        __syncthreads();
-        {  // bias gradient: thread (c = tid / 8, part = tid % 8) sums 32 points of channel c
-            const int c = tid >> 3, part = tid & 7;
-            float s = 0.0f;
-#pragma unroll 8
-            for (int i = 0; i < 32; ++i) s += (float)gT[c * WG_PITCH + part * 32 + i];
-            dbacc += s;
-        }
-        bf16x8 a[WG_CHUNK / 32];
+            for (int f = 0; f < NF; ++f) v[t * NF + f] = fld[f * g.n + nb.at(IN ? t : NTAP - 1 - t)];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");  // the last chunk's reads come first
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 #pragma unroll
-        for (int ks = 0; ks < WG_CHUNK / 32; ++ks)
-            a[ks] = *reinterpret_cast<const bf16x8 *>(&gT[(mt * 16 + m) * WG_PITCH + ks * 32 + kq * 8]);
-        bf16x8 xr[4];
+        for (int q = 0; q < 4; ++q) hw[q * 64 + lane] = p0 * 4 + q * 64 + lane < g.n * 4 ? hr[q] : bf16x8{};
 #pragma unroll
-        for (int q = 0; q < 4; ++q) xr[q] = valid ? xv[(long long)nb.at(0) * 4 + q] : zero8;
+        for (int i = 0; i < COLS; ++i) cw[i * WF_PITCH + lane] = valid ? v[i] : 0.0f;
+        if (!IN && valid) bias += v[NTAP / 2];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+        // points s and s + 32 of the chunk per instruction (lane halves)
+        const int half = (lane >> 5) * 32, cl = lane & 31;
+#pragma unroll 2
+        for (int s = 0; s < 32; s += 4) {
+            floatx4 b[NCT];
 #pragma unroll
-        for (int t = 0; t < NTAP; ++t) {
-            __syncthreads();  // previous tap's readers are done with xT
+            for (int q = 0; q < NCT; ++q)
+                b[q] = *reinterpret_cast<const floatx4 *>(&cw[min(q * 32 + cl, COLS) * WF_PITCH + half + s]);
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
+            for (int e = 0; e < 4; ++e) {
+                const float a = (float)hs[wave][(half + s + e) * CH + cl];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) xT[(q * 8 + e) * WG_PITCH + tid] = xr[q][e];
-            __syncthreads();
-            if (t + 1 < NTAP) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) xr[q] = valid ? xv[(long long)nb.at(t + 1) * 4 + q] : zero8;
+                for (int q = 0; q < NCT; ++q)
+                    acc[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b[q][e], acc[q], 0, 0, 0);
             }
+        }
+    }
+    // the waves' sums, in the order of the waves
+    __shared__ float bs[WF_WAVES];
+    if constexpr (!IN) {
+        for (int o = 32; o > 0; o >>= 1) bias += __shfl_down(bias, o);
+        if (lane == 0) bs[wave] = bias;
+    }
+    __syncthreads();
+    constexpr int WSUM = NCT * 1024;  // <= NCOL * WF_PITCH, a wave's part
 #pragma unroll
-            for (int ks = 0; ks < WG_CHUNK / 32; ++ks) {
-                const bf16x8 b = *reinterpret_cast<const bf16x8 *>(&xT[(nt * 16 + m) * WG_PITCH + ks * 32 + kq * 8]);
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ks], b, acc[t], 0, 0, 0);
+    for (int q = 0; q < NCT; ++q)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) cw[q * 1024 + i * 64 + lane] = acc[q][i];
+    __syncthreads();
+    const int K = COLS * CH + (IN ? CH : 1);
+    float *pp = partials + (long long)blockIdx.x * K;
+    for (int e = threadIdx.x; e < WSUM; e += 64 * WF_WAVES) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < WF_WAVES; ++w) sum += cols[w][e];
+        const int l = e & 63, i = (e >> 6) & 15, q = e >> 10;
+        const int col = q * 32 + (l & 31), c = (l >> 5) * 4 + (i & 3) + 8 * (i >> 2);
+        if (col < COLS + (IN ? 1 : 0)) pp[col * CH + c] = sum;
+    }
+    if (!IN && threadIdx.x == 0) pp[KOUT] = bs[0] + bs[1] + bs[2] + bs[3];
+}
+
+// Mid-layer weight gradient: dW[t][co][ci] = sum_p g[p][co] x[p + off_t][ci],
+// BF16 matrix instructions (32 co x 32 ci x 16 points) with FP32 sums.
+//
+// A workgroup walks a range of rows in steps of d along y (the rows y, y + d,
+// ... modulo ny form closed chains) for one x plane and z tile of ZT points.
+// At a step the x rows of chain position k (three planes x - d, x, x + d, with
+// the z halo) and the g row of position k + 1 are staged in LDS as they are in
+// memory; wave (i, kz) of nine takes the plane i and z tap kz and multiplies
+// its x fragments with the g rows k - 1, k and k + 1 (the three y taps), which
+// stay in registers: two fragments read per three products.  The points are
+// the contraction, so both operands are read transposed (ds_read_tr16: lane l
+// gets channel l % 32 of 8 points).  LDS reads (85 bytes per CU and cycle at
+// the full matrix rate), the imbalance of nine waves on four SIMDs and the
+// partial sums (57 MB each way; half as many workgroups would take 14 us less
+// and sum twice as many products in FP32) bound it.  96^3 with the final sum:
+// 88 us; 326 with the x rows staged transposed by scalar writes, for each tap
+// anew.  partials[block][KMID + 32].
+constexpr int WM_THREADS = 576;
+
+__device__ __forceinline__ bf16x8 frag_tr(const bf16x8 *rows, int lane) {
+    // lanes of a 16-lane group read 4 rows of 32 bytes and get a column each
+    using v4 = __attribute__((__vector_size__(4 * sizeof(short)))) short;
+    using lds4 = __attribute__((address_space(3))) v4;
+    const char *p = reinterpret_cast<const char *>(rows) + ((lane >> 5) * 8 + ((lane >> 2) & 3)) * (CH * 2) +
+                    ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+    union {
+        v4 h[2];
+        bf16x8 f;
+    } u;
+    u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4 *)p);
+    u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4 *)(p + 4 * CH * 2));
+    return u.f;
+}
+
+// a barrier that leaves the loads from memory in flight
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// SLOTS: 16-byte vectors a thread stages per step
+template <int ZT, int SLOTS>
+__global__ void __launch_bounds__(WM_THREADS) k_cnn_wgrad_mid(Geo g, const __bf16 *__restrict__ gin,
+                                                              const __bf16 *__restrict__ xin, int nzt, int cyc,
+                                                              float *__restrict__ partials) {
+    extern __shared__ bf16x8 lds[];  // 2 x ([ZT][4] g row + 3 x [xw][4] x rows)
+    constexpr int NK = ZT / 16;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wi = wave / 3, wk = wave % 3;
+    const bf16x8 *gv = reinterpret_cast<const bf16x8 *>(gin);
+    const bf16x8 *xv = reinterpret_cast<const bf16x8 *>(xin);
+    // staged z of x: [z0 - d, z0 + ZT + d), or the three taps' tiles where d > ZT
+    const int ds = min(g.d, ZT), xw = ZT + 2 * ds, nvec = (ZT + 3 * xw) * 4;
+    const int len = g.ny / cyc, nyz = g.ny * g.nz;
+    floatx16 acc[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[j][i] = 0.0f;
+    float db[8] = {};
+    // consecutive ranges to one XCD: neighbouring planes share its L2
+    const unsigned nb = gridDim.x;
+    const unsigned bl = nb % 8 == 0 ? (blockIdx.x % 8) * (nb / 8) + blockIdx.x / 8 : blockIdx.x;
+    const long long total = (long long)g.nx * nzt * g.ny;
+    const long long hi = total * (bl + 1) / nb;
+    int buf = 0;
+    for (long long r = total * bl / nb; r < hi;) {
+        const int item = (int)(r / len), k0 = (int)(r - (long long)item * len);
+        const int k1 = (int)min((long long)len, k0 + (hi - r));  // g rows [k0, k1) of the chain
+        r += k1 - k0;
+        const int c = item % cyc, zt = (item / cyc) % nzt, x = item / cyc / nzt, z0 = zt * ZT;
+        int base[SLOTS];  // point index of the slot's vector in row y = 0
+#pragma unroll
+        for (int s = 0; s < SLOTS; ++s) {
+            const int pt = (tid + s * WM_THREADS) >> 2;
+            if (pt < ZT) {
+                base[s] = z0 + pt < g.nz ? x * nyz + z0 + pt : -1;
+            } else {
+                const int e = min(pt - ZT, 3 * xw - 1), pl = e / xw, i = e - pl * xw;
+                const int dz = g.d <= ZT ? i - g.d : i % ZT + (i / ZT - 1) * g.d;
+                base[s] = wrapi(x + (pl - 1) * g.d, g.nx) * nyz + (z0 + dz + g.nz) % g.nz;
             }
+        }
+        // x rows of chain position k, g row of k + 1.  Straight-line: rows past the
+        // range are loaded again and replaced by zeros on their way to LDS, so
+        // that no wait stands behind a branch.
+        auto load = [&](bf16x8(&st)[SLOTS], int k) {
+            const int kx = min(k, k1), kg = min(k + 1, k1 - 1);
+            const int yx = (int)((unsigned)(c + (kx < 0 ? kx + len : (kx >= len ? kx - len : kx)) * g.d) % (unsigned)g.ny);
+            const int yg = (int)((unsigned)(c + kg * g.d) % (unsigned)g.ny);  // kg d < ny d < n
+#pragma unroll
+            for (int s = 0; s < SLOTS; ++s) {
+                const int v = tid + s * WM_THREADS;
+                const bf16x8 *src = v < ZT * 4 ? gv : xv;
+                const int row = (v < ZT * 4 ? yg : yx) * g.nz;
+                st[s] = src[(long long)(max(base[s], 0) + row) * 4 + (v & 3)];
+            }
+        };
+        auto store = [&](const bf16x8(&st)[SLOTS], int k, bf16x8 *dst) {
+            const bool g0 = tid < ZT * 4 && (base[0] < 0 || k + 1 >= k1);  // slot 0 has the g row
+            const bf16x8 f = g0 ? bf16x8{} : st[0];
+            dst[tid] = f;
+#pragma unroll
+            for (int s = 1; s < SLOTS; ++s)
+                if (tid + s * WM_THREADS < nvec) dst[tid + s * WM_THREADS] = st[s];
+            if (tid < ZT * 4) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) db[e] += (float)f[e];
+            }
+        };
+        // loads run two steps ahead of the stores to LDS
+        bf16x8 ga[NK] = {}, gb[NK] = {}, gc[NK] = {}, s0[SLOTS], s1[SLOTS];
+        load(s0, k0 - 1);
+        load(s1, k0);
+        __syncthreads();
+        store(s0, k0 - 1, lds + buf * nvec);
+        load(s0, k0 + 1);
+        lds_barrier();
+        auto step = [&](int k, bf16x8(&g0)[NK], bf16x8(&g1)[NK], bf16x8(&g2)[NK], bf16x8(&st)[SLOTS]) {
+            const bf16x8 *gr = lds + buf * nvec, *xr = gr + (ZT + wi * xw + wk * ds) * 4;
+#pragma unroll
+            for (int q = 0; q < NK; ++q) {
+                g2[q] = frag_tr(gr + q * 64, lane);
+                const bf16x8 xf = frag_tr(xr + q * 64, lane);
+                acc[2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(g0[q], xf, acc[2], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(g1[q], xf, acc[1], 0, 0, 0);
+                acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(g2[q], xf, acc[0], 0, 0, 0);
+            }
+            buf ^= 1;
+            store(st, k + 1, lds + buf * nvec);
+            load(st, k + 3);
+            lds_barrier();
+        };
+#pragma unroll 1
+        for (int k = k0 - 1; k <= k1; k += 6) {
+            step(k, ga, gb, gc, s1);
+            if (k + 1 <= k1) step(k + 1, gb, gc, ga, s0);
+            if (k + 2 <= k1) step(k + 2, gc, ga, gb, s1);
+            if (k + 3 <= k1) step(k + 3, ga, gb, gc, s0);
+            if (k + 4 <= k1) step(k + 4, gb, gc, ga, s1);
+            if (k + 5 <= k1) step(k + 5, gc, ga, gb, s0);
         }
     }
     float *pp = partials + (long long)blockIdx.x * (KMID + CH);
 #pragma unroll
-    for (int t = 0; t < NTAP; ++t)
+    for (int j = 0; j < 3; ++j)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) pp[t * CH * CH + (mt * 16 + kq * 4 + i) * CH + nt * 16 + m] = acc[t][i];
-    // bias: 8 partial sums per channel, reduced in LDS
+        for (int i = 0; i < 16; ++i) {
+            const int co = (lane >> 5) * 4 + (i & 3) + 8 * (i >> 2);
+            pp[((wi * 3 + j) * 3 + wk) * CH * CH + co * CH + (lane & 31)] = acc[j][i];
+        }
+    // bias: threads tid % 4 hold channels 8 (tid % 4) .. + 7 of their points
+    float *red = reinterpret_cast<float *>(lds);
     __syncthreads();
-    float *red = reinterpret_cast<float *>(gT);
-    red[tid] = dbacc;
+    if (tid < ZT * 4)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) red[tid * 8 + e] = db[e];
     __syncthreads();
     if (tid < CH) {
         float s = 0.0f;
-        for (int part = 0; part < 8; ++part) s += red[tid * 8 + part];
+        for (int i = 0; i < ZT; ++i) s += red[i * CH + tid];
         pp[KMID + tid] = s;
     }
 }
 
-// out[j] = sum_b partials[b * K + j]  (FP64 accumulation)
-__global__ void k_cnn_reduce(const float *__restrict__ partials, int nblk, int K, float *__restrict__ out) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= K) return;
+// out[j] = sum_b partials[b * K + j]  (FP64 accumulation): 64 columns a
+// workgroup, 16 slices of the rows (a thread per column took 124 us for 512
+// rows, whatever the layer)
+constexpr int RED_SLICES = 16;
+__global__ void __launch_bounds__(64 * RED_SLICES)
+    k_cnn_reduce(const float *__restrict__ partials, int nblk, int K, float *__restrict__ out) {
+    __shared__ double sm[RED_SLICES][64];
+    const int j = blockIdx.x * 64 + (threadIdx.x & 63), sl = threadIdx.x >> 6;
     double s = 0.0;
-    for (int b = 0; b < nblk; ++b) s += (double)partials[(long long)b * K + j];
-    out[j] = (float)s;
+    if (j < K) {
+#pragma unroll 8
+        for (int b = sl; b < nblk; b += RED_SLICES) s += (double)partials[(long long)b * K + j];
+    }
+    sm[sl][threadIdx.x & 63] = s;
+    __syncthreads();
+    if (sl == 0 && j < K) {
+        for (int i = 1; i < RED_SLICES; ++i) s += sm[i][threadIdx.x];
+        out[j] = (float)s;
+    }
 }
 
 // wf[t][co][ci] = bf16(W[t][co][ci]);  wb[t][ci][co] = bf16(W[26-t][co][ci])
@@ -1571,7 +1678,7 @@ int ofdft_cnn_out_backward(const int nr[3], int dil, const float *dout, const fl
     return cnn_guard([&] {
         const Geo g = make_geo(nr, dil);
         OFDFT_REQUIRE(dout && w && mask && dh && gout, "null pointer");
-        hipLaunchKernelGGL(k_cnn_out_bwd, dim3(blocks_for(g.n, 256)), dim3(256), 0, St(stream), g, dout, w,
+        hipLaunchKernelGGL(k_cnn_out_bwd, dim3(blocks_for(g.n, 512)), dim3(256), 0, St(stream), g, dout, w,
                            reinterpret_cast<const __bf16 *>(mask), dh, reinterpret_cast<__bf16 *>(gout));
         OFDFT_HIP(hipGetLastError());
     });
@@ -1582,30 +1689,71 @@ size_t ofdft_cnn_wgrad_partials(int layer, int nblk) {
     return (size_t)nblk * K;
 }
 
+static int launch_wgrad_mid(const Geo &g, const __bf16 *gin, const __bf16 *xin, float *partials, int most,
+                            hipStream_t st) {
+    // the tile with the least work: per padded point of 96^3 a 48-point tile
+    // takes 1.1 times as long as one of 64 and a 32-point tile 1.28 times
+    // (88, 73 and 85 us with tiles of 64 (a third of it padding), 48 and 32)
+    const int tiles[3] = {64, 48, 32};
+    const double cost[3] = {1.0, 1.1, 1.28};
+    int zt = 0;
+    double best = 0.0;
+    for (int i = 0; i < 3; ++i) {
+        const double c = (double)((g.nz + tiles[i] - 1) / tiles[i]) * tiles[i] * cost[i];
+        if (zt == 0 || c < best) {
+            best = c;
+            zt = tiles[i];
+        }
+    }
+    const int nzt = (g.nz + zt - 1) / zt, cyc = std::gcd(g.ny, g.d);
+    const int rows = (int)std::min<long long>(most, (long long)g.nx * nzt * g.ny);
+    const int nvec = (zt + 3 * (zt + 2 * std::min(g.d, zt))) * 4;
+    const size_t lds = 2 * (size_t)nvec * sizeof(bf16x8);  // <= 80 KB
+#define WM_LAUNCH(ZT, MORE)                                                                                          \
+    if (nvec <= 2 * WM_THREADS) {                                                                                    \
+        hipLaunchKernelGGL((k_cnn_wgrad_mid<ZT, 2>), dim3(rows), dim3(WM_THREADS), lds, st, g, gin, xin, nzt, cyc,    \
+                           partials);                                                                                \
+    } else {                                                                                                         \
+        rows_lds_limit((const void *)&k_cnn_wgrad_mid<ZT, MORE>, lds);                                               \
+        hipLaunchKernelGGL((k_cnn_wgrad_mid<ZT, MORE>), dim3(rows), dim3(WM_THREADS), lds, st, g, gin, xin, nzt, cyc, \
+                           partials);                                                                                \
+    }
+    if (zt == 64) {
+        WM_LAUNCH(64, 5)
+    } else if (zt == 48) {
+        WM_LAUNCH(48, 4)
+    } else {
+        WM_LAUNCH(32, 3)
+    }
+#undef WM_LAUNCH
+    return rows;
+}
+
 int ofdft_cnn_wgrad(const int nr[3], int dil, int layer, const void *g_in, const void *x, float *partials, int nblk,
                     float *dw, void *stream) {
     return cnn_guard([&] {
         const Geo g = make_geo(nr, dil);
         OFDFT_REQUIRE(g_in && x && partials && dw, "null pointer");
         OFDFT_REQUIRE(nblk >= 1 && nblk <= 65535, "nblk out of range");
-        int K = 0;
+        OFDFT_REQUIRE(layer >= 0 && layer <= 2, "layer must be 0 (input), 1 (32->32) or 2 (output)");
+        // as many of the nblk workgroups as have work
+        int K = 0, rows = (int)std::min<long long>(nblk, (g.n + WF_POINTS * WF_WAVES - 1) / (WF_POINTS * WF_WAVES));
         if (layer == 0) {
             K = KIN + CH;
-            hipLaunchKernelGGL(k_cnn_wgrad_in, dim3(nblk), dim3(256), 0, St(stream), g,
+            hipLaunchKernelGGL(k_cnn_wgrad_f32<true>, dim3(rows), dim3(64 * WF_WAVES), 0, St(stream), g,
                                reinterpret_cast<const __bf16 *>(g_in), reinterpret_cast<const float *>(x), partials);
         } else if (layer == 1) {
             K = KMID + CH;
-            hipLaunchKernelGGL(k_cnn_wgrad_mid, dim3(nblk), dim3(256), 0, St(stream), g,
-                               reinterpret_cast<const __bf16 *>(g_in), reinterpret_cast<const __bf16 *>(x), partials);
-        } else if (layer == 2) {
-            K = KOUT + 1;
-            hipLaunchKernelGGL(k_cnn_wgrad_out, dim3(nblk), dim3(128), 0, St(stream), g,
-                               reinterpret_cast<const float *>(g_in), reinterpret_cast<const __bf16 *>(x), partials);
+            rows = launch_wgrad_mid(g, reinterpret_cast<const __bf16 *>(g_in), reinterpret_cast<const __bf16 *>(x),
+                                    partials, nblk, St(stream));
         } else {
-            OFDFT_REQUIRE(false, "layer must be 0 (input), 1 (32->32) or 2 (output)");
+            K = KOUT + 1;
+            hipLaunchKernelGGL(k_cnn_wgrad_f32<false>, dim3(rows), dim3(64 * WF_WAVES), 0, St(stream), g,
+                               reinterpret_cast<const __bf16 *>(x), reinterpret_cast<const float *>(g_in), partials);
         }
         OFDFT_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_cnn_reduce, dim3(blocks_for(K, 256)), dim3(256), 0, St(stream), partials, nblk, K, dw);
+        hipLaunchKernelGGL(k_cnn_reduce, dim3(blocks_for(K, 64)), dim3(64 * RED_SLICES), 0, St(stream), partials,
+                           rows, K, dw);
         OFDFT_HIP(hipGetLastError());
     });
 }

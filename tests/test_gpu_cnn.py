@@ -267,3 +267,66 @@ def test_spectral_loss_matches_numpy():
         assert np.abs(g - gref).max() < 1e-5 * np.abs(gref).max()
         if np.all(w == 1):
             assert abs(ref - float((d * d).mean())) < 1e-9 * ref
+
+
+@pytest.mark.parametrize("nr,d,nblk", [((12, 10, 14), 1, 512), ((9, 8, 33), 4, 7), ((40, 36, 40), 30, 64), ((5, 6, 96), 2, 1),
+                                       ((40, 41, 70), 36, 512), ((70, 66, 128), 65, 512), ((12, 12, 48), 3, 512),
+                                       ((34, 33, 48), 31, 100), ((20, 20, 64), 8, 512), ((2, 2, 2), 1, 512)])
+def test_weight_gradients_of_one_layer(nr, d, nblk):
+    """Each layer's weight-gradient kernel against FP64 sums: FP32 sums of m
+    products in a workgroup (m its share of the points, with the rounding of
+    the product and the final addition) are within (m + 2) ulps / 2 of the sum
+    of the magnitudes.  Tiles of 64, 48 and 32 points, dilations beyond a tile,
+    closed chains of rows, more workgroups than work."""
+    from dftpy_amd import _lib
+    L, n = _lib.lib, int(np.prod(nr))
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=gen)  # noqa: E731
+    h, h2, f2, f1 = rnd(n, 32).bfloat16(), rnd(n, 32).bfloat16(), rnd(2, n), rnd(n)
+    nrc = np.ascontiguousarray(nr, dtype=np.int32)
+    for layer, g, x in ((0, h, f2), (1, h, h2), (2, f1, h)):
+        K = int(L.ofdft_cnn_wgrad_partials(layer, 1))
+        part = torch.full((K * nblk,), float("nan"), device="cuda")
+        dw = torch.empty(K, device="cuda")
+        _lib.check(L.ofdft_cnn_wgrad(_lib.iptr(nrc), d, layer, g.data_ptr(), x.data_ptr(), part.data_ptr(), nblk,
+                                     dw.data_ptr(), _lib.stream()))
+        rows = min(nblk, (n + 255) // 256) if layer != 1 else min(nblk, nr[0] * nr[1] * -(-nr[2] // 64))
+        for mag in (False, True):
+            G, X = (g.double().abs(), x.double().abs()) if mag else (g.double(), x.double())
+            sh = lambda a, t: torch.roll(a, [-d * (i - 1) for i in (t // 9, t // 3 % 3, t % 3)], (0, 1, 2))  # noqa: E731
+            out = []
+            for t in range(27):
+                if layer == 0:
+                    out += [G.T @ sh(X[c].view(*nr), t).reshape(-1) for c in range(2)]
+                elif layer == 1:
+                    out.append((G.T @ sh(X.view(*nr, 32), t).reshape(-1, 32)).reshape(-1))
+                else:
+                    out.append(G @ sh(X.view(*nr, 32), t).reshape(-1, 32))
+            out.append(G.sum(0).reshape(-1))
+            out = torch.cat(out)
+            if not mag:
+                ref = out
+        m = -(-n // rows) + 64
+        assert ((dw.double() - ref).abs() <= (m + 2) * 2.0 ** -24 * out).all()
+
+
+@pytest.mark.parametrize("nr,d", [((7, 6, 9), 2), ((32, 4, 5), 3), ((2, 2, 2), 1), ((16, 8, 33), 4)])
+def test_output_layer_backward(nr, d):
+    """dh against FP64 (27 products: 28 ulps / 2 of the magnitudes) and its
+    masked BF16 copy exactly."""
+    from dftpy_amd import _lib
+    n = int(np.prod(nr))
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    dout, w = torch.randn(n, device="cuda", generator=gen), torch.randn(27, 32, device="cuda", generator=gen)
+    mask = torch.randn(n, 32, device="cuda", generator=gen).bfloat16()
+    dh = torch.empty(n, 32, device="cuda")
+    go = torch.empty(n, 32, device="cuda", dtype=torch.bfloat16)
+    nrc = np.ascontiguousarray(nr, dtype=np.int32)
+    _lib.check(_lib.lib.ofdft_cnn_out_backward(_lib.iptr(nrc), d, dout.data_ptr(), w.data_ptr(), mask.data_ptr(),
+                                               dh.data_ptr(), go.data_ptr(), _lib.stream()))
+    ref = mag = 0.0
+    for t in range(27):
+        s = torch.roll(dout.double().view(*nr), [d * (i - 1) for i in (t // 9, t // 3 % 3, t % 3)], (0, 1, 2)).reshape(-1, 1)
+        ref, mag = ref + s * w[t].double(), mag + s.abs() * w[t].double().abs()
+    assert ((dh.double() - ref).abs() <= 28 * 2.0 ** -24 * mag).all()
+    assert torch.equal(go, torch.where(mask > 0, dh, torch.zeros_like(dh)).bfloat16())
