@@ -154,8 +154,8 @@ int ofdft_plan_create(const int nr[3], const double lattice[9], int precision, i
             const size_t nred = std::max<size_t>(
                 {4096 * 16, (size_t)nr[0] * nr[1] / 2 + 1, 7 * ((size_t)P->N / 1024 + 1)});
             OFDFT_HIP(hipMalloc(&P->red, sizeof(double) * nred));
-            OFDFT_HIP(hipMalloc(&P->scal, sizeof(double) * kScalSlots));
-            OFDFT_HIP(hipMemset(P->scal, 0, sizeof(double) * kScalSlots));
+            OFDFT_HIP(hipMalloc(&P->scal, sizeof(double) * (kScalSlots + kRunSlots)));
+            OFDFT_HIP(hipMemset(P->scal, 0, sizeof(double) * (kScalSlots + kRunSlots)));
             OFDFT_HIP(hipHostMalloc((void **)&P->pinned, 128 * sizeof(double), hipHostMallocMapped));
             OFDFT_HIP(hipHostGetDevicePointer((void **)&P->pinned_dev, P->pinned, 0));
             P->ws_bytes = spec_bytes + work_bytes + sizeof(double) * (nred + kScalSlots);

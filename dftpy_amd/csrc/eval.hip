@@ -128,7 +128,7 @@ static void gspace_apply(Plan &P, cpx<T> *spec, int ns, long long ncp, long long
     if (fused) {
         const long long ncols = (long long)P.nr[1] * pitch;
         find_ops<T>(P.nr[0])->xfused(P.var_cols[0], spec, ns, ncp, ncols, pitch, P.nzc,
-                                     reinterpret_cast<const cpx<T> *>(P.tw[0]), gp, ~0u, s, P.gate);
+                                     reinterpret_cast<const cpx<T> *>(P.tw[0]), gp, nullptr, s, P.gate);
     } else {
         hipLaunchKernelGGL((k_gspace<T>), dim3(grid_blocks(ncp)), dim3(256), 0, s, spec, ncp, gp, P.gate);
     }

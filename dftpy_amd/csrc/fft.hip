@@ -428,7 +428,7 @@ void plan_fft_free(Plan &P) {
 
 template <typename T>
 void fft_cols(Plan &P, int axis, bool full_grid, bool inverse, const cpx<T> *in, cpx<T> *out, int batch,
-              long long bs, double scale, hipStream_t s, long long pitch, unsigned mask) {
+              long long bs, double scale, hipStream_t s, long long pitch, const double *live) {
     const int n = P.nr[axis];
     const long long zlen = full_grid ? P.nr[2] : P.nzc;
     if (pitch <= 0) pitch = zlen;
@@ -448,12 +448,12 @@ void fft_cols(Plan &P, int axis, bool full_grid, bool inverse, const cpx<T> *in,
             Ss = ncols;
         }
         ops->cols(P.var_cols[axis], inverse, in, out, batch, bs, ncols, Pp, Qq, Ss, zlen,
-                  reinterpret_cast<const cpx<T> *>(P.tw[axis]), (T)scale, mask, s, P.gate);
+                  reinterpret_cast<const cpx<T> *>(P.tw[axis]), (T)scale, live, s, P.gate);
         OFDFT_HIP(hipGetLastError());
         return;
     }
     OFDFT_REQUIRE(pitch == zlen, "generic column pass needs an unpadded layout");
-    OFDFT_REQUIRE(P.gate == nullptr && mask == ~0u, "gated launch of a generic FFT pass");
+    OFDFT_REQUIRE(P.gate == nullptr && live == nullptr, "gated launch of a generic FFT pass");
     long long M, outer;
     PassShape sh;
     if (axis == 1) {
@@ -554,9 +554,9 @@ void fft_c2c(Plan &P, const cpx<T> *in, cpx<T> *out, bool inverse, int batch, lo
     OFDFT_REQUIRE(P.gate == nullptr, "gated launch of a generic FFT pass");
     if (const SizeOps<T> *ops = axis_ops<T>(P, 2)) {
         if (inverse)
-            ops->rows_inv(0, in, out, batch, bs, nrows, tw, sz, ApplyArgs<T>{}, 0, ~0u, s, nullptr);
+            ops->rows_inv(0, in, out, batch, bs, nrows, tw, sz, ApplyArgs<T>{}, 0, nullptr, s, nullptr);
         else
-            ops->rows_fwd(in, out, batch, bs, nrows, tw, sz, nullptr, ~0u, s, nullptr);
+            ops->rows_fwd(in, out, batch, bs, nrows, tw, sz, nullptr, nullptr, s, nullptr);
     } else if (inverse)
         hipLaunchKernelGGL((k_rows_c2c<T, true>), grid, dim3(sh.threads), sh.lds, s, in, out, bs, nrows, P.nr[2],
                            P.ax[2], tw, sh.tile, sz);
@@ -700,7 +700,7 @@ template void bench_rows_c2r<double>(Plan &, const double2 *, double *, int, hip
 
 #define INST(T)                                                                                               \
     template void fft_cols<T>(Plan &, int, bool, bool, const cpx<T> *, cpx<T> *, int, long long, double,       \
-                              hipStream_t, long long, unsigned);                                              \
+                              hipStream_t, long long, const double *);                                              \
     template void fft_r2c<T>(Plan &, const T *, cpx<T> *, int, long long, long long, double, const Prologue *, \
                              double *, hipStream_t, long long, bool);                                               \
     template void fft_c2r<T>(Plan &, const cpx<T> *, cpx<T> *, T *, int, long long, long long, long long,      \

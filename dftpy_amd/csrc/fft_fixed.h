@@ -137,15 +137,16 @@ __device__ __forceinline__ void dfts(C *buf, const C *tw, C (&v)[R], F &&done) {
     }
 }
 
-// runs of a batch that a launch leaves out (a set bit takes part)
-__device__ __forceinline__ bool run_off(unsigned mask, unsigned b) { return b < 32 && !((mask >> b) & 1u); }
+// runs of a batch that a launch leaves out: those whose entry of live (device
+// memory, null: none) is 0
+__device__ __forceinline__ bool run_off(const double *live, unsigned b) { return live != nullptr && live[b] == 0.0; }
 
 // ---------------------------------------------------------------- column pass
 template <typename T, int N, int TILE, bool INV>
 __global__ void __launch_bounds__((TILE *SL<T, N>::TP))
     k_cols_f(const cpx<T> *in, cpx<T> *out, long long bs, unsigned ncols, unsigned P, long long Q, long long S,
-             unsigned vp, const cpx<T> *__restrict__ twg, T scale, unsigned mask, const double *gate) {
-    if (gate_off(gate) || run_off(mask, blockIdx.y)) return;
+             unsigned vp, const cpx<T> *__restrict__ twg, T scale, const double *live, const double *gate) {
+    if (gate_off(gate) || run_off(live, blockIdx.y)) return;
     using C = cpx<T>;
     constexpr int R = SL<T, N>::first, TP = SL<T, N>::TP;
     __shared__ C tw[N];
@@ -234,8 +235,8 @@ __device__ __forceinline__ void xfactors(T *fac, const GParams &gp, int kind, in
 template <typename T, int N, int TILE>
 __global__ void __launch_bounds__((TILE *SL<T, N>::TP))
     k_xfused_f(cpx<T> *data, long long bs, unsigned ncols, unsigned pitch, unsigned vp,
-               const cpx<T> *__restrict__ twg, GParams gp, unsigned mask, const double *gate) {
-    if (gate_off(gate) || run_off(mask, blockIdx.y)) return;
+               const cpx<T> *__restrict__ twg, GParams gp, const double *live, const double *gate) {
+    if (gate_off(gate) || run_off(live, blockIdx.y)) return;
     using C = cpx<T>;
     constexpr int R = SL<T, N>::first, RL = SL<T, N>::last, TP = SL<T, N>::TP;
     __shared__ C tw[N];
@@ -506,12 +507,11 @@ __global__ void __launch_bounds__((NPEN *SL<T, N>::TP))
 }
 
 // ---------------------------------------------------------------- complex rows
-// per-run scalars of a lock-step batch of linear solves
+// Per-run scalars of a lock-step batch of linear solves, in device memory:
+// value k of run r at st[k * kMaxRuns + r]
 constexpr int kMaxRuns = 16;
-struct RunScalars {
-    double ar[kMaxRuns], ai[kMaxRuns], br[kMaxRuns], bi[kMaxRuns];
-    int active[kMaxRuns];
-};
+enum { RS_AR, RS_AI, RS_BR, RS_BI, RS_RR, RS_RI, RS_NORM, RS_ATOL, RS_ITERS, RS_STATUS, RS_LIVE, RS_COUNT };
+__device__ __forceinline__ double run_val(const double *st, int k, int run) { return st[k * kMaxRuns + run]; }
 
 // What the forward z pass of a lock-step batch reads: the field itself, or
 // the conjugate-gradient step x += a p, p = res + b p (the new p is
@@ -519,15 +519,15 @@ struct RunScalars {
 template <typename T> struct CgStep {
     cpx<T> *x, *p;
     const cpx<T> *res;
-    RunScalars s;
+    const double *st;
 };
 
 // Rows C2C forward.  STEP: the CG update above, else `in` is transformed.
 template <typename T, int N, int NPEN, bool STEP>
 __global__ void __launch_bounds__((NPEN *SL<T, N>::TP))
     k_rows_fwd_f(const cpx<T> *in, cpx<T> *out, long long bs, int nrows, const cpx<T> *__restrict__ twg, T scale,
-                 CgStep<T> cg, unsigned mask, const double *gate) {
-    if (gate_off(gate) || run_off(mask, blockIdx.y)) return;
+                 CgStep<T> cg, const double *live, const double *gate) {
+    if (gate_off(gate) || run_off(live, blockIdx.y)) return;
     using C = cpx<T>;
     constexpr int R = SL<T, N>::first, RL = SL<T, N>::last, TP = SL<T, N>::TP, LD = N + 1;
     __shared__ C tw[N];
@@ -545,8 +545,9 @@ __global__ void __launch_bounds__((NPEN *SL<T, N>::TP))
             r0[r] = cg.res[o + r * TP];
             x0[r] = cg.x[o + r * TP];
         }
-        const double ar = cg.s.ar[blockIdx.y], ai = cg.s.ai[blockIdx.y], br = cg.s.br[blockIdx.y],
-                     bi = cg.s.bi[blockIdx.y];
+        const int run = blockIdx.y;
+        const double ar = run_val(cg.st, RS_AR, run), ai = run_val(cg.st, RS_AI, run),
+                     br = run_val(cg.st, RS_BR, run), bi = run_val(cg.st, RS_BI, run);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const C pp = v[r], xx = x0[r], rr = r0[r];
@@ -589,8 +590,8 @@ template <typename T> struct ApplyArgs {
 template <typename T, int N, int NPEN, int MODE>
 __global__ void __launch_bounds__((NPEN *SL<T, N>::TP))
     k_rows_inv_f(const cpx<T> *in, cpx<T> *out, long long bs, int nrows, int ntiles, const cpx<T> *__restrict__ twg,
-                 T scale, ApplyArgs<T> ap, unsigned mask, const double *gate) {
-    if (gate_off(gate) || run_off(mask, blockIdx.y)) return;
+                 T scale, ApplyArgs<T> ap, const double *live, const double *gate) {
+    if (gate_off(gate) || run_off(live, blockIdx.y)) return;
     using C = cpx<T>;
     constexpr int R = SL<T, N>::first, RL = SL<T, N>::last, TP = SL<T, N>::TP, LD = N + 1;
     constexpr int K = MODE == 1 ? 2 : 1;
@@ -669,10 +670,10 @@ inline int tile_blocks(long long tiles, long long cap) {
 
 template <typename T> struct SizeOps {
     void (*cols)(int var, bool inv, const cpx<T> *in, cpx<T> *out, int batch, long long bs, long long ncols,
-                 long long P, long long Q, long long S, long long vp, const cpx<T> *tw, T scale, unsigned mask,
+                 long long P, long long Q, long long S, long long vp, const cpx<T> *tw, T scale, const double *live,
                  hipStream_t s, const double *gate);
     void (*xfused)(int var, cpx<T> *data, int batch, long long bs, long long ncols, long long pitch, long long vp,
-                   const cpx<T> *tw, const GParams &gp, unsigned mask, hipStream_t s, const double *gate);
+                   const cpx<T> *tw, const GParams &gp, const double *live, hipStream_t s, const double *gate);
     void (*r2c)(int var, const T *in, cpx<T> *out, int batch, long long in_bs, long long out_bs, long long nrows,
                 long long opitch, const cpx<T> *tw, T scale, const Prologue &pro, double *partials, int sum_slot,
                 hipStream_t s, const double *gate);
@@ -680,9 +681,9 @@ template <typename T> struct SizeOps {
     void (*c2r)(int var, const cpx<T> *in, T *out, int batch, long long in_bs, long long out_bs, long long nrows,
                 long long ipitch, const cpx<T> *tw, T scale, hipStream_t s, const double *gate);
     void (*rows_fwd)(const cpx<T> *in, cpx<T> *out, int batch, long long bs, long long nrows, const cpx<T> *tw,
-                     T scale, const CgStep<T> *cg, unsigned mask, hipStream_t s, const double *gate);
+                     T scale, const CgStep<T> *cg, const double *live, hipStream_t s, const double *gate);
     int (*rows_inv)(int mode, const cpx<T> *in, cpx<T> *out, int batch, long long bs, long long nrows,
-                    const cpx<T> *tw, T scale, const ApplyArgs<T> &ap, int cap, unsigned mask, hipStream_t s,
+                    const cpx<T> *tw, T scale, const ApplyArgs<T> &ap, int cap, const double *live, hipStream_t s,
                     const double *gate);
 };
 
@@ -691,7 +692,7 @@ template <typename T, int N> struct Launch {
     static constexpr int TP = SL<T, N>::TP;
 
     static void cols(int var, bool inv, const C *in, C *out, int batch, long long bs, long long ncols, long long P,
-                     long long Q, long long S, long long vp, const C *tw, T scale, unsigned mask, hipStream_t s,
+                     long long Q, long long S, long long vp, const C *tw, T scale, const double *live, hipStream_t s,
                      const double *gate) {
 #define CALL(V)                                                                                                        \
     {                                                                                                                  \
@@ -699,22 +700,22 @@ template <typename T, int N> struct Launch {
         const dim3 grid((unsigned)((ncols + TILE - 1) / TILE), (unsigned)batch);                                       \
         if (inv)                                                                                                       \
             hipLaunchKernelGGL((k_cols_f<T, N, TILE, true>), grid, dim3(TILE * TP), 0, s, in, out, bs, (unsigned)ncols, \
-                               (unsigned)P, Q, S, (unsigned)vp, tw, scale, mask, gate);                           \
+                               (unsigned)P, Q, S, (unsigned)vp, tw, scale, live, gate);                           \
         else                                                                                                           \
             hipLaunchKernelGGL((k_cols_f<T, N, TILE, false>), grid, dim3(TILE * TP), 0, s, in, out, bs,                 \
-                               (unsigned)ncols, (unsigned)P, Q, S, (unsigned)vp, tw, scale, mask, gate);          \
+                               (unsigned)ncols, (unsigned)P, Q, S, (unsigned)vp, tw, scale, live, gate);          \
     }
         OFDFT_VARIANT(var, CALL)
 #undef CALL
     }
     static void xfused(int var, C *data, int batch, long long bs, long long ncols, long long pitch, long long vp,
-                       const C *tw, const GParams &gp, unsigned mask, hipStream_t s, const double *gate) {
+                       const C *tw, const GParams &gp, const double *live, hipStream_t s, const double *gate) {
 #define CALL(V)                                                                                                        \
     {                                                                                                                  \
         constexpr int TILE = col_tile_v<T, N, V>();                                                                       \
         const dim3 grid((unsigned)((ncols + TILE - 1) / TILE), (unsigned)batch);                                       \
         hipLaunchKernelGGL((k_xfused_f<T, N, TILE>), grid, dim3(TILE * TP), 0, s, data, bs, (unsigned)ncols,           \
-                           (unsigned)pitch, (unsigned)vp, tw, gp, mask, gate);                                         \
+                           (unsigned)pitch, (unsigned)vp, tw, gp, live, gate);                                         \
     }
         OFDFT_VARIANT(var, CALL)
 #undef CALL
@@ -764,32 +765,32 @@ template <typename T, int N> struct Launch {
 #undef CALL
     }
     static void rows_fwd(const C *in, C *out, int batch, long long bs, long long nrows, const C *tw, T scale,
-                         const CgStep<T> *cg, unsigned mask, hipStream_t s, const double *gate) {
+                         const CgStep<T> *cg, const double *live, hipStream_t s, const double *gate) {
         constexpr int NP = pens_v<T, N, 1, 0>();
         const dim3 grid((unsigned)((nrows + NP - 1) / NP), (unsigned)batch);
         if (cg)
             hipLaunchKernelGGL((k_rows_fwd_f<T, N, NP, true>), grid, dim3(NP * TP), 0, s, in, out, bs, (int)nrows, tw,
-                               scale, *cg, mask, gate);
+                               scale, *cg, live, gate);
         else
             hipLaunchKernelGGL((k_rows_fwd_f<T, N, NP, false>), grid, dim3(NP * TP), 0, s, in, out, bs, (int)nrows, tw,
-                               scale, CgStep<T>{}, mask, gate);
+                               scale, CgStep<T>{}, live, gate);
     }
     template <int MODE>
     static int inv_mode(const C *in, C *out, int batch, long long bs, long long nrows, const C *tw, T scale,
-                        const ApplyArgs<T> &ap, int cap, unsigned mask, hipStream_t s, const double *gate) {
+                        const ApplyArgs<T> &ap, int cap, const double *live, hipStream_t s, const double *gate) {
         constexpr int NP = pens_v<T, N, 1, 0>();
         const long long tiles = (nrows + NP - 1) / NP;
         const int nb = tile_blocks(tiles, cap);
         hipLaunchKernelGGL((k_rows_inv_f<T, N, NP, MODE>), dim3((unsigned)nb, (unsigned)batch), dim3(NP * TP), 0, s, in,
-                           out, bs, (int)nrows, (int)tiles, tw, scale, ap, mask, gate);
+                           out, bs, (int)nrows, (int)tiles, tw, scale, ap, live, gate);
         return nb;
     }
     static int rows_inv(int mode, const C *in, C *out, int batch, long long bs, long long nrows, const C *tw, T scale,
-                        const ApplyArgs<T> &ap, int cap, unsigned mask, hipStream_t s, const double *gate) {
-        if (mode == 1) return inv_mode<1>(in, out, batch, bs, nrows, tw, scale, ap, cap, mask, s, gate);
-        if (mode == 2) return inv_mode<2>(in, out, batch, bs, nrows, tw, scale, ap, cap, mask, s, gate);
-        if (mode == 3) return inv_mode<3>(in, out, batch, bs, nrows, tw, scale, ap, 1 << 30, mask, s, gate);
-        return inv_mode<0>(in, out, batch, bs, nrows, tw, scale, ap, 1 << 30, mask, s, gate);
+                        const ApplyArgs<T> &ap, int cap, const double *live, hipStream_t s, const double *gate) {
+        if (mode == 1) return inv_mode<1>(in, out, batch, bs, nrows, tw, scale, ap, cap, live, s, gate);
+        if (mode == 2) return inv_mode<2>(in, out, batch, bs, nrows, tw, scale, ap, cap, live, s, gate);
+        if (mode == 3) return inv_mode<3>(in, out, batch, bs, nrows, tw, scale, ap, 1 << 30, live, s, gate);
+        return inv_mode<0>(in, out, batch, bs, nrows, tw, scale, ap, 1 << 30, live, s, gate);
     }
 };
 

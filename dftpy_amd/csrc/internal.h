@@ -98,6 +98,7 @@ constexpr int kColVariants = 6;
 // device scalars of a plan (FP64): [0, 256) the solvers' reduction results
 // and step scalars, [256, 1024) the state of the device-driven TN iteration
 constexpr int kScalSlots = 1024;
+constexpr int kRunSlots = 176;  // behind them: the scalars of a batch of linear solves (td.hip)
 
 // One plan: grid geometry, FFT plans, workspace and functional settings.
 struct Plan {
@@ -194,10 +195,10 @@ template <typename T>
 void fft_c2c(Plan &P, const cpx<T> *in, cpx<T> *out, bool inverse, int batch, long long bs, double scale,
              hipStream_t s);
 // the x/y passes alone (in place allowed), for fused pipelines; batch entries
-// b < 32 whose bit of mask is clear are left out
+// whose element of live (device memory, null: none) is 0 are left out
 template <typename T>
 void fft_cols(Plan &P, int axis, bool full_grid, bool inverse, const cpx<T> *in, cpx<T> *out, int batch,
-              long long bs, double scale, hipStream_t s, long long pitch = 0, unsigned mask = ~0u);
+              long long bs, double scale, hipStream_t s, long long pitch = 0, const double *live = nullptr);
 
 // single passes, for timing
 template <typename T>

@@ -882,7 +882,7 @@ template <typename T> struct Opt {
             gp.tab_inv_dq = 1.0 / P.tn_pre_dq;
             fft_r2c<T>(P, in, spec, 1, 0, ncp, 1.0, nullptr, nullptr, C.s, pitch, true);
             find_ops<T>(P.nr[0])->xfused(P.var_cols[0], spec, 1, ncp, (long long)P.nr[1] * pitch, pitch, P.nzc,
-                                         reinterpret_cast<const cpx<T> *>(P.tw[0]), gp, ~0u, C.s, P.gate);
+                                         reinterpret_cast<const cpx<T> *>(P.tw[0]), gp, nullptr, C.s, P.gate);
             OFDFT_HIP(hipGetLastError());
             fft_c2r<T>(P, spec, spec, out, 1, ncp, ncp, P.N, 1.0, C.s, pitch, true);
             return;

@@ -117,35 +117,34 @@ __global__ void k_tdb_init(const cpx<T> *b, cpx<T> *res, cpx<T> *p, long long n,
 
 // res -= a v ; sums res.res (complex), |res|^2.  X: also x += a p
 template <typename T, bool X>
-__global__ void k_tdb_update(cpx<T> *x, cpx<T> *res, const cpx<T> *p, const cpx<T> *v, RunScalars rs, long long n,
+__global__ void k_tdb_update(cpx<T> *x, cpx<T> *res, const cpx<T> *p, const cpx<T> *v, const double *st, long long n,
                              double *partials) {
     const int run = blockIdx.y;
+    if (run_val(st, RS_LIVE, run) == 0.0) return;
     const long long o = (long long)run * n;
     double acc[3] = {0, 0, 0};
-    if (rs.active[run]) {
-        const double ar = rs.ar[run], ai = rs.ai[run];
-        RUN_LOOP(i, n) {
-            const cpx<T> vv = v[o + i], rr = res[o + i];
-            if constexpr (X) {
-                const cpx<T> pp = p[o + i], xx = x[o + i];
-                x[o + i] = cpx<T>{(T)(xx.x + ar * pp.x - ai * pp.y), (T)(xx.y + ar * pp.y + ai * pp.x)};
-            }
-            const double r0 = rr.x - (ar * vv.x - ai * vv.y), r1 = rr.y - (ar * vv.y + ai * vv.x);
-            res[o + i] = cpx<T>{(T)r0, (T)r1};
-            acc[0] += r0 * r0 - r1 * r1;
-            acc[1] += 2.0 * r0 * r1;
-            acc[2] += r0 * r0 + r1 * r1;
+    const double ar = run_val(st, RS_AR, run), ai = run_val(st, RS_AI, run);
+    RUN_LOOP(i, n) {
+        const cpx<T> vv = v[o + i], rr = res[o + i];
+        if constexpr (X) {
+            const cpx<T> pp = p[o + i], xx = x[o + i];
+            x[o + i] = cpx<T>{(T)(xx.x + ar * pp.x - ai * pp.y), (T)(xx.y + ar * pp.y + ai * pp.x)};
         }
+        const double r0 = rr.x - (ar * vv.x - ai * vv.y), r1 = rr.y - (ar * vv.y + ai * vv.x);
+        res[o + i] = cpx<T>{(T)r0, (T)r1};
+        acc[0] += r0 * r0 - r1 * r1;
+        acc[1] += 2.0 * r0 * r1;
+        acc[2] += r0 * r0 + r1 * r1;
     }
     run_partials<3>(acc, partials);
 }
 
-// x += a p
-template <typename T> __global__ void k_tdb_xupd(cpx<T> *x, const cpx<T> *p, RunScalars rs, long long n) {
+// x += a p of each run's last iteration
+template <typename T> __global__ void k_tdb_xupd(cpx<T> *x, const cpx<T> *p, const double *st, long long n) {
     const int run = blockIdx.y;
-    if (!rs.active[run]) return;
+    if (run_val(st, RS_ITERS, run) == 0.0) return;
     const long long o = (long long)run * n;
-    const double ar = rs.ar[run], ai = rs.ai[run];
+    const double ar = run_val(st, RS_AR, run), ai = run_val(st, RS_AI, run);
     RUN_LOOP(i, n) {
         const cpx<T> pp = p[o + i], xx = x[o + i];
         x[o + i] = cpx<T>{(T)(xx.x + ar * pp.x - ai * pp.y), (T)(xx.y + ar * pp.y + ai * pp.x)};
@@ -153,29 +152,82 @@ template <typename T> __global__ void k_tdb_xupd(cpx<T> *x, const cpx<T> *p, Run
 }
 
 // p = res + b p
-template <typename T> __global__ void k_tdb_pupd(const cpx<T> *res, cpx<T> *p, RunScalars rs, long long n) {
+template <typename T> __global__ void k_tdb_pupd(const cpx<T> *res, cpx<T> *p, const double *st, long long n) {
     const int run = blockIdx.y;
-    if (!rs.active[run]) return;
+    if (run_val(st, RS_LIVE, run) == 0.0) return;
     const long long o = (long long)run * n;
-    const double br = rs.br[run], bi = rs.bi[run];
+    const double br = run_val(st, RS_BR, run), bi = run_val(st, RS_BI, run);
     RUN_LOOP(i, n) {
         const cpx<T> pp = p[o + i], rr = res[o + i];
         p[o + i] = cpx<T>{(T)(rr.x + br * pp.x - bi * pp.y), (T)(rr.y + br * pp.y + bi * pp.x)};
     }
 }
 
-// out[run * K + t] = sum_b partials[(run * nblk + b) * K + t]
-// one workgroup per (run, term); pub (the device view of pinned host memory,
-// or null) receives a copy for the host
-__global__ void k_tdb_reduce(const double *partials, int nblk, int K, double *out, double *pub) {
+// The scalars of the conjugate gradients (linear_solver.py:24-47), one
+// workgroup per run: the sums of a launch's partial rows, then the step they
+// decide.  CG_RHS: the tolerance from |b|^2; CG_INIT: the first residual;
+// CG_PAP: a = r.r / p.A p; CG_RES: the new residual and b, and whether the run
+// goes on.  CG_INIT and CG_RES publish iterations, residual, tolerance,
+// status, live and last the stage's number seq to pub (the device view of
+// pinned host memory, kPub doubles a run).
+enum { CG_RHS, CG_INIT, CG_PAP, CG_RES };
+constexpr int kPub = 6;
+template <int STAGE>
+__global__ void k_tdb_scalars(const double *partials, int nblk, double *st, double tol, int maxiter, double seq,
+                              double *pub) {
+    constexpr int K = STAGE == CG_RHS ? 1 : STAGE == CG_PAP ? 2 : 3;
     __shared__ double sm[16];
-    const int run = blockIdx.x / K, t = blockIdx.x % K;
-    double acc = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) acc += partials[((long long)run * nblk + b) * K + t];
-    acc = block_sum(acc, sm);
-    if (threadIdx.x == 0) {
-        out[blockIdx.x] = acc;
-        if (pub) pub[blockIdx.x] = acc;
+    const int run = blockIdx.x;
+    const bool live = STAGE == CG_RHS || STAGE == CG_INIT || run_val(st, RS_LIVE, run) != 0.0;
+    double h[K];
+    if (live) {  // uniform
+#pragma unroll
+        for (int t = 0; t < K; ++t) {
+            double acc = 0.0;
+            for (int b = threadIdx.x; b < nblk; b += blockDim.x) acc += partials[((long long)run * nblk + b) * K + t];
+            h[t] = block_sum(acc, sm);
+        }
+    }
+    if (threadIdx.x != 0) return;
+    auto v = [&](int k) -> double & { return st[k * kMaxRuns + run]; };
+    if (STAGE == CG_RHS) {
+        const double bn = sqrt(h[0]);
+        v(RS_ATOL) = bn == 0.0 ? tol : tol * bn;
+        return;
+    }
+    if (live) {
+        if constexpr (STAGE == CG_PAP) {
+            const double den = h[0] * h[0] + h[1] * h[1];
+            v(RS_AR) = (v(RS_RR) * h[0] + v(RS_RI) * h[1]) / den;
+            v(RS_AI) = (v(RS_RI) * h[0] - v(RS_RR) * h[1]) / den;
+            return;
+        }
+        if constexpr (STAGE == CG_INIT || STAGE == CG_RES) {
+            const double rn = sqrt(h[2]);
+            const bool done = rn < v(RS_ATOL);
+            const double it = STAGE == CG_INIT ? 0.0 : v(RS_ITERS) + 1.0;
+            if constexpr (STAGE == CG_RES) {
+                const double rr = v(RS_RR), ri = v(RS_RI), d2 = rr * rr + ri * ri;
+                v(RS_BR) = (h[0] * rr + h[1] * ri) / d2;
+                v(RS_BI) = (h[1] * rr - h[0] * ri) / d2;
+            }
+            v(RS_RR) = h[0];
+            v(RS_RI) = h[1];
+            v(RS_NORM) = rn;
+            v(RS_ITERS) = it;
+            v(RS_STATUS) = done ? 0.0 : 1.0;
+            v(RS_LIVE) = done || it >= maxiter ? 0.0 : 1.0;
+        }
+    }
+    if constexpr (STAGE == CG_INIT || STAGE == CG_RES) {
+        double *o = pub + run * kPub;
+        o[0] = v(RS_ITERS);
+        o[1] = v(RS_NORM);
+        o[2] = v(RS_ATOL);
+        o[3] = v(RS_STATUS);
+        o[4] = v(RS_LIVE);
+        __threadfence_system();
+        *(volatile double *)(o + 5) = seq;
     }
 }
 
@@ -207,12 +259,12 @@ template <typename T> struct KinOp {
     // product into out; MODE 1 sums x . out, MODE 2 |out|^2 into P.red;
     // returns the rows of partial sums per run
     template <int MODE>
-    int apply(const cpx<T> *x, const T *v, double hdt, cpx<T> *out, const CgStep<T> *cg, unsigned mask) {
-        const unsigned m = xo ? mask : ~0u;  // generic passes take every run
+    int apply(const cpx<T> *x, const T *v, double hdt, cpx<T> *out, const CgStep<T> *cg, const double *live) {
+        const double *m = xo ? live : nullptr;  // generic passes take every run
         if (zo) {
             const long long nrows = (long long)P.nr[0] * P.nr[1];
             const cpx<T> *tz = reinterpret_cast<const cpx<T> *>(P.tw[2]);
-            zo->rows_fwd(x, kin, nb, n, nrows, tz, (T)1, cg, mask, s, nullptr);
+            zo->rows_fwd(x, kin, nb, n, nrows, tz, (T)1, cg, live, s, nullptr);
             fft_cols<T>(P, 1, true, false, kin, kin, nb, n, 1.0, s, P.nr[2], m);
             if (xo) {
                 GParams gp{};
@@ -225,7 +277,7 @@ template <typename T> struct KinOp {
                 gp.scale = 1.0 / (double)n;
                 gp.sigma = sigma;
                 xo->xfused(P.var_cols[0], kin, nb, n, (long long)P.nr[1] * P.nr[2], P.nr[2], P.nr[2],
-                           reinterpret_cast<const cpx<T> *>(P.tw[0]), gp, mask, s, nullptr);
+                           reinterpret_cast<const cpx<T> *>(P.tw[0]), gp, live, s, nullptr);
             } else {
                 fft_cols<T>(P, 0, true, false, kin, kin, nb, n, 1.0, s, P.nr[2]);
                 gmul();
@@ -234,7 +286,7 @@ template <typename T> struct KinOp {
             fft_cols<T>(P, 1, true, true, kin, kin, nb, n, 1.0, s, P.nr[2], m);
             const ApplyArgs<T> ap{x, v, hdt, P.red};
             const int rows = zo->rows_inv(MODE == 0 ? 3 : MODE, kin, out, nb, n, nrows, tz, (T)1, ap,
-                                          std::min(1024, 32768 / nb), mask, s, nullptr);
+                                          std::min(1024, 32768 / nb), live, s, nullptr);
             OFDFT_HIP(hipGetLastError());
             return rows;
         }
@@ -273,7 +325,7 @@ template <typename T> struct CN {
         return P.pinned;
     }
     template <int MODE> int apply(const cpx<T> *x, const T *v, double hdt, cpx<T> *out) {
-        return H.template apply<MODE>(x, v, hdt, out, nullptr, ~0u);
+        return H.template apply<MODE>(x, v, hdt, out, nullptr, nullptr);
     }
 };
 
@@ -284,6 +336,7 @@ template <typename T> struct CNBatch {
     int nb, nblk;
     KinOp<T> H;
     cpx<T> *b, *res, *p, *Ap;
+    double *st;  // the runs' scalars
     // kin, b, res, p, Ap: nb stacked fields each
     CNBatch(Plan &pl, hipStream_t st, double sg, int nruns, cpx<T> *kin, cpx<T> *work)
         : P(pl), s(st), n(pl.N), nb(nruns), H(pl, st, sg, nruns, kin) {
@@ -293,107 +346,75 @@ template <typename T> struct CNBatch {
         res = work + (long long)nb * n;
         p = work + 2LL * nb * n;
         Ap = work + 3LL * nb * n;
+        static_assert(kMaxRuns * RS_COUNT <= kRunSlots, "scalars of the runs");
+        this->st = P.scal + kScalSlots;
     }
 
-    const double *fetch(int K, int rows) {
-        OFDFT_REQUIRE(nb * K <= 128, "cn_step_batch: read-back larger than the pinned buffer");
-        hipLaunchKernelGGL(k_tdb_reduce, dim3(nb * K), dim3(256), 0, s, P.red, rows, K, P.scal + 128, P.pinned_dev);
+    template <int STAGE> void scalars(int rows, double seq, double tol, int maxiter) {
+        hipLaunchKernelGGL((k_tdb_scalars<STAGE>), dim3(nb), dim3(256), 0, s, P.red, rows, st, tol, maxiter, seq,
+                           P.pinned_dev);
         OFDFT_HIP(hipGetLastError());
-        stream_wait(s);
-        return P.pinned;
     }
-    // The conjugate gradients of linear_solver.py:24-47, run by run.  With
-    // H.steps() the residual is updated alone after each product, and x and p
-    // by the next product's forward z pass (one read of p and one launch less
-    // per iteration); a run's last x is then updated by a kernel of its own.
+    // whether any run is live after stage seq (waits for its publication)
+    bool any_live(double seq) {
+        volatile const double *h = P.pinned;
+        for (int r = 0; r < nb; ++r)
+            for (unsigned spin = 1; h[r * kPub + 5] < seq; ++spin) {
+                if (spin % 1024) continue;
+                const hipError_t e = hipStreamQuery(s);
+                if (e == hipErrorNotReady) continue;
+                OFDFT_HIP(e);
+                OFDFT_REQUIRE(h[r * kPub + 5] >= seq, "cn_step: the solver's state was not published");
+            }
+        bool any = false;
+        for (int r = 0; r < nb; ++r) any = any || h[r * kPub + 4] != 0.0;
+        return any;
+    }
+    // The scalars stay on the device, where every launch looks up which runs
+    // are live; the host queues an iteration ahead and follows the published
+    // state one behind, so the device never waits for it (26 x 50 x 50, one
+    // run: 80 us an iteration with two waits, 47 now).  With H.steps()
+    // the residual is updated alone after each product, and x and p by the next
+    // product's forward z pass (one read of p and one launch less per
+    // iteration); every run's last x is updated at the end.
     void step(const cpx<T> *psi0, const T *v, double dt, double tol, int maxiter, cpx<T> *x, double *info) {
-        unsigned mask = ~0u;
-        int rows = H.template apply<2>(psi0, v, -0.5 * dt, b, nullptr, mask);
-        const double *h = fetch(1, rows);
-        double atol[kMaxRuns], rr_r[kMaxRuns], rr_i[kMaxRuns], rnorm[kMaxRuns];
-        int status[kMaxRuns], iters[kMaxRuns];
-        for (int r = 0; r < nb; ++r) {
-            const double bn = std::sqrt(h[r]);
-            atol[r] = bn == 0.0 ? tol : tol * bn;
-        }
+        const double *live = st + RS_LIVE * kMaxRuns;
+        for (int r = 0; r < nb; ++r) ((volatile double *)P.pinned)[r * kPub + 5] = -1.0;
+        int rows = H.template apply<2>(psi0, v, -0.5 * dt, b, nullptr, nullptr);
+        scalars<CG_RHS>(rows, 0.0, tol, maxiter);
         if (x != psi0)
             OFDFT_HIP(hipMemcpyAsync(x, psi0, (size_t)nb * n * sizeof(cpx<T>), hipMemcpyDeviceToDevice, s));
-        H.template apply<0>(x, v, 0.5 * dt, res, nullptr, mask);
+        H.template apply<0>(x, v, 0.5 * dt, res, nullptr, nullptr);
         hipLaunchKernelGGL((k_tdb_init<T>), dim3(nblk, nb), dim3(256), 0, s, b, res, p, n, P.red);
         OFDFT_HIP(hipGetLastError());
-        h = fetch(3, nblk);
-        CgStep<T> cg{x, p, res, {}};
-        RunScalars &sc = cg.s;
-        int nactive = 0;
-        for (int r = 0; r < nb; ++r) {
-            rr_r[r] = h[3 * r];
-            rr_i[r] = h[3 * r + 1];
-            rnorm[r] = std::sqrt(h[3 * r + 2]);
-            iters[r] = 0;
-            status[r] = rnorm[r] < atol[r] ? 0 : 1;
-            sc.active[r] = status[r];
-            nactive += status[r];
-        }
-        for (int k = 0; k < maxiter && nactive > 0; ++k) {
-            mask = 0;
-            for (int r = 0; r < nb; ++r)
-                if (sc.active[r]) mask |= 1u << r;
-            rows = H.template apply<1>(p, v, 0.5 * dt, Ap, H.steps() && k > 0 ? &cg : nullptr, mask);
-            h = fetch(2, rows);
-            for (int r = 0; r < nb; ++r) {
-                if (!sc.active[r]) continue;
-                const double pv_r = h[2 * r], pv_i = h[2 * r + 1];
-                const double den = pv_r * pv_r + pv_i * pv_i;
-                sc.ar[r] = (rr_r[r] * pv_r + rr_i[r] * pv_i) / den;
-                sc.ai[r] = (rr_i[r] * pv_r - rr_r[r] * pv_i) / den;
-            }
+        scalars<CG_INIT>(nblk, 0.0, tol, maxiter);
+        const CgStep<T> cg{x, p, res, st};
+        for (int k = 0; k < maxiter; ++k) {
+            if (k > 0 && !any_live(k - 1)) break;
+            rows = H.template apply<1>(p, v, 0.5 * dt, Ap, H.steps() && k > 0 ? &cg : nullptr, live);
+            scalars<CG_PAP>(rows, 0.0, tol, maxiter);
             if (H.steps())
-                hipLaunchKernelGGL((k_tdb_update<T, false>), dim3(nblk, nb), dim3(256), 0, s, x, res, p, Ap, sc, n,
+                hipLaunchKernelGGL((k_tdb_update<T, false>), dim3(nblk, nb), dim3(256), 0, s, x, res, p, Ap, st, n,
                                    P.red);
             else
-                hipLaunchKernelGGL((k_tdb_update<T, true>), dim3(nblk, nb), dim3(256), 0, s, x, res, p, Ap, sc, n,
+                hipLaunchKernelGGL((k_tdb_update<T, true>), dim3(nblk, nb), dim3(256), 0, s, x, res, p, Ap, st, n,
                                    P.red);
             OFDFT_HIP(hipGetLastError());
-            h = fetch(3, nblk);
-            RunScalars last = sc;  // the runs that end here
-            bool ends = false;
-            nactive = 0;
-            for (int r = 0; r < nb; ++r) {
-                last.active[r] = 0;
-                if (!sc.active[r]) continue;
-                const double nr_r = h[3 * r], nr_i = h[3 * r + 1];
-                rnorm[r] = std::sqrt(h[3 * r + 2]);
-                iters[r] = k + 1;
-                if (rnorm[r] < atol[r]) status[r] = 0;
-                if (status[r] == 0 || k + 1 == maxiter) {
-                    last.active[r] = 1;
-                    ends = true;
-                }
-                if (status[r] == 0) {
-                    sc.active[r] = 0;
-                    continue;
-                }
-                const double d2 = rr_r[r] * rr_r[r] + rr_i[r] * rr_i[r];
-                sc.br[r] = (nr_r * rr_r[r] + nr_i * rr_i[r]) / d2;
-                sc.bi[r] = (nr_i * rr_r[r] - nr_r * rr_i[r]) / d2;
-                rr_r[r] = nr_r;
-                rr_i[r] = nr_i;
-                ++nactive;
-            }
-            if (H.steps()) {
-                if (ends) hipLaunchKernelGGL((k_tdb_xupd<T>), dim3(nblk, nb), dim3(256), 0, s, x, p, last, n);
-            } else if (nactive > 0) {
-                hipLaunchKernelGGL((k_tdb_pupd<T>), dim3(nblk, nb), dim3(256), 0, s, res, p, sc, n);
-            }
+            scalars<CG_RES>(nblk, k + 1.0, tol, maxiter);
+            if (!H.steps())
+                hipLaunchKernelGGL((k_tdb_pupd<T>), dim3(nblk, nb), dim3(256), 0, s, res, p, st, n);
             OFDFT_HIP(hipGetLastError());
         }
+        if (H.steps()) hipLaunchKernelGGL((k_tdb_xupd<T>), dim3(nblk, nb), dim3(256), 0, s, x, p, st, n);
+        OFDFT_HIP(hipGetLastError());
         stream_wait(s);
         if (info)
             for (int r = 0; r < nb; ++r) {
-                info[4 * r] = status[r];
-                info[4 * r + 1] = iters[r];
-                info[4 * r + 2] = rnorm[r];
-                info[4 * r + 3] = atol[r];
+                const double *h = P.pinned + r * kPub;
+                info[4 * r] = h[3];
+                info[4 * r + 1] = h[0];
+                info[4 * r + 2] = h[1];
+                info[4 * r + 3] = h[2];
             }
     }
 };
