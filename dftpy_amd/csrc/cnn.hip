@@ -605,9 +605,17 @@ constexpr int RING_THREADS = 256;                        // 2 z tiles x 2 channe
 constexpr int RING_PER = (RING_PLANE + RING_THREADS - 1) / RING_THREADS;
 constexpr size_t RING_LDS = (size_t)(4 * RING_PLANE + 2 * RING_OUT) * 16 + CH * sizeof(float);  // + the bias
 
+//
+// MODE 0: out = x + relu(acc + b).  MODE 1 (training) stores relu(acc + b) to
+// out1 as well.  MODE 2 (backward-data): out0 = acc + resid (FP32, in place
+// allowed), out1 = out0 where mask > 0 (BF16), from registers, resid and mask
+// loaded at the top of the step (ahead of the plane that stays in flight).
+// 96^3: MODE 1 61 us and MODE 2 91; 101 and 133 on the row-tiled kernel.
+template <int MODE>
 __global__ void __launch_bounds__(RING_THREADS, 2)
     k_cnn_mid_ring(Geo g, const __bf16 *__restrict__ xin, const __bf16 *__restrict__ w,
-                   const float *__restrict__ bias, __bf16 *__restrict__ out) {
+                   const float *__restrict__ bias, const float *resid, const __bf16 *__restrict__ mask, void *out0,
+                   __bf16 *__restrict__ out1) {
     extern __shared__ bf16x8 lds[];
     bf16x8 *ostage = lds + 4 * RING_PLANE;
     const int d = g.d, nx = g.nx, ny = g.ny, nz = g.nz;
@@ -625,7 +633,7 @@ __global__ void __launch_bounds__(RING_THREADS, 2)
     const int co0 = hh * 16 + kq * 4;
     // the bias lives in LDS after the output stages (read once per step)
     float *bias_s = reinterpret_cast<float *>(ostage + 2 * RING_OUT);
-    if (tid < CH) bias_s[tid] = bias[tid];
+    if (MODE != 2 && tid < CH) bias_s[tid] = bias[tid];
     // y groups: per residue class mod d, ceil((ny / d) / 4) groups of 4 rows
     const int ngroups = d * ((ny / d + 3) / 4), nzb = (nz + RING_Z - 1) / RING_Z, walk = nx / d;
     const long long total = (long long)ngroups * nzb * d * walk;
@@ -716,7 +724,7 @@ __global__ void __launch_bounds__(RING_THREADS, 2)
         const int x = st.c + d * st.j;
         const bf16x8 *src = ostage + buf * RING_OUT;
         bf16x8 *ov =
-            reinterpret_cast<bf16x8 *>(out) + ((long long)x * nyz + (long long)st.y0 * nz + st.zb * RING_Z) * 4;
+            reinterpret_cast<bf16x8 *>(out0) + ((long long)x * nyz + (long long)st.y0 * nz + st.zb * RING_Z) * 4;
         const int ylim = ny - st.y0, zlim = nz - st.zb * RING_Z;  // rows and points of the step inside the grid
 #pragma unroll
         for (int q = 0; q < RING_OUT / RING_THREADS; ++q)
@@ -730,7 +738,7 @@ __global__ void __launch_bounds__(RING_THREADS, 2)
     // one step: `landing` holds plane j + 2 (issued a step earlier, or at the
     // walk's start), `issuing` receives plane j + 3
     auto do_step = [&](long long s, const Step &st, const Step &prev, bf16x8 *landing, bf16x8 *issuing) {
-        if (s > s_begin) copy_out(prev, (int)((s - 1) & 1));
+        if (MODE != 2 && s > s_begin) copy_out(prev, (int)((s - 1) & 1));
         if (s == s_begin || st.j == 0) {
             walk_setup(st);
             // the walk's first three planes, then plane j + 2 into the landing set
@@ -741,6 +749,24 @@ __global__ void __launch_bounds__(RING_THREADS, 2)
             }
             fetch(st, st.j + 2, landing);
             __syncthreads();
+        }
+        // this lane's output points (rows k) and channels co0 .. co0 + 3
+        const int zo = st.zb * RING_Z + zt * 16 + m;
+        long long eo[4];
+        bool on[4];
+        float4 rv[4];
+        bf16x4 mv[4];
+        if (MODE != 0) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int y = st.y0 + k * d;
+                on[k] = y < ny && zo < nz;
+                eo[k] = ((long long)(st.c + d * st.j) * nyz + (on[k] ? y * nz + zo : 0)) * CH + co0;
+                if (MODE == 2) {
+                    rv[k] = *reinterpret_cast<const float4 *>(resid + eo[k]);
+                    mv[k] = *reinterpret_cast<const bf16x4 *>(mask + eo[k]);
+                }
+            }
         }
         fetch(st, st.j + 3, issuing);
         floatx4 acc[4];
@@ -769,7 +795,20 @@ __global__ void __launch_bounds__(RING_THREADS, 2)
                                                                      acc[k], 0, 0, 0);
             }
         }
-        {
+        if constexpr (MODE == 2) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float v[4] = {acc[k][0] + rv[k].x, acc[k][1] + rv[k].y, acc[k][2] + rv[k].z, acc[k][3] + rv[k].w};
+                bf16x4 o4;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o4[e] = (float)mv[k][e] > 0.0f ? (__bf16)v[e] : (__bf16)0.0f;
+                if (on[k]) {
+                    *reinterpret_cast<float4 *>(reinterpret_cast<float *>(out0) + eo[k]) =
+                        make_float4(v[0], v[1], v[2], v[3]);
+                    *reinterpret_cast<bf16x4 *>(out1 + eo[k]) = o4;
+                }
+            }
+        } else {
             const __bf16 *rs = reinterpret_cast<const __bf16 *>(lds + ((head + 1) & 3) * RING_PLANE);
             __bf16 *os = reinterpret_cast<__bf16 *>(ostage + (int)(s & 1) * RING_OUT);
             const int z = zt * 16 + m;
@@ -782,11 +821,15 @@ __global__ void __launch_bounds__(RING_THREADS, 2)
             for (int k = 0; k < 4; ++k) {
                 // 4 channels of one point: one 8-byte LDS read and write
                 const bf16x4 x4 = *reinterpret_cast<const bf16x4 *>(rs + ((k + 1) * RING_ZS + zs) * CH + rin);
-                bf16x4 o4;
-                o4[0] = (__bf16)((float)x4[0] + fmaxf(acc[k][0] + bco.x, 0.0f));
-                o4[1] = (__bf16)((float)x4[1] + fmaxf(acc[k][1] + bco.y, 0.0f));
-                o4[2] = (__bf16)((float)x4[2] + fmaxf(acc[k][2] + bco.z, 0.0f));
-                o4[3] = (__bf16)((float)x4[3] + fmaxf(acc[k][3] + bco.w, 0.0f));
+                const float r[4] = {fmaxf(acc[k][0] + bco.x, 0.0f), fmaxf(acc[k][1] + bco.y, 0.0f),
+                                    fmaxf(acc[k][2] + bco.z, 0.0f), fmaxf(acc[k][3] + bco.w, 0.0f)};
+                bf16x4 o4, r4;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    o4[e] = (__bf16)((float)x4[e] + r[e]);
+                    r4[e] = (__bf16)r[e];
+                }
+                if (MODE == 1 && on[k]) *reinterpret_cast<bf16x4 *>(out1 + eo[k]) = r4;
                 *reinterpret_cast<bf16x4 *>(os + (k * RING_Z + z) * CH + rout) = o4;
             }
         }
@@ -807,7 +850,7 @@ __global__ void __launch_bounds__(RING_THREADS, 2)
         prev = st;
         advance(st);
     }
-    if (s_end > s_begin) copy_out(prev, (int)((s_end - 1) & 1));
+    if (MODE != 2 && s_end > s_begin) copy_out(prev, (int)((s_end - 1) & 1));
 }
 
 // ------------------------------------------------------------ layer 6 (32 -> 1)
@@ -1573,11 +1616,23 @@ int ofdft_cnn_conv_mid(const int nr[3], int dil, int mode, const void *x, const 
         OFDFT_REQUIRE(mode == 0 || mode == 1, "mode must be 0 (forward) or 1 (backward-data)");
         OFDFT_REQUIRE(mode == 1 || bias, "forward mode needs the bias");
         OFDFT_REQUIRE(mode == 0 || (resid && mask), "backward mode needs resid and mask");
-        if (mode == 0 && out1 == nullptr && g.nz >= RING_Z + RING_DMAX && g.ny % g.d == 0 && g.ny >= 4 * g.d &&
-            g.nx % g.d == 0 && g.d <= RING_DMAX) {
-            rows_lds_limit((const void *)&k_cnn_mid_ring, RING_LDS);
-            hipLaunchKernelGGL(k_cnn_mid_ring, dim3((unsigned)(2 * rows_workgroups())), dim3(RING_THREADS), RING_LDS,
-                               St(stream), g, xb, wb, bias, reinterpret_cast<__bf16 *>(out0));
+        const uintptr_t al = reinterpret_cast<uintptr_t>(resid) | reinterpret_cast<uintptr_t>(out0);
+        if (g.nz >= RING_Z + RING_DMAX && g.ny % g.d == 0 && g.ny >= 4 * g.d && g.nx % g.d == 0 && g.d <= RING_DMAX &&
+            (mode == 0 || (al & 15) == 0)) {
+            const dim3 grid((unsigned)(2 * rows_workgroups()));
+#define RING_LAUNCH(MD)                                                                                       \
+    do {                                                                                                      \
+        rows_lds_limit((const void *)&k_cnn_mid_ring<MD>, RING_LDS);                                          \
+        hipLaunchKernelGGL(k_cnn_mid_ring<MD>, grid, dim3(RING_THREADS), RING_LDS, St(stream), g, xb, wb, bias, \
+                           resid, reinterpret_cast<const __bf16 *>(mask), out0, reinterpret_cast<__bf16 *>(out1)); \
+    } while (0)
+            if (mode == 1)
+                RING_LAUNCH(2);
+            else if (out1)
+                RING_LAUNCH(1);
+            else
+                RING_LAUNCH(0);
+#undef RING_LAUNCH
             OFDFT_HIP(hipGetLastError());
             return;
         }
