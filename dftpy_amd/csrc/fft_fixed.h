@@ -141,6 +141,14 @@ __device__ __forceinline__ void dfts(C *buf, const C *tw, C (&v)[R], F &&done) {
 // memory, null: none) is 0
 __device__ __forceinline__ bool run_off(const double *live, unsigned b) { return live != nullptr && live[b] == 0.0; }
 
+// Consecutive workgroups go to the 8 XCDs in turn, each with its own L2.
+// Contiguous tiles to one XCD: where a row of elements is no multiple of a
+// cache line (the half grids' nzc = nz / 2 + 1), neighbouring tiles share lines.
+__device__ __forceinline__ unsigned xcd_tile(unsigned b, unsigned n) {
+    const unsigned q = n / 8, r = n % 8, x = b % 8;
+    return x * q + min(x, r) + b / 8;
+}
+
 // ---------------------------------------------------------------- column pass
 template <typename T, int N, int TILE, bool INV>
 __global__ void __launch_bounds__((TILE *SL<T, N>::TP))
@@ -153,7 +161,7 @@ __global__ void __launch_bounds__((TILE *SL<T, N>::TP))
     __shared__ C buf[N * TILE];
     const int pen = threadIdx.x % TILE;
     const int j = threadIdx.x / TILE;
-    const unsigned c = blockIdx.x * TILE + pen;
+    const unsigned c = xcd_tile(blockIdx.x, gridDim.x) * TILE + pen;
     const unsigned row = c / P, cp = c - row * P;
     const bool valid = c < ncols && cp < vp;  // pad columns of a pitched layout are skipped
     const long long off = (long long)blockIdx.y * bs + (valid ? (long long)row * Q + cp : 0) + j * S;
