@@ -697,6 +697,13 @@ __global__ void k_phase_tables(int nat, const double *__restrict__ frac, int nx,
 __device__ __forceinline__ double2 cmul2(double2 a, double2 b) { return double2{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x}; }
 
 __device__ __forceinline__ void half_index(long long i, int ny, int nzc, int &ix, int &iy, int &iz) {
+    if (i <= 0xffffffffLL) {  // 32-bit divisions: a quarter of the instructions
+        const unsigned u = (unsigned)i, r = u / (unsigned)nzc;
+        iz = (int)(u - r * (unsigned)nzc);
+        ix = (int)(r / (unsigned)ny);
+        iy = (int)(r - (unsigned)ix * (unsigned)ny);
+        return;
+    }
     iz = (int)(i % nzc);
     const long long rest = i / nzc;
     iy = (int)(rest % ny);
@@ -821,15 +828,17 @@ struct StressGIn {
     double eta;
 };
 
-// per masked G != 0, the six g_i g_j sums of: Hartree |rho|^2/G^4,
-// PP Re(rho v')/|G| (v' = sum_s dvloc_s/dq conj(S_s)), WT (g_i g_j/G^2 -
-// delta/3) eta G'(eta) Re(rA conj(rB)), Ewald |S_Z|^2 exp(-G^2/4eta)/G^2
-// (2 g_i g_j (1 + G^2/4eta)/G^2 - delta); partials [block][24]
-__global__ void k_stress_g(long long nc, GGeom g, StressGIn in, double *__restrict__ partials) {
+// per masked G != 0, the six g_i g_j sums of one term, partials [block][6]:
+// ST_H    |rho|^2 / G^4
+// ST_PP   Re(rho v') / |G|, v' = sum_s dvloc_s/dq conj(S_s)
+// ST_WT   (g_i g_j / G^2 - delta / 3) eta G'(eta) Re(rA conj(rB))
+// ST_EW   |S_Z|^2 exp(-G^2 / 4 eta) / G^2 (2 g_i g_j (1 + G^2 / 4 eta) / G^2 - delta)
+// Bound by the FP64 functions.  One term per instance: with all four and 64-bit
+// index divisions in one kernel a 160^3 launch took 63 us; 16 to 28 now.
+enum { ST_H, ST_PP, ST_WT, ST_EW };
+template <int TERM> __global__ void k_stress_g(long long nc, GGeom g, StressGIn in, double *__restrict__ partials) {
     __shared__ double sm[16];
-    double acc[24];
-#pragma unroll
-    for (int k = 0; k < 24; ++k) acc[k] = 0.0;
+    double acc[6] = {};
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < nc;
          i += (long long)gridDim.x * blockDim.x) {
         int ix, iy, iz;
@@ -841,45 +850,43 @@ __global__ void k_stress_g(long long nc, GGeom g, StressGIn in, double *__restri
         double G[3];
         gvec(g, f[0], f[1], f[2], G);
         const double gg = G[0] * G[0] + G[1] * G[1] + G[2] * G[2];
-        const double q = sqrt(gg), ig = 1.0 / gg;
-        double h = 0.0, pp = 0.0, wt = 0.0, ew = 0.0, ewd = 0.0;
-        if (in.rhoG) {
+        double c, diag = 0.0;  // c g_i g_j - diag delta
+        if constexpr (TERM == ST_H) {
             const double2 r = in.rhoG[i];
-            h = (r.x * r.x + r.y * r.y) * ig * ig;
-            if (in.Ss) {
-                double vx = 0.0, vy = 0.0;
-                for (int s = 0; s < in.nsp; ++s) {
-                    const double d = vloc_deriv(in.t, s, q);
-                    const double2 S = in.Ss[(long long)s * nc + i];
-                    vx += d * S.x;
-                    vy -= d * S.y;
-                }
-                pp = (r.x * vx - r.y * vy) / q;
+            const double ig = 1.0 / gg;
+            c = (r.x * r.x + r.y * r.y) * ig * ig;
+        } else if constexpr (TERM == ST_PP) {
+            const double q = sqrt(gg);
+            const double2 r = in.rhoG[i];
+            double vx = 0.0, vy = 0.0;
+            for (int s = 0; s < in.nsp; ++s) {
+                const double d = vloc_deriv(in.t, s, q);
+                const double2 S = in.Ss[(long long)s * nc + i];
+                vx += d * S.x;
+                vy -= d * S.y;
             }
-        }
-        if (in.rA) {
+            c = (r.x * vx - r.y * vy) / q;
+        } else if constexpr (TERM == ST_WT) {
             const double2 a = in.rA[i], b = in.rB[i];
-            wt = lindhard_deriv(q * in.itkf, in.mu) * (a.x * b.x + a.y * b.y);
-        }
-        if (in.SZ) {
+            const double wt = lindhard_deriv(sqrt(gg) * in.itkf, in.mu) * (a.x * b.x + a.y * b.y);
+            c = wt / gg;
+            diag = wt * (1.0 / 3.0);
+        } else {
             const double2 S = in.SZ[i];
-            const double e = (S.x * S.x + S.y * S.y) * exp(-gg / (4.0 * in.eta)) * ig;
-            ew = e * 2.0 * ig * (1.0 + gg / (4.0 * in.eta));
-            ewd = e;
+            const double ig = 1.0 / gg, x = gg / (4.0 * in.eta);
+            diag = (S.x * S.x + S.y * S.y) * exp(-x) * ig;
+            c = diag * 2.0 * ig * (1.0 + x);
         }
-        int k = 0;
-        for (int a = 0; a < 3; ++a)
-            for (int b = a; b < 3; ++b, ++k) {
-                const double gab = G[a] * G[b];
-                acc[k] += gab * h;
-                acc[6 + k] += gab * pp;
-                acc[12 + k] += (gab * ig - (a == b ? 1.0 / 3.0 : 0.0)) * wt;
-                acc[18 + k] += gab * ew - (a == b ? ewd : 0.0);
-            }
+        acc[0] += G[0] * G[0] * c - diag;
+        acc[1] += G[0] * G[1] * c;
+        acc[2] += G[0] * G[2] * c;
+        acc[3] += G[1] * G[1] * c - diag;
+        acc[4] += G[1] * G[2] * c;
+        acc[5] += G[2] * G[2] * c - diag;
     }
-    for (int k = 0; k < 24; ++k) {
+    for (int k = 0; k < 6; ++k) {
         const double v = block_sum(acc[k], sm);
-        if (threadIdx.x == 0) partials[(long long)blockIdx.x * 24 + k] = v;
+        if (threadIdx.x == 0) partials[(long long)blockIdx.x * 6 + k] = v;
     }
 }
 
@@ -898,7 +905,8 @@ __global__ void k_grad_spectra(long long nc, GGeom g, const double2 *__restrict_
     }
 }
 
-// [block][7]: six sums of d_i d_j / rho, and the sum of v_xc rho
+// [block][7]: six sums of d_i d_j / rho (VW), and the sum of v_xc rho (XC)
+template <bool VW, bool XC>
 __global__ void k_real_stress(long long n, const double *__restrict__ rho, const double *__restrict__ d,
                               double *__restrict__ partials) {
     __shared__ double sm[16];
@@ -906,19 +914,23 @@ __global__ void k_real_stress(long long n, const double *__restrict__ rho, const
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
          i += (long long)gridDim.x * blockDim.x) {
         const double r = rho[i];
-        const double g0 = d[i], g1 = d[n + i], g2 = d[2 * n + i];
-        const double ir = 1.0 / r;
-        acc[0] += g0 * g0 * ir;
-        acc[1] += g0 * g1 * ir;
-        acc[2] += g0 * g2 * ir;
-        acc[3] += g1 * g1 * ir;
-        acc[4] += g1 * g2 * ir;
-        acc[5] += g2 * g2 * ir;
-        double e, v;
-        pz_lda<double>(r < 1e-30 ? 1e-10 : cbrt(r), e, v);
-        acc[6] += v * r;
+        if constexpr (VW) {
+            const double g0 = d[i], g1 = d[n + i], g2 = d[2 * n + i];
+            const double ir = 1.0 / r;
+            acc[0] += g0 * g0 * ir;
+            acc[1] += g0 * g1 * ir;
+            acc[2] += g0 * g2 * ir;
+            acc[3] += g1 * g1 * ir;
+            acc[4] += g1 * g2 * ir;
+            acc[5] += g2 * g2 * ir;
+        }
+        if constexpr (XC) {
+            double e, v;
+            pz_lda<double>(r < 1e-30 ? 1e-10 : cbrt(r), e, v);
+            acc[6] += v * r;
+        }
     }
-    for (int k = 0; k < 7; ++k) {
+    for (int k = VW ? 0 : 6; k < (XC ? 7 : 6); ++k) {
         const double v = block_sum(acc[k], sm);
         if (threadIdx.x == 0) partials[(long long)blockIdx.x * 7 + k] = v;
     }
@@ -1074,13 +1086,20 @@ static void reduce_forces(const double *dpart, int na, int nb, const std::vector
         }
 }
 
-static std::vector<double> reduce_cols(const double *dpart, int nb, int K, hipStream_t s) {
-    std::vector<double> h((size_t)nb * K), out(K, 0.0);
-    OFDFT_HIP(hipMemcpyAsync(h.data(), dpart, h.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-    OFDFT_HIP(hipStreamSynchronize(s));
-    for (int b = 0; b < nb; ++b)
-        for (int k = 0; k < K; ++k) out[k] += h[(size_t)b * K + k];
-    return out;
+// column sums, reduced on the device and published to the pinned buffer
+static std::vector<double> reduce_cols(Plan &P, const double *dpart, int nb, int K, hipStream_t s) {
+    double *sums = P.scal + 64;  // K <= kMaxTerms
+    const std::vector<double> ones(K, 1.0);
+    reduce_final(dpart, nb, K, sums, ones.data(), s, nullptr, sums, P.pinned_dev, K);
+    stream_wait(s);
+    return std::vector<double>(P.pinned, P.pinned + K);
+}
+
+template <int TERM>
+static std::vector<double> stress_sums(Plan &P, const StressGIn &si, double *part, int nb, hipStream_t s) {
+    hipLaunchKernelGGL(k_stress_g<TERM>, dim3(nb), dim3(256), 0, s, P.Nc, geom_of(P), si, part);
+    OFDFT_HIP(hipGetLastError());
+    return reduce_cols(P, part, nb, 6, s);
 }
 
 static void sym_add(double *S, const double *v6, double scale) {
@@ -1147,7 +1166,7 @@ void pp_stress(Plan &P, const double *rho, int nspecies, const double *q0, const
     const long long nc = P.Nc;
     const int len = P.nr[0] + P.nr[1] + P.nzc;
     const int nb = 1024;
-    double *ws = fs_workspace(P, sizeof(double) * ((1 + nspecies) * nc * 2 + (size_t)nat * len * 2 + nb * 24));
+    double *ws = fs_workspace(P, sizeof(double) * ((1 + nspecies) * nc * 2 + (size_t)nat * len * 2 + nb * 7));
     double2 *rhoG = reinterpret_cast<double2 *>(ws);
     double2 *Ss = rhoG + nc;
     double2 *tab = Ss + (size_t)nspecies * nc;
@@ -1165,11 +1184,9 @@ void pp_stress(Plan &P, const double *rho, int nspecies, const double *q0, const
     si.Ss = Ss;
     si.nsp = nspecies;
     si.t = in.t;
-    hipLaunchKernelGGL(k_stress_g, dim3(nb), dim3(256), 0, s, nc, geom_of(P), si, part);
-    OFDFT_HIP(hipGetLastError());
-    const std::vector<double> v = reduce_cols(part, nb, 24, s);
+    const std::vector<double> v = stress_sums<ST_PP>(P, si, part, nb, s);
     for (int k = 0; k < 9; ++k) S[k] = 0.0;
-    sym_add(S, v.data() + 6, -2.0 / (P.volume * P.volume));
+    sym_add(S, v.data(), -2.0 / (P.volume * P.volume));
     for (int d = 0; d < 3; ++d) S[4 * d] -= energy / P.volume;
 }
 
@@ -1188,13 +1205,13 @@ void ewald_fs(Plan &P, int nat, const double *pos_cart, const double *pos_frac, 
     const int len = P.nr[0] + P.nr[1] + P.nzc;
     const int nb = 1024;
     double *ws = fs_workspace(P, sizeof(double) * (2 * nc * 2 + (size_t)nat * len * 2 +
-                                                   std::max((size_t)nat * kForceChunks * 3, (size_t)nb * 24) +
+                                                   std::max((size_t)nat * kForceChunks * 3, (size_t)nb * 7) +
                                                    (size_t)nat * 9));
     double2 *SZ = reinterpret_cast<double2 *>(ws);
     double2 *X = SZ + nc;
     double2 *tab = X + nc;
     double *part = reinterpret_cast<double *>(tab + (size_t)nat * len);
-    double *rpart = part + std::max((size_t)nat * kForceChunks * 3, (size_t)nb * 24);
+    double *rpart = part + std::max((size_t)nat * kForceChunks * 3, (size_t)nb * 7);
     phase_tables(P, nat, in.frac, tab, s);
     hipLaunchKernelGGL(k_strf_w, dim3(nblk(nc)), dim3(256), 0, s, nc, P.nr[0], P.nr[1], P.nzc, nat, tab, in.w, SZ);
     OFDFT_HIP(hipGetLastError());
@@ -1232,10 +1249,8 @@ void ewald_fs(Plan &P, int nat, const double *pos_cart, const double *pos_frac, 
         std::memset(&si, 0, sizeof(si));
         si.SZ = SZ;
         si.eta = ep.eta;
-        hipLaunchKernelGGL(k_stress_g, dim3(nb), dim3(256), 0, s, nc, g, si, part);
-        OFDFT_HIP(hipGetLastError());
-        const std::vector<double> v = reduce_cols(part, nb, 24, s);
-        sym_add(S, v.data() + 18, 4.0 * M_PI / (P.volume * P.volume));
+        const std::vector<double> v = stress_sums<ST_EW>(P, si, part, nb, s);
+        sym_add(S, v.data(), 4.0 * M_PI / (P.volume * P.volume));
         double qsum = 0.0;
         for (int a = 0; a < nat; ++a) qsum += charges[a];
         for (int d = 0; d < 3; ++d) S[4 * d] += qsum * qsum * 4.0 * M_PI * (1.0 / (4.0 * ep.eta * P.volume * P.volume) / 2.0);
@@ -1418,7 +1433,7 @@ void pp_stress_pme(Plan &P, const double *rho, int nspecies, const double *q0, c
                               {}, {}, s);
     const long long nc = P.Nc;
     const int nb = 1024;
-    double *ws = fs_workspace(P, sizeof(double) * ((1 + nspecies) * nc * 2 + P.N + nb * 24));
+    double *ws = fs_workspace(P, sizeof(double) * ((1 + nspecies) * nc * 2 + P.N + nb * 7));
     double2 *rhoG = reinterpret_cast<double2 *>(ws);
     double2 *Ss = rhoG + nc;
     double *Q = reinterpret_cast<double *>(Ss + (size_t)nspecies * nc);
@@ -1441,11 +1456,9 @@ void pp_stress_pme(Plan &P, const double *rho, int nspecies, const double *q0, c
     si.Ss = Ss;
     si.nsp = nspecies;
     si.t = in.t;
-    hipLaunchKernelGGL(k_stress_g, dim3(nb), dim3(256), 0, s, nc, g, si, part);
-    OFDFT_HIP(hipGetLastError());
-    const std::vector<double> v = reduce_cols(part, nb, 24, s);
+    const std::vector<double> v = stress_sums<ST_PP>(P, si, part, nb, s);
     for (int k = 0; k < 9; ++k) S[k] = 0.0;
-    sym_add(S, v.data() + 6, -2.0 / (P.volume * P.volume));
+    sym_add(S, v.data(), -2.0 / (P.volume * P.volume));
     for (int d = 0; d < 3; ++d) S[4 * d] -= energy / P.volume;
 }
 
@@ -1463,14 +1476,14 @@ void ewald_fs_pme(Plan &P, int nat, const double *pos_cart, const double *pos_fr
                               pos_frac, nullptr, w, alist, s);
     const long long nc = P.Nc;
     const int nb = 1024;
-    double *ws = fs_workspace(P, sizeof(double) * (2 * nc * 2 + P.N + (size_t)3 * nat + (size_t)nb * 24 +
+    double *ws = fs_workspace(P, sizeof(double) * (2 * nc * 2 + P.N + (size_t)3 * nat + (size_t)nb * 7 +
                                                    (size_t)nat * 9 + nat));
     double2 *SZ = reinterpret_cast<double2 *>(ws);
     double2 *X = SZ + nc;
     double *Q = reinterpret_cast<double *>(X + nc);
     double *Fd = Q + P.N;
     double *part = Fd + 3 * nat;
-    double *rpart = part + (size_t)nb * 24;
+    double *rpart = part + (size_t)nb * 7;
     double *qs = rpart + (size_t)nat * 9;
     const BTab bt = pme_tab(P, order);
     const GGeom g = geom_of(P);
@@ -1519,10 +1532,8 @@ void ewald_fs_pme(Plan &P, int nat, const double *pos_cart, const double *pos_fr
         std::memset(&si, 0, sizeof(si));
         si.SZ = SZ;
         si.eta = ep.eta;
-        hipLaunchKernelGGL(k_stress_g, dim3(nb), dim3(256), 0, s, nc, g, si, part);
-        OFDFT_HIP(hipGetLastError());
-        const std::vector<double> v = reduce_cols(part, nb, 24, s);
-        sym_add(S, v.data() + 18, 4.0 * M_PI / (P.volume * P.volume));
+        const std::vector<double> v = stress_sums<ST_EW>(P, si, part, nb, s);
+        sym_add(S, v.data(), 4.0 * M_PI / (P.volume * P.volume));
         double qsum = 0.0;
         for (int a = 0; a < nat; ++a) qsum += charges[a];
         for (int d = 0; d < 3; ++d)
@@ -1537,22 +1548,23 @@ void functional_stress(Plan &P, const double *rho, const double *energies, doubl
     const long long nc = P.Nc, n = P.N;
     const int nb = 1024;
     for (int k = 0; k < 45; ++k) out[k] = 0.0;
-    double *ws = fs_workspace(P, sizeof(double) * (3 * nc * 2 + (size_t)nb * 24));
+    double *ws = fs_workspace(P, sizeof(double) * (3 * nc * 2 + (size_t)nb * 7));
     double2 *rhoG = reinterpret_cast<double2 *>(ws);
     double2 *rA = rhoG + nc, *rB = rA + nc;
     double *part = reinterpret_cast<double *>(rB + nc);
-    fft_r2c<double>(P, rho, rhoG, 1, n, nc, P.dV, nullptr, nullptr, s);
+    const bool wt = (P.terms & OFDFT_TERM_WT) != 0;
+    // rho(G), which TF and XC do not need
+    if (wt || (P.terms & (OFDFT_TERM_HARTREE | OFDFT_TERM_VW)))
+        fft_r2c<double>(P, rho, rhoG, 1, n, nc, P.dV, nullptr, nullptr, s);
     const GGeom g = geom_of(P);
     const double V = P.volume;
     // rho0 = mean(rho) for the WT kernel (wt.py:79)
     double rho0 = 0.0;
-    {
-        double2 h0;
-        OFDFT_HIP(hipMemcpyAsync(&h0, rhoG, sizeof(h0), hipMemcpyDeviceToHost, s));
-        OFDFT_HIP(hipStreamSynchronize(s));
-        rho0 = h0.x / V;
+    if (wt) {
+        OFDFT_HIP(hipMemcpyAsync(P.pinned, rhoG, sizeof(double), hipMemcpyDeviceToHost, s));
+        stream_wait(s);
+        rho0 = P.pinned[0] / V;
     }
-    const bool wt = (P.terms & OFDFT_TERM_WT) != 0;
     StressGIn si;
     std::memset(&si, 0, sizeof(si));
     si.rhoG = (P.terms & OFDFT_TERM_HARTREE) ? rhoG : nullptr;
@@ -1575,34 +1587,42 @@ void functional_stress(Plan &P, const double *rho, const double *energies, doubl
         si.itkf = 1.0 / tkf;
         si.mu = P.y;
     }
-    if (si.rhoG || si.rA) {
-        hipLaunchKernelGGL(k_stress_g, dim3(nb), dim3(256), 0, s, nc, g, si, part);
-        OFDFT_HIP(hipGetLastError());
-        const std::vector<double> v = reduce_cols(part, nb, 24, s);
-        if (si.rhoG) {
-            sym_add(out + 36, v.data(), 8.0 * M_PI / (V * V));
-            for (int d = 0; d < 3; ++d) out[36 + 4 * d] -= energies[OFDFT_E_H] / V;
-        }
-        if (wt) {
-            const double a = P.alpha, b = P.beta;
-            sym_add(out + 18, v.data() + 12, M_PI * M_PI / (a * b * std::pow(rho0, a + b - 2) * tkf / 2.0) / (V * V));
-            for (int d = 0; d < 3; ++d) out[18 + 4 * d] -= 2.0 / 3.0 * energies[OFDFT_E_NL] / V;
-        }
+    if (si.rhoG) {
+        const std::vector<double> v = stress_sums<ST_H>(P, si, part, nb, s);
+        sym_add(out + 36, v.data(), 8.0 * M_PI / (V * V));
+        for (int d = 0; d < 3; ++d) out[36 + 4 * d] -= energies[OFDFT_E_H] / V;
+    }
+    if (wt) {
+        const std::vector<double> v = stress_sums<ST_WT>(P, si, part, nb, s);
+        const double a = P.alpha, b = P.beta;
+        sym_add(out + 18, v.data(), M_PI * M_PI / (a * b * std::pow(rho0, a + b - 2) * tkf / 2.0) / (V * V));
+        for (int d = 0; d < 3; ++d) out[18 + 4 * d] -= 2.0 / 3.0 * energies[OFDFT_E_NL] / V;
     }
     if (P.terms & OFDFT_TERM_TF)
         for (int d = 0; d < 3; ++d) out[4 * d] = -2.0 / 3.0 * energies[OFDFT_E_TF] / V;
-    if (P.terms & (OFDFT_TERM_VW | OFDFT_TERM_XC)) {
-        // gradients of rho: C2R of i G_d rho(G) into the work fields
-        double2 *gs = reinterpret_cast<double2 *>(P.spec);
+    const bool vw = (P.terms & OFDFT_TERM_VW) != 0, xc = (P.terms & OFDFT_TERM_XC) != 0;
+    if (vw || xc) {
         double *d = reinterpret_cast<double *>(P.work);
-        hipLaunchKernelGGL(k_grad_spectra, dim3(nblk(nc)), dim3(256), 0, s, nc, g, rhoG, gs);
+        if (vw) {  // gradients of rho: C2R of i G_d rho(G) into the work fields
+            double2 *gs = reinterpret_cast<double2 *>(P.spec);
+            hipLaunchKernelGGL(k_grad_spectra, dim3(nblk(nc)), dim3(256), 0, s, nc, g, rhoG, gs);
+            OFDFT_HIP(hipGetLastError());
+            fft_c2r<double>(P, gs, gs, d, 3, nc, nc, n, 1.0 / ((double)n * P.dV), s);
+        }
+        auto sums = [&](auto vc, auto xcc) {
+            hipLaunchKernelGGL((k_real_stress<decltype(vc)::value, decltype(xcc)::value>), dim3(nb), dim3(256), 0, s, n,
+                               rho, d, part);
+        };
+        if (vw && xc)
+            sums(std::true_type{}, std::true_type{});
+        else if (vw)
+            sums(std::true_type{}, std::false_type{});
+        else
+            sums(std::false_type{}, std::true_type{});
         OFDFT_HIP(hipGetLastError());
-        fft_c2r<double>(P, gs, gs, d, 3, nc, nc, n, 1.0 / ((double)n * P.dV), s);
-        hipLaunchKernelGGL(k_real_stress, dim3(nb), dim3(256), 0, s, n, rho, d, part);
-        OFDFT_HIP(hipGetLastError());
-        const std::vector<double> v = reduce_cols(part, nb, 7, s);
-        if (P.terms & OFDFT_TERM_VW) sym_add(out + 9, v.data(), -0.25 / V * P.dV * P.y);
-        if (P.terms & OFDFT_TERM_XC)
+        const std::vector<double> v = reduce_cols(P, part, nb, 7, s);  // columns of a term that is off are not read
+        if (vw) sym_add(out + 9, v.data(), -0.25 / V * P.dV * P.y);
+        if (xc)
             for (int d2 = 0; d2 < 3; ++d2) out[27 + 4 * d2] = (energies[OFDFT_E_XC] - v[6] * P.dV) / V;
     }
 }

@@ -141,3 +141,22 @@ def test_pme_forces_stress_vs_oracle():
     assert ew.PME
     _close(ew.forces, FO.ewald_forces_pme(og, oat), 1e-9)
     _close(ew.stress, FO.ewald_stress_pme(og, oat), 1e-9, 1e-13)
+
+
+@pytest.mark.parametrize("nr,full", [((20, 18, 16), False), ((9, 7, 5), False), ((10, 11, 12), True), ((1, 6, 8), False)])
+def test_functional_stress_of_one_term_and_of_all(nr, full):
+    """Each term's launches alone against all terms at once: the same sums,
+    FP64 rounding of sums over the grid."""
+    from dftpy_amd import DirectField, DirectGrid
+    from dftpy_amd.functional import Functional, functional_stress
+    grid = DirectGrid(np.array([[7.1, 0.2, 0.0], [0.3, 8.0, 0.1], [0.0, 0.5, 9.3]]), nr, full=full)
+    rho = DirectField(grid, data=0.02 + 0.01 * np.random.default_rng(3).random(nr))
+    terms = {"TF": Functional(type="KEDF", name="TF"), "VW": Functional(type="KEDF", name="vW"),
+             "NL": Functional(type="KEDF", name="WT-NL"), "XC": Functional(type="XC", name="LDA"),
+             "HARTREE": Functional(type="HARTREE")}
+    every = functional_stress(list(terms.values()), rho)
+    for k, f in terms.items():
+        one = functional_stress([f], rho)
+        assert np.abs(every[k]).max() > 0
+        _close(one[k], every[k], 1e-11, 1e-16)
+        assert all(np.all(one[o] == 0) for o in terms if o != k)
