@@ -138,16 +138,19 @@ static void gspace_apply(Plan &P, cpx<T> *spec, int ns, long long ncp, long long
 // Energy-only evaluation: the spectral terms as sums over the half spectrum,
 // E = sum_G w(kz) f(G) |F(G)|^2 / N (Parseval; w = 2 for the kz columns whose
 // mirror is not stored), with f the same multiplier the potential path
-// applies.  A flat grid stride over the stored points.  The
+// applies.  A flat grid stride over the stored points, all of a point's loads
+// at once and the WT function only where that term is on (160^3 FP64, Hartree
+// alone: 42 us in a loop over the slots with every kernel in it, 11 now; vW
+// and WT 45 / 20).  The
 // sums land in the k_post partial columns of vW (times y), WT and Hartree
 // (times 1/2), which k_post leaves at zero when it has no fields.
-template <typename T>
-__global__ void __launch_bounds__(256) k_gspace_energy(const cpx<T> *__restrict__ spec, int ns, GParams p,
+template <typename T, bool WT>
+__global__ void __launch_bounds__(256) k_gspace_energy(const cpx<T> *__restrict__ spec, GParams p,
                                                        double y, double *partials, const double *gate) {
     if (gate_off(gate)) return;
     __shared__ double sm[16];
     double tkf = 0.0, wtfac = 0.0;
-    if (p.s_wt >= 0) wt_consts(p, tkf, wtfac);
+    if constexpr (WT) wt_consts(p, tkf, wtfac);
     double acc_vw = 0.0, acc_wt = 0.0, acc_h = 0.0;
     // flat grid-stride over the stored half spectrum (every lane busy; rows
     // are shorter than a workgroup), 32-bit index arithmetic (the half
@@ -173,20 +176,21 @@ __global__ void __launch_bounds__(256) k_gspace_energy(const cpx<T> *__restrict_
         }
         const double w = (iz == 0 || ((p.nz & 1) == 0 && (int)iz == p.nz / 2)) ? 1.0 : 2.0;
         const long long e = (long long)row * p.pitch + iz;
-        for (int sl = 0; sl < ns; ++sl) {
-            const int kind = p.kind[sl];
+        // slot s_*: the point's loads go out together
+        auto square = [&](int sl) {
             const cpx<T> v = spec[sl * p.bs + e];
-            const double a2 = (double)v.x * (double)v.x + (double)v.y * (double)v.y;
+            return (double)v.x * (double)v.x + (double)v.y * (double)v.y;
+        };
+        const double a_vw = p.s_vw >= 0 ? square(p.s_vw) : 0.0, a_h = p.s_h >= 0 ? square(p.s_h) : 0.0;
+        const double a_wt = WT ? square(p.s_wt) : 0.0;
+        auto term = [&](int kind, double a2) {
             double f = kernel_val(p, kind, gg, g0, tkf, wtfac);
             if (nyq) f = 0.5 * (f + kernel_val(p, kind, gg2, g0, tkf, wtfac));
-            const double t = w * (f * p.scale) * a2;
-            if (kind == 0)
-                acc_vw += t;
-            else if (kind == 1)
-                acc_wt += t;
-            else
-                acc_h += t;
-        }
+            return w * (f * p.scale) * a2;
+        };
+        if (p.s_vw >= 0) acc_vw += term(0, a_vw);
+        if (p.s_h >= 0) acc_h += term(2, a_h);
+        if constexpr (WT) acc_wt += term(1, a_wt);
     }
     const double sums[3] = {block_sum(acc_vw, sm), block_sum(acc_wt, sm), block_sum(acc_h, sm)};
     if (threadIdx.x == 0) {
@@ -361,7 +365,10 @@ static void eval_energy(Plan &P, const T *rho, int ns, int s_vw, int s_wt, int s
     const int nb = launch_post<T>(s, rho, nullptr, vloc, nullptr, P.red, pp, P.gate);
     OFDFT_HIP(hipGetLastError());
     OFDFT_REQUIRE((long long)P.nr[0] * P.nr[1] * P.nzc < (1LL << 31), "energy pass: grid too large");
-    hipLaunchKernelGGL((k_gspace_energy<T>), dim3(nb), dim3(256), 0, s, spec, ns, gp, P.y, P.red, P.gate);
+    if (s_wt >= 0)
+        hipLaunchKernelGGL((k_gspace_energy<T, true>), dim3(nb), dim3(256), 0, s, spec, gp, P.y, P.red, P.gate);
+    else
+        hipLaunchKernelGGL((k_gspace_energy<T, false>), dim3(nb), dim3(256), 0, s, spec, gp, P.y, P.red, P.gate);
     OFDFT_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_energy_final, dim3(1), dim3(kFinalThreads), 0, s, P.red, nb, energies, P.dV, P.x, P.eion,
                        P.gate);
