@@ -1,4 +1,4 @@
-// Size-specialised FFT passes: every even length from 16 to 256 with primes up
+// Size-specialised FFT passes: every even length but 242 from 16 to 256 with primes up
 // to 13, which is what a grid chosen for an FFT has (kernels and launchers;
 // instantiated per precision and range of lengths in fft_fixed_f32_*.hip and
 // fft_fixed_f64_*.hip).
@@ -8,12 +8,16 @@
 // inputs from HBM into registers and the last one writes straight back (column
 // and complex row passes); between DFTs the elements cross LDS once.  Few
 // large radices (two, where they fit) mean few crossings and barriers, which
-// bound FP32; their registers cost occupancy, which bounds FP64: radices stop
-// at 20 and 13.  160^3, three spectra: FP32 x pass with the multiply 38 us with
-// 8 4 5, 26 with 10 16; FP64 column passes take 126 registers with 10 16 and 50
-// with 4 5 8 (33 us either way), the z C2R 37 and 33 us.  A length without
-// passes of its own takes the generic kernels (fft.hip): 52 x 78 x 104, FP64,
-// three spectra: y pass 29 us there, 4.5 here.
+// bound large FP32 fields; their registers and few threads bound FP64 and small
+// fields.  So: three radices up to 6 where a length has them in FP64, and in
+// FP32 up to 64 points; else two up to 20 in FP32, two or three up to 13 in
+// FP64.  An evaluation, us: 144^3 FP64 205 with 12 12, 189 with 4 6 6; 64^3 FP64
+// 59 with 8 8, 53 with 4 4 4; 64^3 FP32 45 and 43, 64 x 256 x 256 FP32 154 and
+// 152, 256 x 256 x 64 FP32 158 and 161.  160^3, three spectra: FP32 x pass with
+// the multiply 38 us with 8 4 5, 26 with 10 16; FP64 column passes take 126
+// registers with 10 16 and 50 with 4 5 8 (33 us either way), the z C2R 37 and
+// 33 us.  A length without passes of its own takes the generic kernels
+// (fft.hip): 52 x 78 x 104, FP64, three spectra: y pass 29 us there, 4.5 here.
 //
 // Column passes address a flattened set of pencils c in [0, ncols): base(c) =
 // (c / P) * Q + c % P, element stride S, which covers the y pass (P = nzc, Q =
@@ -65,8 +69,10 @@ constexpr Radices split(int n, int most) {
 
 // the DFTs of length N; REV: in the opposite order
 template <typename T, int N> struct SL {
+    static constexpr bool small = (sizeof(T) == 8 || N <= 64) && split(N, 6).n == 3;
     // FP64: 14 where 13 leaves only a split from 2 (98, 154, 182)
-    static constexpr int most = sizeof(T) == 4 ? 20 : (split(N, 13).r[0] > 2 ? 13 : 14);
+    static constexpr int large = sizeof(T) == 4 ? 20 : (split(N, 13).r[0] > 2 ? 13 : 14);
+    static constexpr int most = small ? 6 : large;
     static constexpr Radices s = split(N, most);
     static_assert(s.n >= 2, "length without a split");
     static constexpr int n = s.n;

@@ -146,7 +146,7 @@ def test_tile_variants_agree(shape, dtype):
         assert np.max(np.abs(p - tiles[0][2])) <= tol * np.max(np.abs(tiles[0][2]))
 
 
-# every length with size-specialised passes (16 to 256, even, primes up to 13),
+# every length with size-specialised passes (16 to 256, even, primes up to 13; not 242),
 # beside odd and generic lengths on the other axes
 def _smooth(n):
     for p in (2, 3, 5, 7, 11, 13):
