@@ -1616,9 +1616,11 @@ int ofdft_cnn_conv_mid(const int nr[3], int dil, int mode, const void *x, const 
         OFDFT_REQUIRE(mode == 0 || mode == 1, "mode must be 0 (forward) or 1 (backward-data)");
         OFDFT_REQUIRE(mode == 1 || bias, "forward mode needs the bias");
         OFDFT_REQUIRE(mode == 0 || (resid && mask), "backward mode needs resid and mask");
-        const uintptr_t al = reinterpret_cast<uintptr_t>(resid) | reinterpret_cast<uintptr_t>(out0);
+        // vector accesses of the training passes
+        const uintptr_t al = reinterpret_cast<uintptr_t>(resid) | reinterpret_cast<uintptr_t>(out0) |
+                             reinterpret_cast<uintptr_t>(mask) | reinterpret_cast<uintptr_t>(out1);
         if (g.nz >= RING_Z + RING_DMAX && g.ny % g.d == 0 && g.ny >= 4 * g.d && g.nx % g.d == 0 && g.d <= RING_DMAX &&
-            (mode == 0 || (al & 15) == 0)) {
+            ((mode == 0 && out1 == nullptr) || (al & 15) == 0)) {
             const dim3 grid((unsigned)(2 * rows_workgroups()));
 #define RING_LAUNCH(MD)                                                                                       \
     do {                                                                                                      \
