@@ -1335,7 +1335,7 @@ __global__ void __launch_bounds__(WM_THREADS) k_cnn_wgrad_mid(Geo g, const __bf1
         auto store = [&](const bf16x8(&st)[SLOTS], int k, bf16x8 *dst) {
             const bool g0 = tid < ZT * 4 && (base[0] < 0 || k + 1 >= k1);  // slot 0 has the g row
             const bf16x8 f = g0 ? bf16x8{} : st[0];
-            dst[tid] = f;
+            if (ZT > 32 || tid < nvec) dst[tid] = f;  // ZT = 32: 536 vectors with d = 1, 560 with d = 2
 #pragma unroll
             for (int s = 1; s < SLOTS; ++s)
                 if (tid + s * WM_THREADS < nvec) dst[tid + s * WM_THREADS] = st[s];

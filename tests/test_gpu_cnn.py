@@ -271,7 +271,11 @@ def test_spectral_loss_matches_numpy():
 
 @pytest.mark.parametrize("nr,d,nblk", [((12, 10, 14), 1, 512), ((9, 8, 33), 4, 7), ((40, 36, 40), 30, 64), ((5, 6, 96), 2, 1),
                                        ((40, 41, 70), 36, 512), ((70, 66, 128), 65, 512), ((12, 12, 48), 3, 512),
-                                       ((34, 33, 48), 31, 100), ((20, 20, 64), 8, 512), ((2, 2, 2), 1, 512)])
+                                       ((34, 33, 48), 31, 100), ((20, 20, 64), 8, 512), ((2, 2, 2), 1, 512),
+                                       # tiles of 32 whose stage has fewer vectors than the workgroup threads (d = 1
+                                       # and 2), many steps a workgroup
+                                       ((9, 40, 32), 1, 2), ((8, 37, 30), 2, 3), ((4, 66, 17), 2, 1),
+                                       ((12, 96, 32), 2, 8), ((12, 96, 24), 1, 16), ((6, 50, 32), 3, 4)])
 def test_weight_gradients_of_one_layer(nr, d, nblk):
     """Each layer's weight-gradient kernel against FP64 sums: FP32 sums of m
     products in a workgroup (m its share of the points, with the rounding of
