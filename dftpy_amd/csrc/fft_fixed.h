@@ -185,15 +185,24 @@ __global__ void __launch_bounds__((TILE *SL<T, N>::TP))
     });
 }
 
+// FP32 half grids form the G-space factors of the evaluation in FP32 at these
+// x lengths; every other FP32 pass with the multiply (full grids, the other
+// lengths, the kinetic operator) forms and applies them in FP64, as the
+// stand-alone multiply does.  An FP32 evaluation of 160^3: 167 us on the half
+// grid, 178 on the full one; with FP32 factors 167 and 169.
+constexpr bool f32_factors(int n) {
+    for (int m : {32, 48, 64, 72, 80, 96, 100, 120, 128, 144, 160, 192, 200, 240, 256})
+        if (n == m) return true;
+    return false;
+}
+
 // G-space factors of the elements e = j, j + TP, ... of one (iy, iz) column,
 // into fac[e * TILE], from |G|^2 of the column's fixed part plus fx * b1 in
-// the plan precision (the kinetic operator's in FP64).  Unrolled: around a
-// loop the compiler keeps the constants of the FP64 functions in 100
-// registers more.
-template <typename T, int N, int TILE>
+// the factors' precision T.  Unrolled: around a loop the compiler keeps the
+// constants of the FP64 functions in 100 registers more.
+template <typename T, int N, int TP, int TILE>
 __device__ __forceinline__ void xfactors(T *fac, const GParams &gp, int kind, int iy, int iz, int j, double tkf,
                                          double wtfac) {
-    constexpr int TP = SL<T, N>::TP;
     const int fy = ffreq(iy, gp.ny);
     // kinetic: the complex grid (fftfreq on all axes)
     const int fz = kind == 4 ? ffreq(iz, gp.nz) : (gp.full ? wrapf(iz, gp.nz) : iz);
@@ -201,41 +210,40 @@ __device__ __forceinline__ void xfactors(T *fac, const GParams &gp, int kind, in
     const bool yz0 = iy == 0 && iz == 0;
     const bool yznyq =
         gp.full && (((gp.ny & 1) == 0 && iy == gp.ny / 2) || ((gp.nz & 1) == 0 && iz == gp.nz / 2));
-    auto each = [&](auto one, auto &&val) {
-        using CT = decltype(one);
-        const CT bx = (CT)gp.B[0], by = (CT)gp.B[1], bz = (CT)gp.B[2], dx = (CT)cx, dy = (CT)cy, dz = (CT)cz;
+    auto each = [&](auto &&val) {
+        const T bx = (T)gp.B[0], by = (T)gp.B[1], bz = (T)gp.B[2], dx = (T)cx, dy = (T)cy, dz = (T)cz;
 #pragma unroll
         for (int i = 0; i < N / TP; ++i) {
             const int e = j + i * TP;
-            const CT fx = (CT)ffreq(e, N);
-            const CT gx = fx * bx + dx, gy = fx * by + dy, gz = fx * bz + dz;
-            CT f = val(gx * gx + gy * gy + gz * gz, yz0 && e == 0);
+            const T fx = (T)ffreq(e, N);
+            const T gx = fx * bx + dx, gy = fx * by + dy, gz = fx * bz + dz;
+            T f = val(gx * gx + gy * gy + gz * gz, yz0 && e == 0);
             // a Nyquist point of a full grid: the mean with the alias partner
             if (kind != 4 && (yznyq || (gp.full && 2 * e == N)))
-                f = (CT)0.5 * (f + val((CT)gsq(gp.B, wrapf(-ffreq(e, N), N), wrapf(-fy, gp.ny), wrapf(-fz, gp.nz)),
-                                       false));
-            fac[e * TILE] = (T)f;
+                f = (T)0.5 * (f + val((T)gsq(gp.B, wrapf(-ffreq(e, N), N), wrapf(-fy, gp.ny), wrapf(-fz, gp.nz)),
+                                      false));
+            fac[e * TILE] = f;
         }
     };
     const T sc = (T)gp.scale;
     if (kind == 0) {
         const T sig = (T)(gp.sigma * gp.sigma / 4.0);
-        each((T)1, [&](T gg, bool) {
+        each([&](T gg, bool) {
             T f = (T)0.5 * gg * sc;
             if (gp.sigma > 0) f *= exp(-gg * sig);
             return f;
         });
     } else if (kind == 1) {
         const T itkf = (T)(1.0 / tkf), wsc = (T)(wtfac * gp.scale), lb = (T)gp.lbda;
-        each((T)1, [&](T gg, bool) { return lindhard_t<T>(fm::sqrt_n(gg) * itkf, lb, (T)1) * wsc; });
+        each([&](T gg, bool) { return lindhard_t<T>(fm::sqrt_n(gg) * itkf, lb, (T)1) * wsc; });
     } else if (kind == 2) {
-        each((T)1, [&](T gg, bool g0) { return g0 ? (T)0 : gdiv<T>((T)(4.0 * M_PI) * sc, gg); });
+        each([&](T gg, bool g0) { return g0 ? (T)0 : gdiv<T>((T)(4.0 * M_PI) * sc, gg); });
     } else if (kind == 3) {
-        each((T)1, [&](T gg, bool) { return (T)(radial_table(gp, sqrt((double)gg)) * gp.scale); });
+        each([&](T gg, bool) { return (T)(radial_table(gp, sqrt((double)gg)) * gp.scale); });
     } else {
         // kinetic: 1/2 G^2 exp(-G^2 sigma^2 / 2)
-        const double s2 = gp.sigma * gp.sigma / 2.0;
-        each(1.0, [&](double gg, bool) { return 0.5 * gg * exp(-gg * s2) * gp.scale; });
+        const T s2 = (T)(gp.sigma * gp.sigma / 2.0);
+        each([&](T gg, bool) { return (T)0.5 * gg * exp(-gg * s2) * sc; });
     }
 }
 
@@ -245,8 +253,8 @@ __device__ __forceinline__ void xfactors(T *fac, const GParams &gp, int kind, in
 // very elements a thread holds after the forward transform, so the multiply
 // works on registers.  All threads make the factors (fewer hold spectrum
 // elements after a large last radix) while the column loads are on their way,
-// and hand them over in LDS.
-template <typename T, int N, int TILE>
+// and hand them over in LDS.  FT: the precision of the factors and the product.
+template <typename T, typename FT, int N, int TILE>
 __global__ void __launch_bounds__((TILE *SL<T, N>::TP))
     k_xfused_f(cpx<T> *data, long long bs, unsigned ncols, unsigned pitch, unsigned vp,
                const cpx<T> *__restrict__ twg, GParams gp, const double *live, const double *gate) {
@@ -255,7 +263,7 @@ __global__ void __launch_bounds__((TILE *SL<T, N>::TP))
     constexpr int R = SL<T, N>::first, RL = SL<T, N>::last, TP = SL<T, N>::TP;
     __shared__ C tw[N];
     __shared__ C buf[N * TILE];
-    __shared__ T fac[N * TILE];
+    __shared__ FT fac[N * TILE];
     const int pen = threadIdx.x % TILE;
     const int j = threadIdx.x / TILE;
     const unsigned c = blockIdx.x * TILE + pen;
@@ -270,7 +278,7 @@ __global__ void __launch_bounds__((TILE *SL<T, N>::TP))
     const int kind = gp.kind[gp.c2c ? 0 : blockIdx.y];
     double tkf = 1.0, wtfac = 1.0;
     if (kind == 1) wt_consts(gp, tkf, wtfac);
-    if (valid) xfactors<T, N, TILE>(fac + pen, gp, kind, (int)iy, (int)iz, j, tkf, wtfac);
+    if (valid) xfactors<FT, N, TP, TILE>(fac + pen, gp, kind, (int)iy, (int)iz, j, tkf, wtfac);
     C u[RL];
     dfts<T, N, ColMap<TILE>, false, false, 0, 1>(buf, tw, v, [&](auto &, auto &w) {
 #pragma unroll
@@ -280,9 +288,9 @@ __global__ void __launch_bounds__((TILE *SL<T, N>::TP))
     if (j < N / RL) {
 #pragma unroll
         for (int r = 0; r < RL; ++r) {
-            const T f = fac[(j + r * (N / RL)) * TILE + pen];
-            u[r].x *= f;
-            u[r].y *= f;
+            const FT f = fac[(j + r * (N / RL)) * TILE + pen];
+            u[r].x = (T)(u[r].x * f);
+            u[r].y = (T)(u[r].y * f);
         }
     }
     __syncthreads();
@@ -724,11 +732,19 @@ template <typename T, int N> struct Launch {
     }
     static void xfused(int var, C *data, int batch, long long bs, long long ncols, long long pitch, long long vp,
                        const C *tw, const GParams &gp, const double *live, hipStream_t s, const double *gate) {
+        if constexpr (sizeof(T) == 4 && f32_factors(N)) {
+            if (!gp.full && !gp.c2c) return xfused_ft<T>(var, data, batch, bs, ncols, pitch, vp, tw, gp, live, s, gate);
+        }
+        xfused_ft<double>(var, data, batch, bs, ncols, pitch, vp, tw, gp, live, s, gate);
+    }
+    template <typename FT>
+    static void xfused_ft(int var, C *data, int batch, long long bs, long long ncols, long long pitch, long long vp,
+                          const C *tw, const GParams &gp, const double *live, hipStream_t s, const double *gate) {
 #define CALL(V)                                                                                                        \
     {                                                                                                                  \
         constexpr int TILE = col_tile_v<T, N, V>();                                                                       \
         const dim3 grid((unsigned)((ncols + TILE - 1) / TILE), (unsigned)batch);                                       \
-        hipLaunchKernelGGL((k_xfused_f<T, N, TILE>), grid, dim3(TILE * TP), 0, s, data, bs, (unsigned)ncols,           \
+        hipLaunchKernelGGL((k_xfused_f<T, FT, N, TILE>), grid, dim3(TILE * TP), 0, s, data, bs, (unsigned)ncols,           \
                            (unsigned)pitch, (unsigned)vp, tw, gp, live, gate);                                         \
     }
         OFDFT_VARIANT(var, CALL)

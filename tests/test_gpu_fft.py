@@ -240,3 +240,49 @@ def test_cn_batch_on_fixed_and_generic_passes(shape, dtype, maxiter):
         diff = float((y1[r] - y0[r]).abs().square().sum().sqrt())
         size = float(y0[r].abs().square().sum().sqrt())
         assert diff <= (2 * cn.last_info[r]["atol"] if s0[r] == 0 else 0.0) + 100 * eps * size
+
+
+@pytest.mark.parametrize("nx,full", [(28, False), (52, False), (104, False), (36, True), (32, True), (160, True)])
+def test_f32_multiply_keeps_f64_factors(nx, full):
+    """FP32 grids whose G-space factors are FP64 ones (full grids, and half
+    grids of the later x lengths), on a density whose transforms are exact: 1
+    + cos(G.r) of period 4 along y and z and constant along x.  The Hartree
+    potential is then 4 pi / G^2 cos(G.r) with the one rounding of the
+    multiply, 2^-24, and what the x transforms of a constant leave, which the
+    mean over x takes to a quarter of it."""
+    from dftpy_amd import DirectField, DirectGrid
+    from dftpy_amd.functional import Functional, TotalFunctional
+    rng = np.random.default_rng(1)
+    ev = TotalFunctional(H=Functional(type="HARTREE"))
+    yz = (np.arange(4)[:, None] + np.arange(4)[None, :]) % 4
+    cos = np.array([1.0, 0.0, -1.0, 0.0])[yz]
+    for _ in range(24):
+        lat = np.diag([7.1, 8.0, 9.3]) + 0.4 * rng.standard_normal((3, 3))
+        g = DirectGrid(lat, (nx, 4, 4), full=full, dtype=torch.float32)
+        v = ev(DirectField(g, data=np.broadcast_to(1.0 + cos, (nx, 4, 4)).copy())).potential.data
+        v = v.double().mean(0).cpu().numpy()
+        B = 2.0 * np.pi * np.linalg.inv(lat).T
+        exact = 4.0 * np.pi / np.sum((B[1] + B[2]) ** 2)
+        assert np.abs(v - exact * cos).max() <= 1.25 * 2.0 ** -24 * exact
+
+
+@pytest.mark.parametrize("nx", [26, 50, 52])
+def test_f32_kinetic_keeps_f64_factors(nx):
+    """The kinetic operator of FP32 Crank-Nicolson steps on a plane wave of
+    period 4 along z, exact but for the rounding of the multiply as above:
+    after no iteration the workspace holds b = psi - i dt/2 G^2/2 psi."""
+    from dftpy_amd import DirectGrid
+    from dftpy_amd.td import CrankNicholsonBatch
+    rng = np.random.default_rng(1)
+    psi = torch.tensor([1, 1j, -1, -1j], dtype=torch.complex64).repeat(nx, 1, 4)[None].cuda().contiguous()
+    v = torch.zeros((1, nx, 1, 16), device="cuda")
+    for _ in range(24):
+        lat = np.diag([71.0, 8.0, 9.3]) + 0.4 * rng.standard_normal((3, 3))  # small G_x: it amplifies what x leaves
+        g = DirectGrid(lat, (nx, 1, 16), full=True, dtype=torch.float32)
+        cn = CrankNicholsonBatch(4.0, maxiter=0, sigma=0.0)
+        cn(g, psi, v)
+        n = 16 * nx
+        b = next(iter(cn._work.values())).view(torch.complex64)[n:2 * n].view(nx, 16)[:, ::4]
+        exact = np.sum((4 * 2.0 * np.pi * np.linalg.inv(lat).T[2]) ** 2)
+        err = np.abs(-b.imag.double().mean(0).cpu().numpy() - exact).max()
+        assert err <= 1.25 * 2.0 ** -24 * exact
