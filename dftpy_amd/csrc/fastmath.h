@@ -1,5 +1,8 @@
 // Transcendental functions of the point-wise and G-space kernels, by
-// precision.  FP64 keeps the correctly rounded library functions.  FP32 (the
+// precision.  FP64 has the library's logarithm, exponential and general power;
+// its roots and quotients are those at the end of this file, whose largest
+// errors are stated there (the library's division and square root: half an
+// ulp; 1 / sqrt 1.5).  FP32 (the
 // FP32-bulk pipeline, whose accuracy is set by single-precision storage and
 // FFTs anyway) uses the hardware approximations v_sqrt_f32, v_rsq_f32,
 // v_rcp_f32, v_log_f32 (log2) and v_exp_f32 (exp2), each within about 1 ulp,
@@ -57,37 +60,41 @@ template <> __device__ __forceinline__ float cbrt<float>(float x) {
     return x > 0.0f ? z : 0.0f;
 }
 
-// a^(-1/6) for finite a > 0 in FP64: one third-order step from the FP32
-// hardware log2 and exp2 of a scaled by a power of 2^6 into [1/2, 32), so
-// every exponent (denormals too) has the same seed.  Below 1 ulp; about 20
-// instructions, where the library's cbrt, sqrt and division, whose results
-// the powers of it give, take ten times that.
-__device__ __forceinline__ double inv_sixth_root(double a) {
-    const int e = __builtin_amdgcn_frexp_exp(a);
-    const int q = (e + 1536) / 6 - 256;  // floor(e / 6)
-    const double m = __builtin_amdgcn_ldexp(__builtin_amdgcn_frexp_mant(a), e - 6 * q);
-    double s = (double)__builtin_amdgcn_exp2f(__builtin_amdgcn_logf((float)m) * (-1.0f / 6.0f));
-    const double s3 = s * s * s;
-    const double h = __builtin_fma(-m, s3 * s3, 1.0);
-    s = __builtin_fma(s * h, __builtin_fma(h, 7.0 / 72.0, 1.0 / 6.0), s);
-    return __builtin_amdgcn_ldexp(s, -q);
-}
-// square root, reciprocal square root and cube root of a > 0 from s =
-// a^(-1/6), each with one correction
-__device__ __forceinline__ double sqrt_s(double a, double s) {
-    const double s3 = s * s * s, y = a * s3;
-    return __builtin_fma(__builtin_fma(-y, y, a), 0.5 * s3, y);
-}
-__device__ __forceinline__ double rsq_s(double a, double s) {
-    const double y = s * s * s;
-    return __builtin_fma(__builtin_fma(-a * y, y, 1.0), 0.5 * y, y);
-}
-__device__ __forceinline__ double cbrt_s(double a, double s) {
-    const double s2 = s * s, s4 = s2 * s2, y = a * s4;
-    return __builtin_fma(__builtin_fma(-y * y, y, a), s4 * (1.0 / 3.0), y);
-}
-// square root of x >= 0 in FP64 for normal x or 0: a Goldschmidt step on the
-// hardware reciprocal root and a correction
+// Roots of one finite a > 0 in FP64, denormals too: a = m 2^(6 q) with m in
+// [1/2, 32), and s = m^(-1/6) by one third-order step from the FP32 hardware
+// log2 and exp2.  Its powers, each with one correction, give the roots, about
+// 20 instructions in all, where the library's cbrt, sqrt and division take ten
+// times that.  Largest errors in ulps: a^(-1/6) 0.9, square root 0.5,
+// reciprocal square root 1.0, cube root 0.75.
+struct SixthRoot {
+    double m, s;
+    int q;
+    __device__ __forceinline__ explicit SixthRoot(double a) {
+        const int e = __builtin_amdgcn_frexp_exp(a);
+        q = (e + 1536) / 6 - 256;  // floor(e / 6)
+        m = __builtin_amdgcn_ldexp(__builtin_amdgcn_frexp_mant(a), e - 6 * q);
+        s = (double)__builtin_amdgcn_exp2f(__builtin_amdgcn_logf((float)m) * (-1.0f / 6.0f));
+        const double s3 = s * s * s;
+        const double h = __builtin_fma(-m, s3 * s3, 1.0);
+        s = __builtin_fma(s * h, __builtin_fma(h, 7.0 / 72.0, 1.0 / 6.0), s);
+    }
+    __device__ __forceinline__ double inv_sixth() const { return __builtin_amdgcn_ldexp(s, -q); }
+    __device__ __forceinline__ double sqrt() const {
+        const double s3 = s * s * s, y = m * s3;
+        return __builtin_amdgcn_ldexp(__builtin_fma(__builtin_fma(-y, y, m), 0.5 * s3, y), 3 * q);
+    }
+    __device__ __forceinline__ double rsq() const {
+        const double y = s * s * s;
+        return __builtin_amdgcn_ldexp(__builtin_fma(__builtin_fma(-m * y, y, 1.0), 0.5 * y, y), -3 * q);
+    }
+    __device__ __forceinline__ double cbrt() const {
+        const double s2 = s * s, s4 = s2 * s2, y = m * s4;
+        return __builtin_amdgcn_ldexp(__builtin_fma(__builtin_fma(-y * y, y, m), s4 * (1.0 / 3.0), y), 2 * q);
+    }
+};
+// square root in FP64 of normal numbers, zeros, infinity and NaN (negative:
+// NaN), within half an ulp: a Goldschmidt step on the hardware reciprocal root
+// and a correction
 __device__ __forceinline__ double sqrt_n(double x) {
     const double y = __builtin_amdgcn_rsq(x);
     double g = x * y, h = 0.5 * y;
@@ -95,17 +102,18 @@ __device__ __forceinline__ double sqrt_n(double x) {
     g = __builtin_fma(g, r, g);
     h = __builtin_fma(h, r, h);
     g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
-    return x > 0.0 ? g : x;
+    return x == 0.0 || x == (double)INFINITY ? x : g;
 }
 __device__ __forceinline__ float sqrt_n(float x) { return sqrt(x); }
-// a / b in FP64 for normal b and quotient: two Newton steps on the hardware
+// a / b in FP64 within half an ulp for |b| and the quotient within 2^+-1000,
+// zeros, infinities and NaN as the division: two Newton steps on the hardware
 // reciprocal and a correction of the quotient
 __device__ __forceinline__ double div_n(double a, double b) {
     double r = __builtin_amdgcn_rcp(b);
     r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
     r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
     const double q = a * r;
-    return __builtin_fma(__builtin_fma(-b, q, a), r, q);
+    return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), r, q), b, a);
 }
 
 }  // namespace fm

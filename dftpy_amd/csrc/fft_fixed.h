@@ -341,9 +341,9 @@ __device__ __forceinline__ void prologue_t(const int (&code)[NF], T x, T beta, T
         rc = base < (T)1e-30 ? (T)1e-30 : base;
         if constexpr (std::is_same<T, double>::value) {
             const bool fin = rc < (double)INFINITY;
-            const double a = base > 0.0 ? base : 1e-30, s = fm::inv_sixth_root(a);
-            sq = fin ? fm::sqrt_s(a, s) : rc;
-            if constexpr (B56) cb = base < 1e-30 ? 1e-10 : (fin ? fm::cbrt_s(a, s) : rc);
+            const fm::SixthRoot s(base > 0.0 ? base : 1e-30);
+            sq = fin ? s.sqrt() : rc;
+            if constexpr (B56) cb = base < 1e-30 ? 1e-10 : (fin ? s.cbrt() : rc);
         } else {
             sq = fm::sqrt_c(base > (T)0 ? base : (T)1e-30);
             if constexpr (B56) cb = fm::cbrt(rc);

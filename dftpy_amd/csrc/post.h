@@ -31,16 +31,14 @@ constexpr double PZ_G = -0.1423, PZ_B1 = 1.0529, PZ_B2 = 0.3334;
 constexpr double kCtf = 2.871234000188191, kCbrt34Pi = 0.6203504908994001, kCbrt3Pi = 0.9847450218426965;
 
 // Reciprocal and reciprocal square root: the hardware approximations (about
-// 1 ulp) for the FP32-bulk pipeline; in FP64 the reciprocal of a normal
-// number by Newton steps (within an ulp, without the library division's
-// scaling) and the library root.
+// 1 ulp) for the FP32-bulk pipeline; in FP64 the reciprocal by Newton steps
+// (without the library division's scaling) and the library root.
 template <typename CT> __device__ __forceinline__ CT rcp_p(CT x) { return fm::rcp(x); }
 template <> __device__ __forceinline__ double rcp_p<double>(double x) { return fm::div_n(1.0, x); }
 template <typename CT> __device__ __forceinline__ CT rsq_p(CT x) { return fm::rsq(x); }
 
 // The powers of the density at a point that its terms use.  FP64 takes them
-// all from one inverse sixth root; the corrected square and cube roots are
-// within an ulp, as the library's.
+// all from one inverse sixth root (fastmath.h).
 template <typename CT> struct RhoPowers {
     CT cr;     // cbrt(rho)
     CT isq;    // 1 / sqrt(rho > 0 ? rho : 1e-30)
@@ -56,10 +54,11 @@ template <typename CT> __device__ __forceinline__ RhoPowers<CT> rho_powers(CT r)
 }
 template <> __device__ __forceinline__ RhoPowers<double> rho_powers(double r) {
     RhoPowers<double> w;
-    const double a = fabs(r), s = fm::inv_sixth_root(a);
-    w.cr = (a > 0.0 && a < (double)INFINITY) ? copysign(fm::cbrt_s(a, s), r) : r;
-    w.isq = r <= 0.0 ? 1e15 : (a < (double)INFINITY ? fm::rsq_s(a, s) : (a == a ? 0.0 : a));
-    w.rb_rc = r < 1e-30 ? 1e5 : s;
+    const double a = fabs(r);
+    const fm::SixthRoot s(a);
+    w.cr = (a > 0.0 && a < (double)INFINITY) ? copysign(s.cbrt(), r) : r;
+    w.isq = r <= 0.0 ? 1e15 : (a < (double)INFINITY ? s.rsq() : (a == a ? 0.0 : a));
+    w.rb_rc = r < 1e-30 ? 1e5 : s.inv_sixth();
     return w;
 }
 

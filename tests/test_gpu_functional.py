@@ -389,3 +389,40 @@ def test_vw_gaussian_sigma_vs_oracle():
         assert np.max(np.abs(out.potential.numpy() - v_ref)) < 1e-10 * np.max(np.abs(v_ref))
     e0 = Functional(type="KEDF", name="vW")(DirectField(g, data=rho)).energy
     assert abs(e0 - OF.vw(rho, og)[0]) < 1e-12 * abs(e0) and abs(e0 - out.energy) > 1e-6
+
+
+@pytest.mark.parametrize("nr", [(4, 8, 16), (3, 5, 7)])
+def test_point_terms_over_the_range_of_densities(nr):
+    """TF and LDA potentials at densities of every size, denormal ones, zero
+    and infinity among them, against 64-bit mantissas.  TF: 2 x 0.75 ulp of the
+    cube root and three roundings; LDA: terms of one sign, about a dozen
+    roundings, and the constants' own."""
+    from dftpy_amd import DirectField, DirectGrid
+    from dftpy_amd.functional import Functional, TotalFunctional
+    n = int(np.prod(nr))
+    r = 10.0 ** np.linspace(-320.0, 40.0, n)
+    r[:3] = 0.0, 5e-324, 1e-310
+    grid = DirectGrid(np.diag([4.0, 5.0, 6.0]), nr, full=False)
+    rho = DirectField(grid, data=r.reshape(nr))
+    ld = np.longdouble
+
+    def pot(ev):
+        return ev.compute(rho, calcType=["V"]).potential.numpy().reshape(-1).astype(ld)
+
+    def close(v, ref, ulps):
+        assert np.all(np.abs(v - ref) <= ulps * 2.0 ** -53 * np.abs(ref) + 1e-320)
+
+    pi = ld("3.14159265358979323846264338327950288")
+    c = np.cbrt(r.astype(ld))
+    close(pot(TotalFunctional(TF=Functional(type="KEDF", name="TF"))), pi ** 2 / 2 * np.cbrt(3 / pi) ** 2 * c * c, 10)
+    c = np.where(c < ld(1e-30), ld(1e-30), c)
+    rs = np.cbrt(3 / (4 * pi)) / c
+    A, B, C, D, G, B1, B2 = (float(x) for x in (0.0311, -0.048, 0.0020, -0.0116, -0.1423, 1.0529, 0.3334))
+    sr, lr = np.sqrt(rs), np.log(rs)
+    high = lr * (A + 2 * C / 3 * rs) + B - A / 3 + (2 * D - C) / 3 * rs
+    low = G * (1 + ld(7) / 6 * B1 * sr + ld(4) / 3 * B2 * rs) / (1 + B1 * sr + B2 * rs) ** 2
+    v = pot(TotalFunctional(XC=Functional(type="XC", name="LDA")))
+    close(v, -np.cbrt(3 / pi) * c + np.where(rs < 1, high, low), 24)
+    rho[:] = np.inf
+    assert bool((TotalFunctional(TF=Functional(type="KEDF", name="TF")).compute(rho, calcType=["V"]).potential.data
+                 == np.inf).all())
