@@ -112,7 +112,9 @@ __device__ __forceinline__ T prologue(int code, T x, double beta, bool b56, cons
 // `tile` adjacent columns.  in may equal out.
 template <typename T, bool INV>
 __global__ void k_cols(const cpx<T> *__restrict__ in, cpx<T> *__restrict__ out, long long bs, int n,
-                       long long M, int tiles, AxisPlan ap, const cpx<T> *__restrict__ twg, int tile, T scale) {
+                       long long M, int tiles, AxisPlan ap, const cpx<T> *__restrict__ twg, int tile, T scale,
+                       const double *live) {
+    if (run_off(live, blockIdx.y)) return;
     using C = cpx<T>;
     extern __shared__ unsigned char smem_raw[];
     C *tw = reinterpret_cast<C *>(smem_raw);
@@ -265,7 +267,8 @@ __global__ void k_rows_c2r(const cpx<T> *__restrict__ in, T *__restrict__ out, l
 // Rows pass, complex -> complex on contiguous rows of length n.
 template <typename T, bool INV>
 __global__ void k_rows_c2c(const cpx<T> *__restrict__ in, cpx<T> *__restrict__ out, long long bs, long long nrows,
-                           int n, AxisPlan ap, const cpx<T> *__restrict__ twg, int rows, T scale) {
+                           int n, AxisPlan ap, const cpx<T> *__restrict__ twg, int rows, T scale, const double *live) {
+    if (run_off(live, blockIdx.y)) return;
     using C = cpx<T>;
     extern __shared__ unsigned char smem_raw[];
     C *tw = reinterpret_cast<C *>(smem_raw);
@@ -453,7 +456,7 @@ void fft_cols(Plan &P, int axis, bool full_grid, bool inverse, const cpx<T> *in,
         return;
     }
     OFDFT_REQUIRE(pitch == zlen, "generic column pass needs an unpadded layout");
-    OFDFT_REQUIRE(P.gate == nullptr && live == nullptr, "gated launch of a generic FFT pass");
+    OFDFT_REQUIRE(P.gate == nullptr, "gated launch of a generic FFT pass");
     long long M, outer;
     PassShape sh;
     if (axis == 1) {
@@ -470,10 +473,10 @@ void fft_cols(Plan &P, int axis, bool full_grid, bool inverse, const cpx<T> *in,
     const cpx<T> *tw = reinterpret_cast<const cpx<T> *>(P.tw[axis]);
     if (inverse)
         hipLaunchKernelGGL((k_cols<T, true>), grid, dim3(sh.threads), sh.lds, s, in, out, bs, n, M, tiles,
-                           P.ax[axis], tw, sh.tile, (T)scale);
+                           P.ax[axis], tw, sh.tile, (T)scale, live);
     else
         hipLaunchKernelGGL((k_cols<T, false>), grid, dim3(sh.threads), sh.lds, s, in, out, bs, n, M, tiles,
-                           P.ax[axis], tw, sh.tile, (T)scale);
+                           P.ax[axis], tw, sh.tile, (T)scale, live);
     OFDFT_HIP(hipGetLastError());
 }
 
@@ -544,7 +547,7 @@ void fft_c2r(Plan &P, const cpx<T> *in, cpx<T> *tmp, T *out, int batch, long lon
 
 template <typename T>
 void fft_c2c(Plan &P, const cpx<T> *in, cpx<T> *out, bool inverse, int batch, long long bs, double scale,
-             hipStream_t s) {
+             hipStream_t s, const double *live) {
     const long long nrows = (long long)P.nr[0] * P.nr[1];
     const PassShape sh = P.rows_c2c;
     dim3 grid((unsigned)((nrows + sh.tile - 1) / sh.tile), (unsigned)batch);
@@ -554,19 +557,19 @@ void fft_c2c(Plan &P, const cpx<T> *in, cpx<T> *out, bool inverse, int batch, lo
     OFDFT_REQUIRE(P.gate == nullptr, "gated launch of a generic FFT pass");
     if (const SizeOps<T> *ops = axis_ops<T>(P, 2)) {
         if (inverse)
-            ops->rows_inv(0, in, out, batch, bs, nrows, tw, sz, ApplyArgs<T>{}, 0, nullptr, s, nullptr);
+            ops->rows_inv(0, in, out, batch, bs, nrows, tw, sz, ApplyArgs<T>{}, 0, live, s, nullptr);
         else
-            ops->rows_fwd(in, out, batch, bs, nrows, tw, sz, nullptr, nullptr, s, nullptr);
+            ops->rows_fwd(in, out, batch, bs, nrows, tw, sz, nullptr, live, s, nullptr);
     } else if (inverse)
         hipLaunchKernelGGL((k_rows_c2c<T, true>), grid, dim3(sh.threads), sh.lds, s, in, out, bs, nrows, P.nr[2],
-                           P.ax[2], tw, sh.tile, sz);
+                           P.ax[2], tw, sh.tile, sz, live);
     else
         hipLaunchKernelGGL((k_rows_c2c<T, false>), grid, dim3(sh.threads), sh.lds, s, in, out, bs, nrows, P.nr[2],
-                           P.ax[2], tw, sh.tile, sz);
+                           P.ax[2], tw, sh.tile, sz, live);
     OFDFT_HIP(hipGetLastError());
     if (last_z) return;
-    fft_cols<T>(P, 1, true, inverse, out, out, batch, bs, 1.0, s, P.nr[2]);
-    fft_cols<T>(P, 0, true, inverse, out, out, batch, bs, scale, s, P.nr[2]);
+    fft_cols<T>(P, 1, true, inverse, out, out, batch, bs, 1.0, s, P.nr[2], live);
+    fft_cols<T>(P, 0, true, inverse, out, out, batch, bs, scale, s, P.nr[2], live);
 }
 
 template <typename T>
@@ -705,7 +708,8 @@ template void bench_rows_c2r<double>(Plan &, const double2 *, double *, int, hip
                              double *, hipStream_t, long long, bool);                                               \
     template void fft_c2r<T>(Plan &, const cpx<T> *, cpx<T> *, T *, int, long long, long long, long long,      \
                              double, hipStream_t, long long, bool);                                                 \
-    template void fft_c2c<T>(Plan &, const cpx<T> *, cpx<T> *, bool, int, long long, double, hipStream_t);
+    template void fft_c2c<T>(Plan &, const cpx<T> *, cpx<T> *, bool, int, long long, double, hipStream_t,        \
+                             const double *);
 INST(float)
 INST(double)
 #undef INST

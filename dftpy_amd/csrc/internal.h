@@ -193,9 +193,10 @@ void fft_c2r(Plan &P, const cpx<T> *in, cpx<T> *tmp, T *out, int batch, long lon
 bool fixed_size(int n);
 template <typename T>
 void fft_c2c(Plan &P, const cpx<T> *in, cpx<T> *out, bool inverse, int batch, long long bs, double scale,
-             hipStream_t s);
+             hipStream_t s, const double *live = nullptr);
 // the x/y passes alone (in place allowed), for fused pipelines; batch entries
-// whose element of live (device memory, null: none) is 0 are left out
+// whose element of live (device memory, null: none) is 0 are left out (fft_c2c
+// likewise)
 template <typename T>
 void fft_cols(Plan &P, int axis, bool full_grid, bool inverse, const cpx<T> *in, cpx<T> *out, int batch,
               long long bs, double scale, hipStream_t s, long long pitch = 0, const double *live = nullptr);

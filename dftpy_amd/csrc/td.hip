@@ -32,13 +32,14 @@ template <int K> __device__ __forceinline__ void td_partials(double *acc, double
 __device__ __forceinline__ int ffreq_td(int i, int n) { return i <= (n - 1) / 2 ? i : i - n; }
 
 // spec *= 1/2 G^2 exp(-G^2 sigma^2 / 2) / N (full grid, fftfreq on all axes);
-// element j of the stacked runs has grid index j % n
+// stacked runs, blockIdx.y = run
 template <typename T>
-__global__ void k_td_gmul_b(cpx<T> *spec, long long tot, long long n, int nx, int ny, int nz, double B0, double B1,
-                            double B2, double B3, double B4, double B5, double B6, double B7, double B8, double sigma,
-                            double scale) {
-    GRID_LOOP(j, tot) {
-        const long long i = j % n;
+__global__ void k_td_gmul_b(cpx<T> *spec, long long n, int nx, int ny, int nz, double B0, double B1, double B2,
+                            double B3, double B4, double B5, double B6, double B7, double B8, double sigma,
+                            double scale, const double *live) {
+    if (run_off(live, blockIdx.y)) return;
+    spec += (long long)blockIdx.y * n;
+    GRID_LOOP(i, n) {
         const int iz = (int)(i % nz);
         const long long r = i / nz;
         const int iy = (int)(r % ny), ix = (int)(r / ny);
@@ -48,8 +49,8 @@ __global__ void k_td_gmul_b(cpx<T> *spec, long long tot, long long n, int nx, in
         const double gz = fx * B2 + fy * B5 + fz * B8;
         const double gg = gx * gx + gy * gy + gz * gz;
         const double f = 0.5 * gg * exp(-gg * sigma * sigma / 2.0) * scale;
-        cpx<T> v = spec[j];
-        spec[j] = cpx<T>{(T)(v.x * f), (T)(v.y * f)};
+        cpx<T> v = spec[i];
+        spec[i] = cpx<T>{(T)(v.x * f), (T)(v.y * f)};
     }
 }
 
@@ -75,7 +76,8 @@ template <int K> __device__ __forceinline__ void run_partials(double *acc, doubl
 
 template <typename T, int MODE>
 __global__ void k_tdb_apply(const cpx<T> *x, const cpx<T> *kin, const T *v, double hdt, cpx<T> *out, long long n,
-                            double *partials) {
+                            double *partials, const double *live) {
+    if (run_off(live, blockIdx.y)) return;
     const long long o = (long long)blockIdx.y * n;
     x += o;
     kin += o;
@@ -237,7 +239,8 @@ __global__ void k_tdb_scalars(const double *partials, int nblk, double *st, doub
 // stacked runs.  Where the axes have size-specialised passes the kinetic
 // multiply is part of the x pass and the rest of the product (and its sums)
 // part of the inverse z pass; a CgStep, if given, is applied by the forward z
-// pass.  Else the complete transforms and separate kernels run.
+// pass.  Else the complete transforms and separate kernels run.  All of them
+// leave out the runs whose element of live, if given, is 0.
 template <typename T> struct KinOp {
     Plan &P;
     hipStream_t s;
@@ -260,12 +263,11 @@ template <typename T> struct KinOp {
     // returns the rows of partial sums per run
     template <int MODE>
     int apply(const cpx<T> *x, const T *v, double hdt, cpx<T> *out, const CgStep<T> *cg, const double *live) {
-        const double *m = xo ? live : nullptr;  // generic passes take every run
         if (zo) {
             const long long nrows = (long long)P.nr[0] * P.nr[1];
             const cpx<T> *tz = reinterpret_cast<const cpx<T> *>(P.tw[2]);
             zo->rows_fwd(x, kin, nb, n, nrows, tz, (T)1, cg, live, s, nullptr);
-            fft_cols<T>(P, 1, true, false, kin, kin, nb, n, 1.0, s, P.nr[2], m);
+            fft_cols<T>(P, 1, true, false, kin, kin, nb, n, 1.0, s, P.nr[2], live);
             if (xo) {
                 GParams gp{};
                 for (int i = 0; i < 9; ++i) gp.B[i] = P.B[i];
@@ -279,29 +281,29 @@ template <typename T> struct KinOp {
                 xo->xfused(P.var_cols[0], kin, nb, n, (long long)P.nr[1] * P.nr[2], P.nr[2], P.nr[2],
                            reinterpret_cast<const cpx<T> *>(P.tw[0]), gp, live, s, nullptr);
             } else {
-                fft_cols<T>(P, 0, true, false, kin, kin, nb, n, 1.0, s, P.nr[2]);
-                gmul();
-                fft_cols<T>(P, 0, true, true, kin, kin, nb, n, 1.0, s, P.nr[2]);
+                fft_cols<T>(P, 0, true, false, kin, kin, nb, n, 1.0, s, P.nr[2], live);
+                gmul(live);
+                fft_cols<T>(P, 0, true, true, kin, kin, nb, n, 1.0, s, P.nr[2], live);
             }
-            fft_cols<T>(P, 1, true, true, kin, kin, nb, n, 1.0, s, P.nr[2], m);
+            fft_cols<T>(P, 1, true, true, kin, kin, nb, n, 1.0, s, P.nr[2], live);
             const ApplyArgs<T> ap{x, v, hdt, P.red};
             const int rows = zo->rows_inv(MODE == 0 ? 3 : MODE, kin, out, nb, n, nrows, tz, (T)1, ap,
                                           std::min(1024, 32768 / nb), live, s, nullptr);
             OFDFT_HIP(hipGetLastError());
             return rows;
         }
-        fft_c2c<T>(P, x, kin, false, nb, n, 1.0, s);
-        gmul();
-        fft_c2c<T>(P, kin, kin, true, nb, n, 1.0, s);
-        hipLaunchKernelGGL((k_tdb_apply<T, MODE>), dim3(nblk, nb), dim3(256), 0, s, x, kin, v, hdt, out, n, P.red);
+        fft_c2c<T>(P, x, kin, false, nb, n, 1.0, s, live);
+        gmul(live);
+        fft_c2c<T>(P, kin, kin, true, nb, n, 1.0, s, live);
+        hipLaunchKernelGGL((k_tdb_apply<T, MODE>), dim3(nblk, nb), dim3(256), 0, s, x, kin, v, hdt, out, n, P.red,
+                           live);
         OFDFT_HIP(hipGetLastError());
         return nblk;
     }
-    void gmul() {
-        const long long tot = (long long)nb * n;
-        hipLaunchKernelGGL((k_td_gmul_b<T>), dim3(std::min<long long>((tot + 255) / 256, 8192)), dim3(256), 0, s, kin,
-                           tot, n, P.nr[0], P.nr[1], P.nr[2], P.B[0], P.B[1], P.B[2], P.B[3], P.B[4], P.B[5], P.B[6],
-                           P.B[7], P.B[8], sigma, 1.0 / (double)n);
+    void gmul(const double *live) {
+        hipLaunchKernelGGL((k_td_gmul_b<T>), dim3(std::min<long long>((n + 255) / 256, 8192 / nb), nb), dim3(256), 0, s,
+                           kin, n, P.nr[0], P.nr[1], P.nr[2], P.B[0], P.B[1], P.B[2], P.B[3], P.B[4], P.B[5], P.B[6],
+                           P.B[7], P.B[8], sigma, 1.0 / (double)n, live);
         OFDFT_HIP(hipGetLastError());
     }
 };

@@ -286,3 +286,28 @@ def test_f32_kinetic_keeps_f64_factors(nx):
         exact = np.sum((4 * 2.0 * np.pi * np.linalg.inv(lat).T[2]) ** 2)
         err = np.abs(-b.imag.double().mean(0).cpu().numpy() - exact).max()
         assert err <= 1.25 * 2.0 ** -24 * exact
+
+
+@pytest.mark.parametrize("shape", [(9, 15, 27), (27, 32, 40), (16, 18, 20)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_cn_batch_leaves_out_products_of_converged_runs(shape, dtype):
+    """A solve that starts converged applies the Hamiltonian twice (right side,
+    first residual): the workspace has the fields of one stopped there, and the
+    product of the first iteration was not written."""
+    from dftpy_amd.td import CrankNicholsonBatch
+    g = _grid(shape, dtype, full=True)
+    ct = torch.complex128 if dtype == torch.float64 else torch.complex64
+    rng = np.random.default_rng(5)
+    psi = torch.as_tensor(rng.standard_normal((2,) + shape) + 1j * rng.standard_normal((2,) + shape)).to(ct).cuda()
+    v = torch.as_tensor(rng.random((2,) + shape)).to(dtype).cuda()
+    n, out = int(np.prod(shape)), []
+    for tol, maxiter in ((1e-6, 0), (1e3, 50)):
+        cn = CrankNicholsonBatch(0.005, tol=tol, maxiter=maxiter)
+        cn(g, psi, v)
+        work = next(iter(cn._work.values())).view(ct)
+        work.fill_(7.0)
+        cn(g, psi, v)
+        assert [d["iterations"] for d in cn.last_info] == [0, 0]
+        assert bool((work[8 * n:] == 7.0).all())
+        out.append(work.clone())
+    assert torch.equal(out[0], out[1])
