@@ -158,7 +158,7 @@ int ofdft_plan_create(const int nr[3], const double lattice[9], int precision, i
             OFDFT_HIP(hipMemset(P->scal, 0, sizeof(double) * (kScalSlots + kRunSlots)));
             OFDFT_HIP(hipHostMalloc((void **)&P->pinned, 128 * sizeof(double), hipHostMallocMapped));
             OFDFT_HIP(hipHostGetDevicePointer((void **)&P->pinned_dev, P->pinned, 0));
-            P->ws_bytes = spec_bytes + work_bytes + sizeof(double) * (nred + kScalSlots);
+            P->ws_bytes = spec_bytes + work_bytes + sizeof(double) * (nred + kScalSlots + kRunSlots);
             plan_aux_setup(*P);
             P->ws_bytes += P->aux_bytes;
             OFDFT_HIP(hipDeviceSynchronize());

@@ -557,9 +557,9 @@ void fft_c2c(Plan &P, const cpx<T> *in, cpx<T> *out, bool inverse, int batch, lo
     OFDFT_REQUIRE(P.gate == nullptr, "gated launch of a generic FFT pass");
     if (const SizeOps<T> *ops = axis_ops<T>(P, 2)) {
         if (inverse)
-            ops->rows_inv(0, in, out, batch, bs, nrows, tw, sz, ApplyArgs<T>{}, 0, live, s, nullptr);
+            ops->rows_inv(0, in, out, batch, bs, nrows, tw, sz, ApplyArgs<T>{}, 0, live, s);
         else
-            ops->rows_fwd(in, out, batch, bs, nrows, tw, sz, nullptr, live, s, nullptr);
+            ops->rows_fwd(in, out, batch, bs, nrows, tw, sz, nullptr, live, s);
     } else if (inverse)
         hipLaunchKernelGGL((k_rows_c2c<T, true>), grid, dim3(sh.threads), sh.lds, s, in, out, bs, nrows, P.nr[2],
                            P.ax[2], tw, sh.tile, sz, live);

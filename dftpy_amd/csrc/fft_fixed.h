@@ -548,8 +548,8 @@ template <typename T> struct CgStep {
 template <typename T, int N, int NPEN, bool STEP>
 __global__ void __launch_bounds__((NPEN *SL<T, N>::TP))
     k_rows_fwd_f(const cpx<T> *in, cpx<T> *out, long long bs, int nrows, const cpx<T> *__restrict__ twg, T scale,
-                 CgStep<T> cg, const double *live, const double *gate) {
-    if (gate_off(gate) || run_off(live, blockIdx.y)) return;
+                 CgStep<T> cg, const double *live) {
+    if (run_off(live, blockIdx.y)) return;
     using C = cpx<T>;
     constexpr int R = SL<T, N>::first, RL = SL<T, N>::last, TP = SL<T, N>::TP, LD = N + 1;
     __shared__ C tw[N];
@@ -612,8 +612,8 @@ template <typename T> struct ApplyArgs {
 template <typename T, int N, int NPEN, int MODE>
 __global__ void __launch_bounds__((NPEN *SL<T, N>::TP))
     k_rows_inv_f(const cpx<T> *in, cpx<T> *out, long long bs, int nrows, int ntiles, const cpx<T> *__restrict__ twg,
-                 T scale, ApplyArgs<T> ap, const double *live, const double *gate) {
-    if (gate_off(gate) || run_off(live, blockIdx.y)) return;
+                 T scale, ApplyArgs<T> ap, const double *live) {
+    if (run_off(live, blockIdx.y)) return;
     using C = cpx<T>;
     constexpr int R = SL<T, N>::first, RL = SL<T, N>::last, TP = SL<T, N>::TP, LD = N + 1;
     constexpr int K = MODE == 1 ? 2 : 1;
@@ -703,10 +703,10 @@ template <typename T> struct SizeOps {
     void (*c2r)(int var, const cpx<T> *in, T *out, int batch, long long in_bs, long long out_bs, long long nrows,
                 long long ipitch, const cpx<T> *tw, T scale, hipStream_t s, const double *gate);
     void (*rows_fwd)(const cpx<T> *in, cpx<T> *out, int batch, long long bs, long long nrows, const cpx<T> *tw,
-                     T scale, const CgStep<T> *cg, const double *live, hipStream_t s, const double *gate);
+                     T scale, const CgStep<T> *cg, const double *live, hipStream_t s);
+    // scale: of mode 0
     int (*rows_inv)(int mode, const cpx<T> *in, cpx<T> *out, int batch, long long bs, long long nrows,
-                    const cpx<T> *tw, T scale, const ApplyArgs<T> &ap, int cap, const double *live, hipStream_t s,
-                    const double *gate);
+                    const cpx<T> *tw, T scale, const ApplyArgs<T> &ap, int cap, const double *live, hipStream_t s);
 };
 
 template <typename T, int N> struct Launch {
@@ -795,32 +795,33 @@ template <typename T, int N> struct Launch {
 #undef CALL
     }
     static void rows_fwd(const C *in, C *out, int batch, long long bs, long long nrows, const C *tw, T scale,
-                         const CgStep<T> *cg, const double *live, hipStream_t s, const double *gate) {
+                         const CgStep<T> *cg, const double *live, hipStream_t s) {
         constexpr int NP = pens_v<T, N, 1, 0>();
         const dim3 grid((unsigned)((nrows + NP - 1) / NP), (unsigned)batch);
         if (cg)
             hipLaunchKernelGGL((k_rows_fwd_f<T, N, NP, true>), grid, dim3(NP * TP), 0, s, in, out, bs, (int)nrows, tw,
-                               scale, *cg, live, gate);
+                               scale, *cg, live);
         else
             hipLaunchKernelGGL((k_rows_fwd_f<T, N, NP, false>), grid, dim3(NP * TP), 0, s, in, out, bs, (int)nrows, tw,
-                               scale, CgStep<T>{}, live, gate);
+                               scale, CgStep<T>{}, live);
     }
     template <int MODE>
     static int inv_mode(const C *in, C *out, int batch, long long bs, long long nrows, const C *tw, T scale,
-                        const ApplyArgs<T> &ap, int cap, const double *live, hipStream_t s, const double *gate) {
+                        const ApplyArgs<T> &ap, int cap, const double *live, hipStream_t s) {
         constexpr int NP = pens_v<T, N, 1, 0>();
         const long long tiles = (nrows + NP - 1) / NP;
         const int nb = tile_blocks(tiles, cap);
         hipLaunchKernelGGL((k_rows_inv_f<T, N, NP, MODE>), dim3((unsigned)nb, (unsigned)batch), dim3(NP * TP), 0, s, in,
-                           out, bs, (int)nrows, (int)tiles, tw, scale, ap, live, gate);
+                           out, bs, (int)nrows, (int)tiles, tw, scale, ap, live);
         return nb;
     }
     static int rows_inv(int mode, const C *in, C *out, int batch, long long bs, long long nrows, const C *tw, T scale,
-                        const ApplyArgs<T> &ap, int cap, const double *live, hipStream_t s, const double *gate) {
-        if (mode == 1) return inv_mode<1>(in, out, batch, bs, nrows, tw, scale, ap, cap, live, s, gate);
-        if (mode == 2) return inv_mode<2>(in, out, batch, bs, nrows, tw, scale, ap, cap, live, s, gate);
-        if (mode == 3) return inv_mode<3>(in, out, batch, bs, nrows, tw, scale, ap, 1 << 30, live, s, gate);
-        return inv_mode<0>(in, out, batch, bs, nrows, tw, scale, ap, 1 << 30, live, s, gate);
+                        const ApplyArgs<T> &ap, int cap, const double *live, hipStream_t s) {
+        OFDFT_REQUIRE(mode == 0 || scale == (T)1, "inverse z pass: the product takes the unscaled transform");
+        if (mode == 1) return inv_mode<1>(in, out, batch, bs, nrows, tw, scale, ap, cap, live, s);
+        if (mode == 2) return inv_mode<2>(in, out, batch, bs, nrows, tw, scale, ap, cap, live, s);
+        if (mode == 3) return inv_mode<3>(in, out, batch, bs, nrows, tw, scale, ap, 1 << 30, live, s);
+        return inv_mode<0>(in, out, batch, bs, nrows, tw, scale, ap, 1 << 30, live, s);
     }
 };
 

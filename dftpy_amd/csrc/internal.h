@@ -89,8 +89,9 @@ struct Prologue {
 
 struct LmgpState;  // LMGP nonlocal KEDF tables and workspace (lmgp.hip)
 
-// variants of the size-specialised FFT passes: two tiles each (variant % 2),
-// which the autotuner times; the ranges accepted by ofdft_plan_set_variants
+// variants of the size-specialised FFT passes: two tiles each, which the
+// autotuner times; ofdft_plan_set_variants accepts 3 numbers for the row passes
+// and 6 for the column passes (callers may hold them), variant v is tile v % 2
 constexpr int kTiles = 2;
 constexpr int kTileVariants = 3;
 constexpr int kColVariants = 6;

@@ -266,7 +266,7 @@ template <typename T> struct KinOp {
         if (zo) {
             const long long nrows = (long long)P.nr[0] * P.nr[1];
             const cpx<T> *tz = reinterpret_cast<const cpx<T> *>(P.tw[2]);
-            zo->rows_fwd(x, kin, nb, n, nrows, tz, (T)1, cg, live, s, nullptr);
+            zo->rows_fwd(x, kin, nb, n, nrows, tz, (T)1, cg, live, s);
             fft_cols<T>(P, 1, true, false, kin, kin, nb, n, 1.0, s, P.nr[2], live);
             if (xo) {
                 GParams gp{};
@@ -288,7 +288,7 @@ template <typename T> struct KinOp {
             fft_cols<T>(P, 1, true, true, kin, kin, nb, n, 1.0, s, P.nr[2], live);
             const ApplyArgs<T> ap{x, v, hdt, P.red};
             const int rows = zo->rows_inv(MODE == 0 ? 3 : MODE, kin, out, nb, n, nrows, tz, (T)1, ap,
-                                          std::min(1024, 32768 / nb), live, s, nullptr);
+                                          std::min(1024, 32768 / nb), live, s);
             OFDFT_HIP(hipGetLastError());
             return rows;
         }

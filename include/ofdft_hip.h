@@ -79,8 +79,9 @@ int ofdft_plan_set_fft_kernels(ofdft_plan *plan, int fixed);
 /* FFT autotuner (no counterpart in the reference): times the variants of each
  * size-specialised pass on the plan's shapes and keeps the fastest: two tiles
  * a pass.  Variants 0..2 of the z R2C and C2R row passes and 0..5 of the x and
- * y column passes are accepted; variant v has tile v % 2 and all give the same
- * results.
+ * y column passes are accepted; variant v is tile v % 2.  Both tiles give the
+ * same transforms bit for bit; the R2C pass's tile sets the order in which the
+ * mean density of the WT kernel is summed.
  * variants (optional, 4 ints): chosen variant of the z R2C, z C2R, x and y
  * passes; times (optional, 24 floats): mean ms of each variant, 6 per pass
  * in that order (-1 for those not timed).  The choice for a grid shape and
