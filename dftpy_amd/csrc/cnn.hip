@@ -19,7 +19,7 @@
 // W[co][ci] with v_mfma_f32_16x16x32_bf16 (16 points x 16 channels x 32 input
 // channels).  Backward-data is the same kernel with the weights transposed and
 // the taps mirrored; the weight gradient is a second MFMA kernel reducing over
-// points (K = points) through LDS-transposed tiles.
+// points (K = points), whose operands are read from LDS transposed.
 #include <algorithm>
 #include <cmath>
 #include <numeric>
@@ -572,9 +572,9 @@ __global__ void __launch_bounds__(ROWS_MAX_THREADS)
     if (MODE == 0 && nq > 0) copy_out(nq - 1);
 }
 
-// Ring-staged forward (inference: no ReLU output kept) for nz >= 36,
-// ny % d == 0, ny >= 4 d, nx % d == 0 and d <= 4.  A step computes 4 output
-// rows y0 + k d (k = 0..3) of one x plane for one 32-point z block; the rows
+// Ring-staged layer, forward and backward-data, for nz >= 36, ny % d == 0,
+// ny >= 4 d, nx % d == 0 and d <= 4.  A step computes 4 output rows y0 + k d
+// (k = 0..3) of one x plane for one 32-point z block; the rows
 // past ny of a residue class's last group and the points past nz of the last
 // z block are computed from wrapped inputs and not written (the staged rows
 // and points wrap once: ny >= 4 d, nz >= 36).  The steps of

@@ -10,13 +10,12 @@ pytestmark = pytest.mark.gpu
 
 SHAPE = (12, 10, 15)
 DIL = (1, 2, 1, 3, 2, 1)
-# (12, 10, 15): every layer on the point-tiled kernel; (6, 8, 32),
-# (4, 16, 64), (4, 8, 96) and (4, 8, 160): layers with ny % 4d == 0 on the
-# row-tiled kernel (one instance per nz / 32 = 1, 2, 3, 5: 96 is the
-# training grid, 160 the 500-atom cell's), the rest on the point-tiled one;
-# (6, 12, 40): the inference forward's ring-staged kernel with a partial z
+# middle layers, forward and backward-data: (12, 10, 15) on the point-tiled
+# kernel; (6, 8, 32) with d = 1 and 2 on the row-tiled one; (4, 16, 64),
+# (4, 8, 96) and (4, 8, 160) with d = 1 and 2 on the ring-staged one, with d = 3
+# on the point-tiled one; (6, 12, 40) on the ring-staged one with a partial z
 # block (40 = 32 + 8) and partial y groups (12 / d rows per residue class,
-# d = 1, 2, 3)
+# d = 1, 2, 3).  test_middle_layer_kernels has every instance.
 SHAPES = [(12, 10, 15), (6, 8, 32), (4, 16, 64), (4, 8, 96), (4, 8, 160), (6, 12, 40)]
 
 
@@ -98,13 +97,11 @@ def test_backward_matches_oracle(shape):
 @pytest.mark.parametrize("shape", [(8, 16, 96), (8, 16, 160), (8, 20, 72)])
 def test_shipped_dilations_match_oracle(shape):
     """The shipped network's dilations (1, 2, 4, 4, 2, 1) with nx and ny
-    multiples of d for every layer: the inference forward runs all four
-    middle layers on the ring-staged kernel, the training forward and the
-    backward on the row-tiled instances of the 96^3 training grid
-    (nz / 32 = 3) and of the 160^3 cell (nz / 32 = 5); (8, 20, 72) is a
-    batch-cell z size (72 = 2 x 32 + 8) with y groups that end short for
-    d = 4 (20 / 4 = 5 rows per residue class), its training forward and
-    backward on the point-tiled kernel."""
+    multiples of d for every layer: inference, training forward and backward
+    run all four middle layers on the ring-staged kernel.  96 is the training
+    grid's z size, 160 the 500-atom cell's; (8, 20, 72) is a batch-cell z size
+    (72 = 2 x 32 + 8) with y groups that end short for d = 4 (20 / 4 = 5 rows
+    per residue class)."""
     from oracle import cnn
     from dftpy_amd import DirectGrid
     from dftpy_amd.learned import WarmStartNet
@@ -131,30 +128,101 @@ def test_shipped_dilations_match_oracle(shape):
         assert _rel(got, g) < 1e-2, k
 
 
-def test_ring_forward_matches_row_kernel_at_160():
-    """At the 500-atom cell's full 160^3 grid (where the FP64 oracle is too
-    slow to run), the inference forward (ring-staged middle layers) against
-    the training forward (row-tiled middle layers, the instance the oracle
-    tests above pin at nz = 160): the same network, the same bf16 rounding
-    points, FP32 accumulation in a different order."""
-    from dftpy_amd.learned import WarmStartNet
-    from oracle import cnn
+def _mid(shape, d, mode, x, w, bias, resid, mask, off):
+    """One 32 -> 32 layer through its C entry.  off: elements by which the
+    fields that only need their element's alignment are moved in their
+    buffers, which keeps the layer off the ring-staged kernel's training modes.
+    Mode 0: (x + relu, relu), mode 1: (FP32 sum, masked BF16 copy)."""
+    from dftpy_amd import _lib
+    n = int(np.prod(shape))
+    nr = np.ascontiguousarray(shape, dtype=np.int32)
+
+    def moved(t):
+        v = torch.empty(n * 32 + 8, device="cuda", dtype=t.dtype)[off:off + n * 32]
+        return v.copy_(t.reshape(-1))
+
+    out1 = moved(torch.full((n, 32), float("nan"), device="cuda", dtype=torch.bfloat16))
+    if mode == 0:
+        out0 = torch.full((n * 32,), float("nan"), device="cuda", dtype=torch.bfloat16)
+        args = (bias.data_ptr(), None, None)
+    else:
+        out0, mask = moved(resid), moved(mask)
+        args = (None, out0.data_ptr(), mask.data_ptr())  # the residual in place, as the backward pass has it
+    _lib.check(_lib.lib.ofdft_cnn_conv_mid(_lib.iptr(nr), d, mode, x.data_ptr(), w.data_ptr(), *args, out0.data_ptr(),
+                                           out1.data_ptr(), _lib.stream()))
+    return out0.view(n, 32), out1.view(n, 32)
+
+
+def _mid_inputs(shape, seed=8):
+    n = int(np.prod(shape))
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=gen)  # noqa: E731
+    return rnd(n, 32).bfloat16(), (0.1 * rnd(27, 32, 32)).bfloat16(), rnd(32), rnd(n, 32), rnd(n, 32).bfloat16()
+
+
+# Row-tiled kernel, every instance (nz / 32 = 1 to 5): nz below the ring's 36,
+# nx no multiple of d, d above the ring's 4, or unaligned fields (off) on shapes
+# the ring takes otherwise; the point-tiled kernel likewise; the ring with
+# partial z blocks and row groups
+ROWS_CASES = [((6, 8, 32), 2, 0), ((5, 8, 64), 2, 0), ((5, 8, 96), 2, 0), ((7, 8, 128), 2, 0), ((6, 16, 160), 4, 0),
+              ((6, 20, 64), 5, 0), ((6, 20, 96), 5, 0), ((4, 16, 64), 1, 1), ((4, 8, 96), 2, 1), ((4, 8, 128), 1, 3),
+              ((8, 16, 160), 4, 1)]
+OTHER_CASES = [((6, 12, 40), 3, 1), ((5, 7, 48), 4, 1), ((6, 12, 40), 3, 0), ((4, 8, 96), 2, 0), ((8, 20, 72), 4, 0),
+               ((8, 16, 160), 4, 0)]
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("shape,d,off", ROWS_CASES + OTHER_CASES)
+def test_middle_layer_kernels(shape, d, off, mode):
+    """Each kernel of a 32 -> 32 layer, forward with the ReLU kept and
+    backward-data, against FP64: an FP32 sum of 864 products, the bias or
+    residual is within 866 ulps / 2 of the sum of the magnitudes; its BF16
+    copies are roundings (2^-9) of it, the masked one exactly that of out0."""
+    x, w, bias, resid, mask = _mid_inputs(shape)
+    out0, out1 = _mid(shape, d, mode, x, w, bias, resid, mask, off)
+    add = bias if mode == 0 else resid
+    ref, mag = add.double().expand(x.shape), add.double().abs().expand(x.shape)
+    for t in range(27):
+        sh = [-d * (i - 1) for i in (t // 9, t // 3 % 3, t % 3)]
+        xs = torch.roll(x.double().view(*shape, 32), sh, (0, 1, 2)).view(-1, 32)
+        wt = w[t].double().T.contiguous()
+        ref, mag = ref + xs @ wt, mag + xs.abs() @ wt.abs()
+    tol = 866 * 2.0 ** -24 * mag
+    if mode == 0:
+        ref = ref.clamp(min=0.0)
+        assert ((out1.double() - ref).abs() <= tol + 2.0 ** -8 * ref).all()
+        ref = ref + x.double()
+        assert ((out0.double() - ref).abs() <= tol + 2.0 ** -8 * ref.abs()).all()
+    else:
+        assert ((out0.double() - ref).abs() <= tol).all()
+        assert torch.equal(out1, torch.where(mask > 0, out0, torch.zeros_like(out0)).bfloat16())
+
+
+@pytest.mark.parametrize("d", [2, 4])
+def test_ring_forward_matches_row_kernel_at_160(d):
+    """At the 500-atom cell's full 160^3 grid (where FP64 sums are too slow),
+    one middle layer on the ring-staged kernel (aligned fields) against the
+    row-tiled kernel (fields off by an element; its instances are compared with
+    FP64 above): the same products, FP32 sums in a different order, forward
+    (BF16 outputs: a sum near a rounding boundary moves by 2^-8) and
+    backward-data.  The inference form of the ring, which keeps no ReLU, stores
+    the same sums bit for bit."""
+    from dftpy_amd import _lib
     shape = (160, 160, 160)
-    p = cnn.init_params(21, scale=1.5)
-    rng = np.random.default_rng(21)
-    for k in p:
-        if k.startswith("b"):
-            p[k] = rng.normal(0, 0.2, p[k].shape)
-    net = WarmStartNet()
-    net.set_params({k: v.astype(np.float32).astype(np.float64) for k, v in p.items()})
-    x = torch.randn((2, int(np.prod(shape))), dtype=torch.float32, device="cuda",
-                    generator=torch.Generator(device="cuda").manual_seed(5))
-    a = net.forward(x, shape, train=False).clone()
-    b = net.forward(x, shape, train=True).clone()
-    rel = float((a - b).norm() / b.norm())
-    print("ring vs row kernel at 160^3: rel L2 %.2e, max %.2e" % (rel, float((a - b).abs().max())))
-    assert rel < 1e-3
-    assert float((a - b).abs().max()) < 1e-2 * float(b.abs().max())
+    x, w, bias, resid, mask = _mid_inputs(shape)
+    ring, rows = (_mid(shape, d, 0, x, w, bias, resid, mask, off) for off in (0, 1))
+    for a, b in zip(ring, rows):
+        a, b = a.float(), b.float()
+        assert float((a - b).norm() / b.norm()) < 1e-3
+        assert bool(((a - b).abs() <= 2.0 ** -7 * b.abs() + 1e-3).all())
+    plain = torch.full_like(ring[0], float("nan"))
+    nr = np.ascontiguousarray(shape, dtype=np.int32)
+    _lib.check(_lib.lib.ofdft_cnn_conv_mid(_lib.iptr(nr), d, 0, x.data_ptr(), w.data_ptr(), bias.data_ptr(), None, None,
+                                           plain.data_ptr(), None, _lib.stream()))
+    assert torch.equal(plain, ring[0])
+    ring, rows = (_mid(shape, d, 1, x, w, bias, resid, mask, off) for off in (0, 1))
+    assert float((ring[0] - rows[0]).norm() / rows[0].norm()) < 1e-5
+    assert float((ring[0] - rows[0]).abs().max()) < 1e-3
 
 
 @pytest.mark.parametrize("shape,dil", [((12, 10, 15), 1), ((4, 8, 160), 1), ((9, 6, 40), 2), ((8, 7, 300), 3),
