@@ -185,12 +185,14 @@ __global__ void __launch_bounds__((TILE *SL<T, N>::TP))
     });
 }
 
-// FP32 half grids form the G-space factors of the evaluation in FP32 at these
-// x lengths; every other FP32 pass with the multiply (full grids, the other
-// lengths, the kinetic operator) forms and applies them in FP64, as the
-// stand-alone multiply does.  An FP32 evaluation of 160^3: 167 us on the half
-// grid, 178 on the full one; with FP32 factors 167 and 169.
-constexpr bool f32_factors(int n) {
+// The lengths that had passes of their own first.  Two things hold for them
+// alone, as before the others got theirs: the device-driven TN accepts them
+// (opt.hip), and FP32 half grids form the G-space factors of the evaluation in
+// FP32 at these x lengths.  Every other FP32 pass with the multiply (full
+// grids, the other lengths, the kinetic operator) forms and applies them in
+// FP64, as the stand-alone multiply does.  An FP32 evaluation of 160^3: 167 us
+// on the half grid, 178 on the full one; with FP32 factors 167 and 169.
+constexpr bool first_length(int n) {
     for (int m : {32, 48, 64, 72, 80, 96, 100, 120, 128, 144, 160, 192, 200, 240, 256})
         if (n == m) return true;
     return false;
@@ -732,7 +734,7 @@ template <typename T, int N> struct Launch {
     }
     static void xfused(int var, C *data, int batch, long long bs, long long ncols, long long pitch, long long vp,
                        const C *tw, const GParams &gp, const double *live, hipStream_t s, const double *gate) {
-        if constexpr (sizeof(T) == 4 && f32_factors(N)) {
+        if constexpr (sizeof(T) == 4 && first_length(N)) {
             if (!gp.full && !gp.c2c) return xfused_ft<T>(var, data, batch, bs, ncols, pitch, vp, tw, gp, live, s, gate);
         }
         xfused_ft<double>(var, data, batch, bs, ncols, pitch, vp, tw, gp, live, s, gate);

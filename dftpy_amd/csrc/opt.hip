@@ -816,13 +816,6 @@ struct Ctx {
 #define PW_RED(K, ...) PW_LAUNCH_(K, C.nb, __VA_ARGS__)
 #define PW_STREAM(K, ...) PW_LAUNCH_(K, C.nbw, __VA_ARGS__)
 
-// lengths the device-driven iteration is accepted for
-static bool graph_size(int n) {
-    for (int m : {32, 48, 64, 72, 80, 96, 100, 120, 128, 144, 160, 192, 200, 240, 256})
-        if (n == m) return true;
-    return false;
-}
-
 template <typename T> struct Opt {
     Plan &P;
     Ctx C;
@@ -1296,10 +1289,12 @@ template <typename T> struct Opt {
                   double *history, int hcap) {
         OFDFT_REQUIRE(G >= 1 && G <= 64 && L >= 1 && L <= 64, "optimize_tn_graph: steps per superstep out of range");
         OFDFT_REQUIRE(!(P.terms & OFDFT_TERM_LMGP), "optimize_tn_graph: LMGP is not supported");
+        // the gated launches need passes of the axis' own; lengths that got
+        // theirs later are refused as before
         for (int d = 0; d < 3; ++d)
-            OFDFT_REQUIRE(P.use_fixed && (P.nr[d] == 1 || graph_size(P.nr[d])),
-                          "optimize_tn_graph: every axis needs a size-specialised FFT pass (2/3/5-smooth sizes of "
-                          "the fixed table)");
+            OFDFT_REQUIRE(P.use_fixed && (P.nr[d] == 1 || first_length(P.nr[d])),
+                          "optimize_tn_graph: every axis needs size-specialised FFT passes of 32, 48, 64, 72, 80, 96, "
+                          "100, 120, 128, 144, 160, 192, 200, 240 or 256 points (or 1 point)");
         const double econv = opts[0];
         const int maxiter = (int)opts[1], maxfun = (int)opts[2], maxls = (int)opts[3];
         const auto t0 = std::chrono::steady_clock::now();

@@ -369,7 +369,8 @@ int ofdft_optimize(ofdft_plan *plan, void *rho, void *pot, int method, int hvp, 
  * results equal ofdft_optimize's up to the last bits of cos/sin of the line
  * search step (device vs host libm).  stats[7] = supersteps launched,
  * stats[8], stats[9] = graph captures / in-place updates on this plan so far.
- * Needs size-specialised FFT passes on every axis and no LMGP term.  The
+ * Needs axes of 32, 48, 64, 72, 80, 96, 100, 120, 128, 144, 160, 192, 200,
+ * 240 or 256 points (or 1) with size-specialised FFT passes, and no LMGP term.  The
  * first call on a plan (and any call after its settings change) captures;
  * the capture stream is created once per plan (default priority).
  * No counterpart in the reference beyond get_direction_TN / optimize_rho. */

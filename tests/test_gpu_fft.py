@@ -311,3 +311,23 @@ def test_cn_batch_leaves_out_products_of_converged_runs(shape, dtype):
         assert bool((work[8 * n:] == 7.0).all())
         out.append(work.clone())
     assert torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("n", [210, 224, 234, 240, 250, 252, 256])
+def test_f32_full_grids_of_the_longest_axes(n):
+    """The x pass with FP64 factors needs the most LDS here (130 KB at 256 with
+    the second tile): both tiles against the generic kernels, to FP32 rounding
+    that vW's G^2 multiplies."""
+    from dftpy_amd import DirectField, _lib
+    from dftpy_amd.functional import Functional, TotalFunctional
+    shape = (n, 4, 18)
+    g = _grid(shape, torch.float32, full=True)
+    rho = DirectField(g, data=0.02 + 0.01 * np.random.default_rng(2).random(shape))
+    ev = TotalFunctional(KE=Functional(type="KEDF", name="WT"), H=Functional(type="HARTREE"))
+    out = []
+    for fixed, tile in ((1, 0), (1, 1), (0, 0)):
+        _lib.check(_lib.lib.ofdft_plan_set_fft_kernels(g.plan().handle, fixed))
+        g.plan().set_variants([tile] * 4)
+        out.append(ev(rho).potential.numpy().astype(np.float64))
+    for v in out[:2]:
+        assert np.max(np.abs(v - out[2])) <= 4e-4 * np.max(np.abs(out[2]))

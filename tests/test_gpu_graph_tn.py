@@ -128,17 +128,19 @@ def test_graph_tn_capture_is_reused_and_updated():
     assert stats[3] == stats[2]
 
 
-def test_graph_tn_needs_fixed_size_passes():
-    """Grids with an axis outside the size-specialised FFT table, and LMGP,
-    are refused with a message (the host-driven TN covers them)."""
+@pytest.mark.parametrize("nr", [(30, 30, 30), (27, 32, 32), (32, 32, 242)])
+def test_graph_tn_needs_fixed_size_passes(nr):
+    """Grids with an axis whose size-specialised FFT passes the device-driven
+    TN is not accepted for (30) or which has none (27, 242) are refused with a
+    message that names the lengths (the host-driven TN covers them)."""
     from dftpy_amd import DirectField, DirectGrid, _lib, systems
     from dftpy_amd.functional import Functional, TotalFunctional
     ions, _ = systems.c1_system()
-    grid = DirectGrid(ions.cell, (30, 30, 30), full=False)
+    grid = DirectGrid(ions.cell, nr, full=False)
     pp = Functional(type="PSEUDO", grid=grid, ions=ions, PP_list={"Al": systems.empty_core_recpot()})
     ev = TotalFunctional(KE=Functional(type="KEDF", name="WT"), XC=Functional(type="XC", name="LDA"),
                          H=Functional(type="HARTREE"), PSEUDO=pp)
     rho = DirectField(grid)
     rho[:] = ions.get_ncharges() / grid.volume
-    with pytest.raises(_lib.OFDFTError, match="size-specialised"):
+    with pytest.raises(_lib.OFDFTError, match="size-specialised.*32, 48"):
         _run(ev, rho, econv=1e-8, maxiter=10, graph=True)
