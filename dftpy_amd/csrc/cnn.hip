@@ -1076,8 +1076,9 @@ __global__ void __launch_bounds__(OUTW_THREADS) k_cnn_out_walk(Geo g, OutWalk wk
 // dh[q][c] = sum_t W6[t][c] dout[q - off_t];  g = mask > 0 ? dh : 0 (bf16).
 // FP32 matrix instructions (32 points x 32 channels x 2 taps, 14 of them, a
 // zero 28th tap): the weights stay in registers and a row of 32 channels leaves
-// as whole lines.  Bound by its 256 bytes per point.  96^3: 58 us, 86 with a
-// thread per point and the weights read from LDS for each.
+// as whole lines.  Bound by its 256 bytes per point.  96^3: 58 us (65 in a
+// training step), 86 with a thread per point and the weights read from LDS for
+// each.
 __global__ void __launch_bounds__(256) k_cnn_out_bwd(Geo g, const float *__restrict__ dout,
                                                      const float *__restrict__ w, const __bf16 *__restrict__ mask,
                                                      float *__restrict__ dh, __bf16 *__restrict__ gout) {

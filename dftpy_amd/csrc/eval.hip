@@ -230,8 +230,8 @@ __global__ void __launch_bounds__(256) k_post(const T *__restrict__ rho, const T
 // would leave the chip idle otherwise, else four per access where the length
 // allows.  FP32 then walks the field in a loop of at most 1024 workgroups (g =
 // 0); FP64, whose constants a loop keeps in 100 registers (160^3: 43 us, 36
-// without), unrolls up to four groups per thread, as many as keep the partial
-// sums near 1500 rows (2000 rows cost the one-workgroup final sum 6 us).
+// to 40 without), unrolls up to four groups per thread, as many as keep the
+// partial sums near 1500 rows (2000 rows cost the one-workgroup final sum 6 us).
 struct PointShape {
     int vec, g = 1, nb;
     PointShape(long long n, bool can4, bool fp64) {
